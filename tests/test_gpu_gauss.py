@@ -52,3 +52,24 @@ def test_sw_rhs_gauss_random_geometry_factors(extents):
     got = host(domain.scalar_wave_rhs_gauss(dev(u), dev(g2), dev(inv), dev(det_inv),
                                             dev(face_inv)))
     assert np.array_equal(got, ref)
+
+
+# the smallest and largest elements of the two-launch form (3^3, 13^3, a flat
+# 20 x 20 x 3) and the ones just outside it (2^3, 14^3, 2 x 2 x 3)
+@pytest.mark.parametrize("extents", [(3, 3, 3), (13, 13, 13), (20, 20, 3), (2, 2, 2),
+                                     (14, 14, 14), (2, 2, 3), (2, 2, 20)])
+def test_sw_rhs_gauss_route_edges(extents):
+    print(f"gauss edges {extents}", flush=True)
+    brick, u, g2, inv, det_inv, face_inv = wl.scalar_wave_plane_wave_gauss(
+        seed=6, elements=(2, 1, 3), extents=extents)
+    rng = np.random.default_rng(12)
+    u = rng.uniform(-1, 1, u.shape)
+    g2 = rng.uniform(0.2, 1.5, g2.shape)
+    inv = rng.uniform(-2, 2, inv.shape)
+    det_inv = rng.uniform(0.5, 3.0, det_inv.shape)
+    face_inv = rng.uniform(-2, 2, face_inv.shape)
+    ref = ol.sw_rhs_gauss(brick.extents, brick.neighbors, u, g2, inv, det_inv, face_inv)
+    domain = dg.Domain.from_brick(brick)
+    got = host(domain.scalar_wave_rhs_gauss(dev(u), dev(g2), dev(inv), dev(det_inv),
+                                            dev(face_inv)))
+    assert np.array_equal(got, ref)
