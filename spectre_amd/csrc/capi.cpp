@@ -24,8 +24,14 @@ namespace sxd {
 // Grown on demand (hipFree, then hipMalloc: a growth waits for the device),
 // or, when `fixed`, a caller-provided block that is never reallocated.
 struct Scratch {
+  // Held while a call enqueues its kernels: calls of several threads on one
+  // stream take their turns, so that none of them writes the work arrays
+  // between another's kernels.
+  std::mutex enqueue;
   double* du = nullptr;
   double* temps = nullptr;
+  // The pair kernels' work array: one size per domain, so it never moves.
+  double* pairs = nullptr;
   size_t du_doubles = 0, temps_doubles = 0;
   bool fixed = false;
   size_t fixed_doubles = 0;  // capacity of a fixed block
@@ -89,8 +95,20 @@ struct Scratch {
     }
     return SXD_OK;
   }
+  int reserve_pairs(size_t n) {
+    if (fixed) {
+      if (n > fixed_doubles) return SXD_ERR_UNSUPPORTED;
+      pairs = du;
+    }
+    if (pairs == nullptr && hipMalloc(&pairs, n * sizeof(double)) != hipSuccess) {
+      pairs = nullptr;
+      return SXD_ERR_OUT_OF_MEMORY;
+    }
+    return SXD_OK;
+  }
   void release() {
     if (!fixed) {
+      if (pairs != nullptr) (void)hipFree(pairs);
       if (du != nullptr) (void)hipFree(du);
       if (temps != nullptr) (void)hipFree(temps);
     }
@@ -104,7 +122,7 @@ struct Scratch {
     }
     side = nullptr;
     fork = join = nullptr;
-    du = temps = nullptr;
+    du = temps = pairs = nullptr;
     du_doubles = temps_doubles = 0;
   }
 };
@@ -912,9 +930,32 @@ int candidate_kernels(const sxd_domain* d, int system, int* k) {
 
 int resolve_kernel(const sxd_domain* d, int system) {
   if (d->kernel[system] != SXD_KERNEL_AUTO) return d->kernel[system];
+  if (system == SXD_SYSTEM_GH && !d->mixed && gh_pairs_faster(d->num_elements, d->ext))
+    return SXD_KERNEL_COMPOSITE;
   int k[3];
   candidate_kernels(d, system, k);
   return k[0];
+}
+
+// The GH kernel of one call on `stream`.  Where the pair kernels stand in for
+// the fused one (gh_pairs_faster) they need a work array that the fused kernel
+// does not: a call recorded into the caller's graph, whose replays may run
+// beside later calls or outlive the array, and a call whose array cannot be
+// allocated, keep the fused kernel.
+int gh_call_kernel(const sxd_domain* d, Scratch& sc, hipStream_t stream) {
+  const int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
+  if (kernel != SXD_KERNEL_COMPOSITE || d->kernel[SXD_SYSTEM_GH] != SXD_KERNEL_AUTO ||
+      d->mixed || !gh_fused_supported(d->ext))
+    return kernel;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
+      capture != hipStreamCaptureStatusNone)
+    return SXD_KERNEL_FUSED;
+  if (sc.reserve_pairs(gh_pairs_work_doubles(d->num_elements, d->ext)) != SXD_OK) {
+    (void)hipGetLastError();
+    return SXD_KERNEL_FUSED;
+  }
+  return kernel;
 }
 
 // Reserve work arrays (status only; finish() words the message).
@@ -1021,6 +1062,12 @@ int run_gh(sxd_domain* d, Scratch& sc, int kernel, const double* u, const double
     return launch_gh_rhs_fused(d->num_elements, d->ext, d->d_nbr, u, gammas, inv_jac, dt,
                                kernel == SXD_KERNEL_FUSED ? kGhFusedValu : kGhFusedMfma,
                                d->threads[SXD_SYSTEM_GH] == 512 ? 512 : 256, ghost, stream);
+  if (gh_pairs_supported(d->ext)) {
+    if (int rc = sc.reserve_pairs(gh_pairs_work_doubles(d->num_elements, d->ext)); rc != SXD_OK)
+      return rc;
+    return launch_gh_rhs_pairs(d->num_elements, d->ext, d->d_nbr, u, gammas, inv_jac, dt,
+                               sc.pairs, ghost, stream);
+  }
   const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];
   if (int rc = reserve_scratch(sc, 150 * np * d->num_elements, 12 * np * d->num_elements);
       rc != SXD_OK)
@@ -1047,6 +1094,7 @@ int sxd_scalar_wave_rhs(const sxd_domain* domain, const double* u, const double*
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
                        static_cast<hipStream_t>(stream)),
                 __func__);
@@ -1064,6 +1112,7 @@ int sxd_scalar_wave_rhs_dirichlet(const sxd_domain* domain, const double* u,
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
                        static_cast<hipStream_t>(stream), ghost),
                 __func__);
@@ -1085,6 +1134,7 @@ int sxd_scalar_wave_rhs_spherical_radiation(const sxd_domain* domain, const doub
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   const int kind = type == SXD_SPHERICAL_RADIATION_SOMMERFELD ? kSwBcSommerfeld
                                                               : kSwBcBaylissTurkel;
   return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
@@ -1109,6 +1159,7 @@ int sxd_scalar_wave_rhs_constraint_preserving_spherical_radiation(
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   const int kind = kSwBcCpsrSommerfeld + (type - SXD_CPSR_SOMMERFELD);
   return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
                        static_cast<hipStream_t>(stream),
@@ -1133,6 +1184,7 @@ int sxd_scalar_wave_rhs_gauss(const sxd_domain* domain, const double* u, const d
   if (device_gauss_tables() == nullptr)
     return fail(SXD_ERR_DEVICE, "%s: upload of the Gauss tables failed", __func__);
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];
   if (int rc = reserve_scratch(sc, 15 * np * d->num_elements, 0); rc != SXD_OK)
     return finish(rc, __func__);
@@ -1152,8 +1204,9 @@ int sxd_gh_rhs(const sxd_domain* domain, const double* u, const double* gammas,
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 50, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
-  return finish(run_gh(d, sc, resolve_kernel(d, SXD_SYSTEM_GH), u, gammas, inv_jac, dt,
-                       static_cast<hipStream_t>(stream)),
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
+  return finish(run_gh(d, sc, gh_call_kernel(d, sc, static_cast<hipStream_t>(stream)), u, gammas,
+                       inv_jac, dt, static_cast<hipStream_t>(stream)),
                 __func__);
 }
 
@@ -1164,6 +1217,9 @@ int sxd_gh_rhs_noalloc(const sxd_domain* domain, const double* u, const double* 
     return fail(SXD_ERR_UNSUPPORTED, "%s: not built for mortar domains", __func__);
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
+  // no work arrays where the caller has not asked for a kernel that needs them
+  if (d->kernel[SXD_SYSTEM_GH] == SXD_KERNEL_AUTO && !d->mixed && gh_fused_supported(d->ext))
+    kernel = SXD_KERNEL_FUSED;
   // the mortar organisation's package buffers do not fit the fixed array at
   // useful sizes: mixed-p domains run the batched mixed-p kernels here
   if (kernel == SXD_KERNEL_MORTAR) kernel = SXD_KERNEL_MIXED_BATCHED;
@@ -1208,7 +1264,8 @@ int sxd_gh_rhs_dirichlet(const sxd_domain* domain, const double* u, const double
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 50, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
-  const int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
+  const int kernel = gh_call_kernel(d, sc, static_cast<hipStream_t>(stream));
   if (kernel == SXD_KERNEL_FUSED_MFMA)
     return fail(SXD_ERR_UNSUPPORTED, "external faces are not built for the MFMA engine; "
                                      "select the fused or composite kernel");
@@ -1264,6 +1321,7 @@ int sxd_rhs_begin(const sxd_domain* domain, int system, const double* u, const d
   if (int rc = check_no_overlap(d, gh ? 50 : 5, u, dt, __func__); rc != SXD_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   Scratch& sc = stream_scratch(d, s);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   const size_t du = gh ? 150 * static_cast<size_t>(d->total_points) : 0;
   int rc = reserve_scratch(sc, du, mortar_work_doubles(gh, d->plan));
   if (rc == SXD_OK)
@@ -1287,6 +1345,7 @@ int sxd_boundary_messages_unpack(const sxd_domain* domain, int system, int sende
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   hipStream_t s = static_cast<hipStream_t>(stream);
   Scratch& sc = stream_scratch(d, s);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   if (!sc.begun || sc.phase_system != system)
     return fail(SXD_ERR_INVALID_ARGUMENT, "%s: no sxd_rhs_begin of this system on this stream",
                 __func__);
@@ -1343,6 +1402,7 @@ int sxd_rhs_end(const sxd_domain* domain, int system, double* dt, void* stream) 
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   hipStream_t s = static_cast<hipStream_t>(stream);
   Scratch& sc = stream_scratch(d, s);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   if (!sc.begun || sc.phase_system != system)
     return fail(SXD_ERR_INVALID_ARGUMENT, "%s: no sxd_rhs_begin of this system on this stream",
                 __func__);
@@ -1401,6 +1461,7 @@ int sxd_gh_rhs_bjorhus(const sxd_domain* domain, int bjorhus_type, const double*
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   if (int rc = check_no_overlap(d, 50, u, dt, __func__); rc != SXD_OK) return rc;
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (d->mixed) {
     // the mixed-p kernels with their face passes (the mortar organisation
@@ -1470,6 +1531,7 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
       rc != SXD_OK)
     return rc;
   Scratch& sc = stream_scratch(domain, s);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   hipEvent_t ev[2];
   if (hipEventCreate(&ev[0]) != hipSuccess) return fail(SXD_ERR_DEVICE, "hipEventCreate failed");
   if (hipEventCreate(&ev[1]) != hipSuccess) {
@@ -1553,6 +1615,7 @@ int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u, const double* 
     return fail(SXD_ERR_UNSUPPORTED, "%s: not built for mortar domains", __func__);
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
   if (d->mixed) {
     if (int rc = reserve_scratch(sc, 150 * static_cast<size_t>(d->total_points), 0);
         rc != SXD_OK)

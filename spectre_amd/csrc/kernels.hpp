@@ -84,6 +84,18 @@ int launch_gh_rhs_composite(int num_elements, const int32_t ext[3], const int32_
                             const double* u, const double* gammas, const double* inv_jac,
                             double* dt, double* scratch_du, double* scratch_temps,
                             const double* ghost, hipStream_t stream);
+// The GH RHS in two kernels (gh_volume.hip).  Doubles of a point's state;
+// work: gh_pairs_work_doubles doubles (the states, and 12 per face point; at
+// most 71 per point).
+constexpr int kGhStateDoubles = 35;
+// The five fields and face corrections of a pair fit the LDS (up to 14^3).
+bool gh_pairs_supported(const int32_t ext[3]);
+size_t gh_pairs_work_doubles(int num_elements, const int32_t ext[3]);
+bool gh_pairs_faster(int num_elements, const int32_t ext[3]);
+// ghost: as for launch_gh_rhs_composite.
+int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* nbr,
+                        const double* u, const double* gammas, const double* inv_jac, double* dt,
+                        double* work, const double* ghost, hipStream_t stream);
 // Derivative engines of the fused GH kernel.
 constexpr int kGhFusedValu = 0;  // LDS pencils on the vector ALUs
 constexpr int kGhFusedMfma = 1;  // v_mfma_f64_16x16x4f64 tiles
