@@ -30,8 +30,9 @@ struct Scratch {
   std::mutex enqueue;
   double* du = nullptr;
   double* temps = nullptr;
-  // The pair kernels' work array: one size per domain, so it never moves.
-  double* pairs = nullptr;
+  // Work arrays of one size per domain and system, so that they never move:
+  // the GH pair kernels' and the lifted corrections of mortar domains.
+  double* block[2] = {nullptr, nullptr};
   size_t du_doubles = 0, temps_doubles = 0;
   bool fixed = false;
   size_t fixed_doubles = 0;  // capacity of a fixed block
@@ -95,20 +96,21 @@ struct Scratch {
     }
     return SXD_OK;
   }
-  int reserve_pairs(size_t n) {
+  int reserve_block(int system, size_t n) {
     if (fixed) {
       if (n > fixed_doubles) return SXD_ERR_UNSUPPORTED;
-      pairs = du;
+      block[system] = du;
     }
-    if (pairs == nullptr && hipMalloc(&pairs, n * sizeof(double)) != hipSuccess) {
-      pairs = nullptr;
+    if (block[system] == nullptr && hipMalloc(&block[system], n * sizeof(double)) != hipSuccess) {
+      block[system] = nullptr;
       return SXD_ERR_OUT_OF_MEMORY;
     }
     return SXD_OK;
   }
   void release() {
     if (!fixed) {
-      if (pairs != nullptr) (void)hipFree(pairs);
+      for (double* b : block)
+        if (b != nullptr) (void)hipFree(b);
       if (du != nullptr) (void)hipFree(du);
       if (temps != nullptr) (void)hipFree(temps);
     }
@@ -122,7 +124,7 @@ struct Scratch {
     }
     side = nullptr;
     fork = join = nullptr;
-    du = temps = pairs = nullptr;
+    du = temps = block[0] = block[1] = nullptr;
     du_doubles = temps_doubles = 0;
   }
 };
@@ -153,6 +155,7 @@ struct sxd_domain {
   int32_t* d_buckets = nullptr;       // elements grouped by extents
   int32_t* d_point_el = nullptr;      // element of each grid point
   std::vector<std::pair<int, int>> buckets;  // (start, count) in d_buckets
+  std::vector<sxd::RaggedClass> classes;     // d_list by element size
   // Mortar domains (non-aligned neighbours, h-refined faces): the ragged
   // element set above (its neighbour table unused) and the mortar tables.
   bool mortars = false;
@@ -690,6 +693,19 @@ int create_mixed_domain(sxd_domain** domain, int num_elements, const int32_t* ex
     d->buckets.emplace_back(i, j - i);
     i = j;
   }
+  // classes of the volume kernels, whose LDS a launch reserves for its largest
+  // element: up to 300, 600, 1000 and more points (12, 24, 40 KB and more of
+  // fields)
+  auto size_class = [&](int i) {
+    const int np = el[list[i]].np;
+    return np > 1000 ? 3 : np > 600 ? 2 : np > 300 ? 1 : 0;
+  };
+  for (int i = 0; i < num_elements;) {
+    int j = i;
+    while (j < num_elements && size_class(j) == size_class(i)) ++j;
+    d->classes.push_back({i, j - i, el[list[i]].np});
+    i = j;
+  }
   d->mixed = true;
   d->has_boundary = has_boundary;
   d->num_elements = num_elements;
@@ -951,7 +967,7 @@ int gh_call_kernel(const sxd_domain* d, Scratch& sc, hipStream_t stream) {
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
       capture != hipStreamCaptureStatusNone)
     return SXD_KERNEL_FUSED;
-  if (sc.reserve_pairs(gh_pairs_work_doubles(d->num_elements, d->ext)) != SXD_OK) {
+  if (sc.reserve_block(SXD_SYSTEM_GH, gh_pairs_work_doubles(d->num_elements, d->ext)) != SXD_OK) {
     (void)hipGetLastError();
     return SXD_KERNEL_FUSED;
   }
@@ -963,45 +979,65 @@ int reserve_scratch(Scratch& sc, size_t du_doubles, size_t temps_doubles) {
   return sc.reserve(du_doubles, temps_doubles);
 }
 
-// Volume terms on the ragged element set, then the corrections of every
-// mortar; work arrays: the derivatives (GH) and the mortar buffers.
+// Volume terms of the ragged element set (state: GH work array).
+int run_ragged_volume(sxd_domain* d, bool gh, const double* u, const double* params,
+                      const double* inv_jac, double* dt, double* state, hipStream_t stream) {
+  if (!gh)
+    return launch_ragged_sw_volume(d->classes, d->d_list, d->d_el, u, params, inv_jac, dt, nullptr,
+                                   nullptr, stream);
+  const int rc = launch_ragged_gh_state(d->num_elements, d->d_list, d->d_el, d->np_max, u, params,
+                                        state, stream);
+  return rc != SXD_OK ? rc
+                      : launch_ragged_gh_volume(d->classes, d->d_list, d->d_el, u, params,
+                                                inv_jac, dt, state, nullptr, nullptr, stream);
+}
+
+// The lifted corrections of every mortar, then the volume terms, which add
+// them.
 int run_mortars(sxd_domain* d, Scratch& sc, bool gh, const double* u, const double* params,
                 const double* inv_jac, double* dt, hipStream_t stream) {
-  const size_t du = gh ? 150 * static_cast<size_t>(d->total_points) : 0;
-  if (int rc = reserve_scratch(sc, du, mortar_work_doubles(gh, d->plan)); rc != SXD_OK) return rc;
-  const int threads = d->threads[gh ? SXD_SYSTEM_GH : SXD_SYSTEM_SCALAR_WAVE];
-  auto volume = [&](hipStream_t s) {
-    return launch_mixed_volume(gh, d->num_elements, d->d_list, d->d_el, d->np_max, u, params,
-                               inv_jac, dt, sc.du, threads, s);
-  };
-  // The packages and boundary terms read u only and write the work array:
-  // they run on a second stream beside the volume terms, and the lift (which
-  // adds into dt after them) waits for both.  Inside a graph capture the
-  // same fork and join become graph edges; a stream first seen inside a
-  // capture (no side stream yet) runs everything in order.
+  const size_t total = static_cast<size_t>(d->total_points);
+  // a partition with remote mortars is evaluated by sxd_rhs_begin and _end
+  if (d->plan.num_remote > 0) return SXD_ERR_UNSUPPORTED;
+  const int system = gh ? SXD_SYSTEM_GH : SXD_SYSTEM_SCALAR_WAVE;
+  const MortarCorrectionsWork size(gh, d->plan, nullptr);
+  if (int rc = sc.reserve_block(system, size.doubles + (gh ? kGhStateDoubles * total : 0));
+      rc != SXD_OK)
+    return rc;
+  const MortarCorrectionsWork w(gh, d->plan, sc.block[system]);
+  if (!gh) {
+    const int rc = launch_mortar_lifted_corrections(false, d->plan, d->d_el, u, params, inv_jac,
+                                                    w.corr, stream);
+    return rc != SXD_OK ? rc
+                        : launch_ragged_sw_volume(d->classes, d->d_list, d->d_el, u, params,
+                                                  inv_jac, dt, d->plan.d_corrections, w.corr,
+                                                  stream);
+  }
+  double* state = w.corr + w.doubles;
+  // The corrections and the point states both read u only: they run beside
+  // each other on two streams, and the pair kernel waits for both.  Inside a
+  // graph capture the same fork and join become graph edges; a stream first
+  // seen inside a capture (no side stream yet) runs everything in order.
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess) return SXD_ERR_DEVICE;
-  const bool fork = d->plan.num_remote == 0 &&
-                    (sc.side != nullptr ||
-                     (capture == hipStreamCaptureStatusNone && sc.ensure_side()));
-  if (!fork) {
-    if (int rc = volume(stream); rc != SXD_OK) return rc;
-    return launch_mortar_faces(gh, d->plan, d->d_el, u, params, inv_jac, dt, sc.temps, stream);
-  }
-  if (hipEventRecord(sc.fork, stream) != hipSuccess ||
-      hipStreamWaitEvent(sc.side, sc.fork, 0) != hipSuccess)
+  const bool fork = sc.side != nullptr ||
+                    (capture == hipStreamCaptureStatusNone && sc.ensure_side());
+  if (fork && (hipEventRecord(sc.fork, stream) != hipSuccess ||
+               hipStreamWaitEvent(sc.side, sc.fork, 0) != hipSuccess))
     return SXD_ERR_DEVICE;
-  int rc = launch_mortar_packages(gh, d->plan, d->d_el, u, params, inv_jac, sc.temps, sc.side);
-  if (rc == SXD_OK) rc = launch_mortar_boundary_terms(gh, d->plan, sc.temps, sc.side);
-  const int rc_volume = volume(stream);
+  const int rc_faces = launch_mortar_lifted_corrections(true, d->plan, d->d_el, u, params, inv_jac,
+                                                        w.corr, fork ? sc.side : stream);
+  const int rc = launch_ragged_gh_state(d->num_elements, d->d_list, d->d_el, d->np_max, u, params,
+                                        state, stream);
   // join in every case, so that no work of this call is left on the side
   // stream after it returns
-  if (hipEventRecord(sc.join, sc.side) != hipSuccess ||
-      hipStreamWaitEvent(stream, sc.join, 0) != hipSuccess)
+  if (fork && (hipEventRecord(sc.join, sc.side) != hipSuccess ||
+               hipStreamWaitEvent(stream, sc.join, 0) != hipSuccess))
     return SXD_ERR_DEVICE;
+  if (rc_faces != SXD_OK) return rc_faces;
   if (rc != SXD_OK) return rc;
-  if (rc_volume != SXD_OK) return rc_volume;
-  return launch_mortar_lift(gh, d->plan, d->d_el, dt, sc.temps, stream);
+  return launch_ragged_gh_volume(d->classes, d->d_list, d->d_el, u, params, inv_jac, dt, state,
+                                 d->plan.d_corrections, w.corr, stream);
 }
 
 int run_mixed(sxd_domain* d, Scratch& sc, bool gh, int kernel, const double* u,
@@ -1026,13 +1062,12 @@ int run_mixed(sxd_domain* d, Scratch& sc, bool gh, int kernel, const double* u,
   }
   const int threads = d->threads[gh ? SXD_SYSTEM_GH : SXD_SYSTEM_SCALAR_WAVE];
   if (kernel == SXD_KERNEL_MIXED_BATCHED)
-    return launch_mixed_rhs(gh, d->num_elements, d->d_list, d->d_el, d->d_nbr, d->np_max, d->kf,
-                            d->km, u, params, inv_jac, dt, scratch, threads, stream, ghost,
-                            bc_kind);
+    return launch_mixed_rhs(gh, d->classes, d->d_list, d->d_el, d->d_nbr, d->kf, d->km, u, params,
+                            inv_jac, dt, scratch, threads, stream, ghost, bc_kind);
   for (const auto& b : d->buckets) {
-    const int rc = launch_mixed_rhs(gh, b.second, d->d_buckets + b.first, d->d_el, d->d_nbr,
-                                    d->np_max, d->kf, d->km, u, params, inv_jac, dt, scratch,
-                                    threads, stream, ghost, bc_kind);
+    const int rc = launch_mixed_rhs(gh, {{0, b.second, d->np_max}}, d->d_buckets + b.first,
+                                    d->d_el, d->d_nbr, d->kf, d->km, u, params, inv_jac, dt,
+                                    scratch, threads, stream, ghost, bc_kind);
     if (rc != SXD_OK) return rc;
   }
   return SXD_OK;
@@ -1063,10 +1098,10 @@ int run_gh(sxd_domain* d, Scratch& sc, int kernel, const double* u, const double
                                kernel == SXD_KERNEL_FUSED ? kGhFusedValu : kGhFusedMfma,
                                d->threads[SXD_SYSTEM_GH] == 512 ? 512 : 256, ghost, stream);
   if (gh_pairs_supported(d->ext)) {
-    if (int rc = sc.reserve_pairs(gh_pairs_work_doubles(d->num_elements, d->ext)); rc != SXD_OK)
+    if (int rc = sc.reserve_block(SXD_SYSTEM_GH, gh_pairs_work_doubles(d->num_elements, d->ext)); rc != SXD_OK)
       return rc;
     return launch_gh_rhs_pairs(d->num_elements, d->ext, d->d_nbr, u, gammas, inv_jac, dt,
-                               sc.pairs, ghost, stream);
+                               sc.block[SXD_SYSTEM_GH], ghost, stream);
   }
   const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];
   if (int rc = reserve_scratch(sc, 150 * np * d->num_elements, 12 * np * d->num_elements);
@@ -1325,8 +1360,7 @@ int sxd_rhs_begin(const sxd_domain* domain, int system, const double* u, const d
   const size_t du = gh ? 150 * static_cast<size_t>(d->total_points) : 0;
   int rc = reserve_scratch(sc, du, mortar_work_doubles(gh, d->plan));
   if (rc == SXD_OK)
-    rc = launch_mixed_volume(gh, d->num_elements, d->d_list, d->d_el, d->np_max, u, params,
-                             inv_jac, dt, sc.du, d->threads[system], s);
+    rc = run_ragged_volume(d, gh, u, params, inv_jac, dt, sc.du, s);
   if (rc == SXD_OK)
     rc = launch_mortar_packages(gh, d->plan, d->d_el, u, params, inv_jac, sc.temps, s);
   if (rc == SXD_OK) rc = launch_mortar_pack(gh, d->plan, sc.temps, send, time_step_id, s);
@@ -1470,8 +1504,8 @@ int sxd_gh_rhs_bjorhus(const sxd_domain* domain, int bjorhus_type, const double*
     if (int rc = reserve_scratch(sc, 150 * static_cast<size_t>(d->total_points), 0); rc != SXD_OK)
       return finish(rc, __func__);
     const int threads = d->threads[SXD_SYSTEM_GH];
-    int rc = launch_mixed_volume(true, d->num_elements, d->d_list, d->d_el, d->np_max, u, gammas,
-                                 inv_jac, dt, sc.du, threads, s);
+    int rc = launch_mixed_gh_volume_du(d->num_elements, d->d_list, d->d_el, d->np_max, u, gammas,
+                                       inv_jac, dt, sc.du, threads, s);
     if (rc == SXD_OK)
       rc = launch_gh_bjorhus_mixed_faces(d->num_elements, physical, d->d_list, d->d_el, d->d_nbr,
                                          u, sc.du, gammas, inv_jac, coords, dt, s);

@@ -58,25 +58,28 @@ __device__ __forceinline__ unsigned divisor(int n) {
   return ((1u << 20) + static_cast<unsigned>(n) - 1) / static_cast<unsigned>(n);
 }
 
+// RAGGED: grid (list length, chunks of 128 points of the largest element).
 template <bool RAGGED>
 __global__ void __launch_bounds__(128)
 gh_state_kernel(int64_t total, int n0, int n1, int n2, const MixedElement* __restrict__ el,
-                const int32_t* __restrict__ point_el, const double* __restrict__ u,
+                const int32_t* __restrict__ list, const double* __restrict__ u,
                 const double* __restrict__ gammas, const double* __restrict__ inv_jac,
                 double* __restrict__ state, double* __restrict__ sides) {
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= total) return;
   int64_t off;
-  int np;
+  int np, p;
   if constexpr (RAGGED) {
-    const MixedElement& m = el[point_el[gid]];
+    const MixedElement& m = el[list[blockIdx.x]];
     off = m.off;
     np = m.np;
+    p = blockIdx.y * blockDim.x + threadIdx.x;
+    if (p >= np) return;
   } else {
+    const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (gid >= total) return;
     np = n0 * n1 * n2;
     off = gid / np * np;
+    p = static_cast<int>(gid - off);
   }
-  const int p = static_cast<int>(gid - off);
   const double* ue = u + 50 * off + p;
   const double* ga = gammas + 3 * off + p;
   double up[50];
@@ -174,6 +177,8 @@ __host__ __device__ inline int pair_lds_doubles(int n0, int n1, int n2, bool fac
 // FACES (uniform domains): faces whose neighbour is -1 take the ghost state
 // [E][50][Np] as exterior state, as gh_face_pass_kernel does; their
 // corrections are added before those of the internal faces.
+// RAGGED: with a table of lifted corrections (launch_ragged_gh_volume) those of
+// the faces a point lies on are added, each face's mortars in order.
 template <bool RAGGED, bool FACES>
 __global__ void __launch_bounds__(512)
 gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __restrict__ el,
@@ -181,7 +186,8 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
                const double* __restrict__ u, const double* __restrict__ gammas,
                const double* __restrict__ inv_jac, const double* __restrict__ state,
                const double* __restrict__ sides, const double* __restrict__ ghost,
-               double* __restrict__ dt, const double* __restrict__ dtab) {
+               double* __restrict__ dt, const double* __restrict__ dtab,
+               const MortarCorrection* __restrict__ table, const double* __restrict__ corr) {
   extern __shared__ double s_lds[];
   int64_t e, off;
   int pr;
@@ -192,10 +198,10 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
     const int at = slot / 10 * kNumXcds + x;
     if (at >= num_elements) return;
     pr = slot % 10;
-    const MixedElement m = el[list[at]];
+    e = list[at];
+    const MixedElement m = el[e];
     n0 = m.n[0], n1 = m.n[1], n2 = m.n[2];
     off = m.off;
-    e = 0;
   } else {
     const int64_t item = xcd_local_element(blockIdx.x, gridDim.x);
     e = item / 10;
@@ -347,6 +353,20 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
         for (int c = 0; c < 5; ++c) out[c] = out[c] + bc[c];
       }
     }
+    if constexpr (RAGGED) {
+      if (table != nullptr) {
+        for (int d = 0; d < 3; ++d) {
+          const int at = d == 0 ? i : d == 1 ? j : k, nd = d == 0 ? n0 : d == 1 ? n1 : n2;
+          if (at != 0 && at != nd - 1) continue;
+          const int nf = d == 0 ? nf0 : d == 1 ? nf1 : nf2;
+          const MortarCorrection t = table[6 * e + 2 * d + (at == 0 ? 0 : 1)];
+          const double* from = corr + 50 * t.off + face_index(n0, n1, d, i, j, k);
+          for (int q = 0; q < t.count; ++q, from += 50 * nf)
+#pragma unroll
+            for (int c = 0; c < 5; ++c) out[c] = out[c] + from[comp[c] * nf];
+        }
+      }
+    }
     double* dte = dt + 50 * off;
 #pragma unroll
     for (int c = 0; c < 5; ++c) (dte + comp[c] * np)[p] = out[c];
@@ -421,8 +441,40 @@ int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* n
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   hipLaunchKernelGGL((gh_pair_kernel<false, true>), dim3(10 * num_elements),
                      dim3(pair_threads(np)), lds, stream, num_elements, ext[0], ext[1], ext[2],
-                     nullptr, nullptr, nbr, u, gammas, inv_jac, work, sides, ghost, dt, dtab);
+                     nullptr, nullptr, nbr, u, gammas, inv_jac, work, sides, ghost, dt, dtab, nullptr, nullptr);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+}
+
+int launch_ragged_gh_state(int count, const int32_t* list, const MixedElement* el, int np_max,
+                           const double* u, const double* gammas, double* state,
+                           hipStream_t stream) {
+  if (count == 0) return SXD_OK;
+  if (state == nullptr) return SXD_ERR_INVALID_ARGUMENT;
+  hipLaunchKernelGGL(gh_state_kernel<true>, dim3(count, (np_max + 127) / 128), dim3(128), 0,
+                     stream, 0, 0, 0, 0, el, list, u, gammas, nullptr, state, nullptr);
+  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+}
+
+int launch_ragged_gh_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+                            const MixedElement* el, const double* u, const double* gammas,
+                            const double* inv_jac, double* dt, const double* state,
+                            const MortarCorrection* table, const double* corr,
+                            hipStream_t stream) {
+  const double* dtab = device_diff_matrices();
+  if (dtab == nullptr) return SXD_ERR_DEVICE;
+  if (state == nullptr) return SXD_ERR_INVALID_ARGUMENT;
+  const void* kernel = reinterpret_cast<const void*>(&gh_pair_kernel<true, false>);
+  for (const RaggedClass& c : classes) {
+    const int lds = (kPairStride * c.np_max + kStagedDiffDoubles) * 8;
+    if (!allow_lds(kernel, lds)) return SXD_ERR_UNSUPPORTED;
+    const int blocks = (c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10;
+    hipLaunchKernelGGL((gh_pair_kernel<true, false>), dim3(blocks),
+                       dim3(c.np_max > 768 ? 384 : c.np_max > 128 ? 256 : 128), lds, stream,
+                       c.count, 0, 0, 0, el, list + c.begin, nullptr, u, gammas, inv_jac, state,
+                       nullptr, nullptr, dt, dtab, table, corr);
+    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  }
+  return SXD_OK;
 }
 
 }  // namespace sxd

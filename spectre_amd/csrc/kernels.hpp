@@ -107,6 +107,7 @@ int launch_gh_rhs_fused(int num_elements, const int32_t ext[3], const int32_t* n
                         double* dt, int variant, int threads, const double* ghost,
                         hipStream_t stream);
 // Mixed p.  Per-element record of the ragged layout.
+struct MortarCorrection;
 struct MixedElement {
   int32_t n[3];  // LGL extents
   int32_t np;    // n0 n1 n2
@@ -115,23 +116,45 @@ struct MixedElement {
 const double* device_mortar_matrices();
 // LDS bytes of the face kernel for faces of <= kf and mortars of <= km points.
 int mixed_face_lds_bytes(int kf, int km);
-// Volume terms and mortar-coupled boundary corrections of the `count`
-// elements in `list` (one workgroup each, `threads` threads: 64, 128, 256).
-// gh: params = gammas [3][Np_e], scratch_du = 150 x total points; otherwise
-// params = gamma2 [Np_e].  Faces whose neighbour is -1 take their exterior
-// state by bc_kind: kSwBcGhostArray from ghost (ragged [nc][Np_e], read at the
-// face's own points); for ScalarWave also kSwBcSommerfeld (ghost unused) and
-// kSwBcBaylissTurkel (ghost = ragged [3][Np_e] coordinates).
-int launch_mixed_rhs(bool gh, int count, const int32_t* list, const MixedElement* el,
-                     const int32_t* nbr, int np_max, int kf, int km, const double* u,
-                     const double* params, const double* inv_jac, double* dt, double* scratch_du,
+// Elements of similar size in a work list: [begin, begin + count), at most
+// np_max points each.
+struct RaggedClass {
+  int begin, count, np_max;
+};
+// Volume terms and mortar-coupled boundary corrections of the elements in
+// `list` (all of its classes; face kernels: one workgroup each, `threads`
+// threads: 64, 128, 256).  gh: params = gammas [3][Np_e], state =
+// kGhStateDoubles x total points; otherwise params = gamma2 [Np_e].  Faces
+// whose neighbour is -1 take their exterior state by bc_kind: kSwBcGhostArray
+// from ghost (ragged [nc][Np_e], read at the face's own points); for ScalarWave
+// also kSwBcSommerfeld (ghost unused) and kSwBcBaylissTurkel (ghost = ragged
+// [3][Np_e] coordinates).
+int launch_mixed_rhs(bool gh, const std::vector<RaggedClass>& classes, const int32_t* list,
+                     const MixedElement* el, const int32_t* nbr, int kf, int km, const double* u,
+                     const double* params, const double* inv_jac, double* dt, double* state,
                      int threads, hipStream_t stream, const double* ghost = nullptr,
                      int bc_kind = kSwBcGhostArray);
-// The volume terms alone of launch_mixed_rhs (dt = point-wise terms).
-int launch_mixed_volume(bool gh, int count, const int32_t* list, const MixedElement* el,
-                        int np_max, const double* u, const double* params,
-                        const double* inv_jac, double* dt, double* scratch_du, int threads,
-                        hipStream_t stream);
+// The GH volume terms of launch_mixed_rhs through the derivative array (du = 150 x
+// total points, left filled for a condition that reads it).
+int launch_mixed_gh_volume_du(int count, const int32_t* list, const MixedElement* el, int np_max,
+                              const double* u, const double* params, const double* inv_jac,
+                              double* dt, double* du, int threads, hipStream_t stream);
+// Volume terms of the listed elements (dt = point-wise terms), one launch per
+// class, with the lifted corrections of their faces added in direction order
+// where a table of them is given (corr: MortarCorrectionsWork).  GH: state =
+// kGhStateDoubles x total points, as launch_ragged_gh_state fills it.
+int launch_ragged_gh_state(int count, const int32_t* list, const MixedElement* el, int np_max,
+                           const double* u, const double* gammas, double* state,
+                           hipStream_t stream);
+int launch_ragged_gh_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+                            const MixedElement* el, const double* u, const double* gammas,
+                            const double* inv_jac, double* dt, const double* state,
+                            const MortarCorrection* table, const double* corr,
+                            hipStream_t stream);
+int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+                            const MixedElement* el, const double* u, const double* gamma2,
+                            const double* inv_jac, double* dt, const MortarCorrection* table,
+                            const double* corr, hipStream_t stream);
 // The GH face corrections alone of launch_mixed_rhs, one launch per dimension,
 // for the faces that `phase` selects (kFacesAll, kFacesExternal with the ghost
 // state, kFacesInternal).
@@ -162,6 +185,18 @@ struct MortarFace {
 struct MortarRecord {
   int32_t face, partner, na, nb, ka, kb, size_a, size_b;
   int64_t mortar_off, rec_off, recv_off;
+  int64_t corr_off;  // offset of its lifted corrections among all records' face points
+};
+// The lifted corrections of one face of an element: those of its `count`
+// mortars, [nc][face points] each, back to back from face point `off`.
+struct MortarCorrection {
+  int64_t off;
+  int32_t count, pad;
+};
+// Mortars launched together: [begin, begin + count) of d_pairs, and the largest
+// LDS of one of them (ScalarWave, GH).
+struct MortarClass {
+  int begin, count, lds_bytes[2];
 };
 // Boundary messages (the BoundaryMessage of
 // Evolution/DiscontinuousGalerkin/Messages/BoundaryMessage.hpp for DG mortar
@@ -212,6 +247,10 @@ struct MortarPlan {
   // largest face, ka nb, and ka na + kb nb (matrix doubles) among the direct faces
   int direct_nf = 0, direct_tmp = 1, direct_mat = 0;
   int64_t face_points = 0, projected_points = 0, record_points = 0, remote_points = 0;
+  // plans without remote mortars: the lifted corrections of mortar_faces.hip
+  int64_t corr_points = 0;
+  std::vector<MortarClass> classes;
+  MortarCorrection* d_corrections = nullptr;  // per element and direction
   int64_t message_bytes[2] = {0, 0};  // the whole send buffer, per system
   std::vector<MortarPeer> peers;      // outgoing groups, ascending rank
   std::map<int, int> expected;        // messages expected from each rank
@@ -243,14 +282,20 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
                       MortarPlan* plan, std::string* error);
 void destroy_mortar_plan(MortarPlan* plan);
 size_t mortar_work_doubles(bool gh, const MortarPlan& plan);
-// Boundary corrections of every mortar added into dt (after the volume
-// terms); work: mortar_work_doubles(gh, plan) doubles.
-int launch_mortar_faces(bool gh, const MortarPlan& plan, const MixedElement* el, const double* u,
-                        const double* params, const double* inv_jac, double* dt, double* work,
-                        hipStream_t stream);
-// The two halves of launch_mortar_faces around a boundary-message exchange:
-// the packages of every mortar, then (with the remote packages received) the
-// corrections.
+// The corrections of a plan without remote mortars (mortar_faces.hip), lifted and ready to be
+// added into dt by the volume kernels (launch_ragged_volume).
+int mortar_corrections_lds_bytes(bool gh, const MortarRecord& r, const MortarRecord& partner);
+struct MortarCorrectionsWork {
+  double *corr, *sides, *speeds;
+  size_t doubles;
+  MortarCorrectionsWork(bool gh, const MortarPlan& plan, double* work);
+};
+int launch_mortar_lifted_corrections(bool gh, const MortarPlan& plan, const MixedElement* el,
+                                     const double* u, const double* params,
+                                     const double* inv_jac, double* work, hipStream_t stream);
+// The boundary corrections around a boundary-message exchange: the packages of
+// every mortar, then (with the remote packages received) the corrections, added
+// into dt after the volume terms; work: mortar_work_doubles(gh, plan) doubles.
 int launch_mortar_packages(bool gh, const MortarPlan& plan, const MixedElement* el,
                            const double* u, const double* params, const double* inv_jac,
                            double* work, hipStream_t stream);

@@ -29,6 +29,7 @@
 // product and then fused multiply-adds, as in the oracle.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <vector>
@@ -79,15 +80,100 @@ __device__ __forceinline__ void logical_derivs(const double* sc, const MixedElem
 }
 
 // ---------------------------------------------------------------------------
-// ScalarWave volume terms.  Dynamic LDS: 5 Np_max doubles.  CPSR: external
+// ScalarWave volume terms, one workgroup per element, with the lifted
+// corrections of its faces added in direction order where `table` is given (a
+// face's mortars in order), so that dt is written once.  The five fields of a
+// point lie next to each other in LDS, so that a pencil step reads them at one
+// address.  Dynamic LDS: 5 Np_max doubles, then the D matrices.  Bound by HBM
+// (20 doubles per point and the corrections); its LDS is sized by a class of
+// elements of similar size and its workgroups are as large as the class
+// allows, since 1000 elements are four per CU: extents 4 .. 12 took 138 us with
+// one LDS size for all and 128 threads.
+__global__ void __launch_bounds__(512)
+sw_ragged_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __restrict__ list,
+                        const double* __restrict__ u, const double* __restrict__ gamma2,
+                        const double* __restrict__ inv_jac, double* __restrict__ dt,
+                        const double* __restrict__ dtab,
+                        const MortarCorrection* __restrict__ table,
+                        const double* __restrict__ corr) {
+  extern __shared__ double s_lds[];
+  const int e = list[blockIdx.x];
+  const MixedElement m = el[e];
+  const int np = m.np, n0 = m.n[0], n1 = m.n[1], n2 = m.n[2];
+  const double* D[3];
+  stage_diff_matrices(dtab, m.n, s_lds + 5 * np, D);
+  const double* ue = u + 5 * m.off;
+  for (unsigned p = threadIdx.x; p < static_cast<unsigned>(np); p += blockDim.x) {
+    double v[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) v[c] = (ue + c * np)[p];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) s_lds[5 * p + c] = v[c];
+  }
+  __syncthreads();
+  const double* ij = inv_jac + 9 * m.off;
+  const double* g2 = gamma2 + m.off;
+  double* dte = dt + 5 * m.off;
+  for (unsigned p = threadIdx.x; p < static_cast<unsigned>(np); p += blockDim.x) {
+    const int row = p / n0, k = row / n1;
+    const int i = p - row * n0, j = row - k * n1;
+    double der[5][3];
+    auto sums = [&](int d, int n, const double* w, const double* x, int step) {
+#pragma unroll
+      for (int c = 0; c < 5; ++c) der[c][d] = w[0] * x[c];
+#pragma unroll 2
+      for (int l = 1; l < n; ++l) {
+        x += step;
+        const double a = w[l];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) der[c][d] = fma(a, x[c], der[c][d]);
+      }
+    };
+    sums(0, n0, D[0] + i * n0, s_lds + 5 * row * n0, 5);
+    sums(1, n1, D[1] + j * n1, s_lds + 5 * (i + n0 * n1 * k), 5 * n0);
+    sums(2, n2, D[2] + k * n2, s_lds + 5 * (i + n0 * j), 5 * n0 * n1);
+    double up[5], dup[15], out[5], w[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) w[c] = (ij + c * np)[p];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      up[c] = s_lds[5 * p + c];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        double s = w[ij3(0, a)] * der[c][0];
+        s = fma(w[ij3(1, a)], der[c][1], s);
+        s = fma(w[ij3(2, a)], der[c][2], s);
+        dup[3 * c + a] = s;
+      }
+    }
+    sw_time_derivative(out, up, dup, g2[p]);
+    if (table != nullptr) {
+      for (int d = 0; d < 3; ++d) {
+        const int at = d == 0 ? i : d == 1 ? j : k, nd = d == 0 ? n0 : d == 1 ? n1 : n2;
+        if (at != 0 && at != nd - 1) continue;
+        const int nf = d == 0 ? n1 * n2 : d == 1 ? n0 * n2 : n0 * n1;
+        const int f = d == 0 ? j + n1 * k : d == 1 ? i + n0 * k : i + n0 * j;
+        const MortarCorrection t = table[6 * e + 2 * d + (at == 0 ? 0 : 1)];
+        const double* from = corr + 5 * t.off + f;
+        for (int q = 0; q < t.count; ++q, from += 5 * nf)
+#pragma unroll
+          for (int c = 0; c < 5; ++c) out[c] = out[c] + from[c * nf];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) (dte + c * np)[p] = out[c];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// ScalarWave volume terms of domains whose external
 // faces (neighbour -1) are closed by the constraint-preserving spherical
 // radiation condition of type bc_kind (kSwBcCpsr*; coords = ragged [3][Np_e]
 // for the Bayliss-Turkel types), a time-derivative condition: a point on such
 // faces adds their dt Pi corrections, in direction order, to its volume terms
-// (the face kernel then skips those faces).
-template <bool CPSR>
+// (the face kernel then skips those faces).  Dynamic LDS: 5 Np_max doubles.
 __global__ void __launch_bounds__(256)
-sw_mixed_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __restrict__ list,
+sw_mixed_cpsr_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __restrict__ list,
                        const double* __restrict__ u, const double* __restrict__ gamma2,
                        const double* __restrict__ inv_jac, double* __restrict__ dt,
                        const double* __restrict__ dtab, const int32_t* __restrict__ nbr,
@@ -121,23 +207,21 @@ sw_mixed_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __res
     }
     double dtp[5];
     sw_time_derivative(dtp, up, dup, gamma2[m.off + p]);
-    if constexpr (CPSR) {
-      const int at[3] = {i, j, k};
-      for (int dir = 0; dir < 6; ++dir) {
-        const int d = dir >> 1, side = dir & 1;
-        if (at[d] != (side == 0 ? 0 : ext_at(m, d) - 1) || nbr[6 * e + dir] >= 0) continue;
-        double n[3], mag;
+    const int at[3] = {i, j, k};
+    for (int dir = 0; dir < 6; ++dir) {
+      const int d = dir >> 1, side = dir & 1;
+      if (at[d] != (side == 0 ? 0 : ext_at(m, d) - 1) || nbr[6 * e + dir] >= 0) continue;
+      double n[3], mag;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          n[a] = ij[ij3(d, a) * np + p];
-          if (side == 0) n[a] = n[a] * -1.0;
-        }
-        flat_normalize(n, &mag);
-        dtp[1] = dtp[1] + sw_cpsr_correction(bc_kind, up, dup, n, gamma2[m.off + p],
-                                             coords != nullptr ? coords + 3 * m.off + p
-                                                               : nullptr,
-                                             np);
+      for (int a = 0; a < 3; ++a) {
+        n[a] = ij[ij3(d, a) * np + p];
+        if (side == 0) n[a] = n[a] * -1.0;
       }
+      flat_normalize(n, &mag);
+      dtp[1] = dtp[1] + sw_cpsr_correction(bc_kind, up, dup, n, gamma2[m.off + p],
+                                           coords != nullptr ? coords + 3 * m.off + p
+                                                             : nullptr,
+                                           np);
     }
 #pragma unroll
     for (int c = 0; c < 5; ++c) dt[5 * m.off + c * np + p] = dtp[c];
@@ -1148,9 +1232,7 @@ bool enable_large_lds() {
   if (static_cast<int>(done.size()) <= dev) done.resize(dev + 1, false);
   if (done[dev]) return true;
   const int lds_max = 160 * 1024;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&sw_mixed_volume_kernel<false>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&sw_mixed_volume_kernel<true>),
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&sw_mixed_cpsr_volume_kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
       hipFuncSetAttribute(reinterpret_cast<const void*>(&sw_mixed_face_kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
@@ -1173,38 +1255,47 @@ bool enable_large_lds() {
 
 int mixed_face_lds_bytes(int kf, int km) { return FacePlan(kf, km, 13).total * 8; }
 
-int launch_mixed_volume(bool gh, int count, const int32_t* list, const MixedElement* el,
-                        int np_max, const double* u, const double* params,
-                        const double* inv_jac, double* dt, double* scratch_du, int threads,
-                        hipStream_t stream) {
+int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+                            const MixedElement* el, const double* u, const double* gamma2,
+                            const double* inv_jac, double* dt, const MortarCorrection* table,
+                            const double* corr, hipStream_t stream) {
+  const double* dtab = device_diff_matrices();
+  if (dtab == nullptr) return SXD_ERR_DEVICE;
+  for (const RaggedClass& c : classes) {
+    const int lds = (5 * c.np_max + kStagedDiffDoubles) * 8;
+    if (!allow_lds(reinterpret_cast<const void*>(&sw_ragged_volume_kernel), lds))
+      return SXD_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL(sw_ragged_volume_kernel, dim3(c.count),
+                       dim3(c.np_max > 256 ? 512 : c.np_max > 128 ? 256 : 128), lds, stream, el,
+                       list + c.begin, u, gamma2, inv_jac, dt, dtab, table, corr);
+    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  }
+  return SXD_OK;
+}
+
+int launch_mixed_gh_volume_du(int count, const int32_t* list, const MixedElement* el, int np_max,
+                              const double* u, const double* params, const double* inv_jac,
+                              double* dt, double* du, int threads, hipStream_t stream) {
   if (count == 0) return SXD_OK;
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   if (threads != 64 && threads != 128 && threads != 256) return SXD_ERR_INVALID_ARGUMENT;
   if (!enable_large_lds()) return SXD_ERR_DEVICE;
-  if (!gh) {
-    if (5 * np_max * 8 > 160 * 1024) return SXD_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(sw_mixed_volume_kernel<false>, dim3(count), dim3(threads),
-                       5 * np_max * 8, stream, el, list, u, params, inv_jac, dt, dtab, nullptr,
-                       kSwBcGhostArray, nullptr);
-    return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
-  }
-  if (scratch_du == nullptr) return SXD_ERR_INVALID_ARGUMENT;
+  if (du == nullptr) return SXD_ERR_INVALID_ARGUMENT;
   hipLaunchKernelGGL(ragged_partial_derivatives_kernel,
                      dim3(count, (50 + kRaggedChunk - 1) / kRaggedChunk), dim3(threads),
-                     (kStagedDiffDoubles + np_max) * 8, stream, el, list, 50, u, inv_jac,
-                     scratch_du, dtab);
+                     (kStagedDiffDoubles + np_max) * 8, stream, el, list, 50, u, inv_jac, du,
+                     dtab);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   hipLaunchKernelGGL(gh_mixed_pointwise_kernel, dim3(count), dim3(threads), 0, stream, el, list,
-                     u, scratch_du, params, dt);
+                     u, du, params, dt);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 
-int launch_mixed_rhs(bool gh, int count, const int32_t* list, const MixedElement* el,
-                     const int32_t* nbr, int np_max, int kf, int km, const double* u,
-                     const double* params, const double* inv_jac, double* dt, double* scratch_du,
+int launch_mixed_rhs(bool gh, const std::vector<RaggedClass>& classes, const int32_t* list,
+                     const MixedElement* el, const int32_t* nbr, int kf, int km, const double* u,
+                     const double* params, const double* inv_jac, double* dt, double* state,
                      int threads, hipStream_t stream, const double* ghost, int bc_kind) {
-  if (count == 0) return SXD_OK;
   if (gh && bc_kind != kSwBcGhostArray) return SXD_ERR_INVALID_ARGUMENT;
   if (bc_kind < kSwBcGhostArray || bc_kind > kSwBcCpsrSecondOrderBt) return SXD_ERR_UNSUPPORTED;
   const double* dtab = device_diff_matrices();
@@ -1214,36 +1305,37 @@ int launch_mixed_rhs(bool gh, int count, const int32_t* list, const MixedElement
   const int face_lds = mixed_face_lds_bytes(kf, km);
   if (face_lds > 160 * 1024) return SXD_ERR_UNSUPPORTED;
   if (!enable_large_lds()) return SXD_ERR_DEVICE;
+  int count = 0, np_max = 0;
+  for (const RaggedClass& c : classes) {
+    count += c.count;
+    np_max = std::max(np_max, c.np_max);
+  }
   if (!gh) {
     const int sw_face_lds = SwFacePlan(kf, km).total * 8;
-    if (5 * np_max * 8 > 160 * 1024) return SXD_ERR_UNSUPPORTED;
-    if (bc_kind >= kSwBcCpsrSommerfeld)
-      hipLaunchKernelGGL(sw_mixed_volume_kernel<true>, dim3(count), dim3(threads),
-                         5 * np_max * 8, stream, el, list, u, params, inv_jac, dt, dtab, nbr,
-                         bc_kind, ghost);
-    else
-      hipLaunchKernelGGL(sw_mixed_volume_kernel<false>, dim3(count), dim3(threads),
-                         5 * np_max * 8, stream, el, list, u, params, inv_jac, dt, dtab, nbr,
-                         bc_kind, nullptr);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    if (bc_kind >= kSwBcCpsrSommerfeld) {
+      if (5 * np_max * 8 > 160 * 1024) return SXD_ERR_UNSUPPORTED;
+      hipLaunchKernelGGL(sw_mixed_cpsr_volume_kernel, dim3(count), dim3(threads), 5 * np_max * 8,
+                         stream, el, list, u, params, inv_jac, dt, dtab, nbr, bc_kind, ghost);
+      if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    } else if (const int rc = launch_ragged_sw_volume(classes, list, el, u, params, inv_jac, dt,
+                                                      nullptr, nullptr, stream);
+               rc != SXD_OK) {
+      return rc;
+    }
     hipLaunchKernelGGL(sw_mixed_face_kernel, dim3(count), dim3(threads), sw_face_lds, stream,
                        el, list, nbr, u, params, inv_jac, dt, mtab, kf, km, ghost, bc_kind);
     return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
   }
-  if (scratch_du == nullptr) return SXD_ERR_INVALID_ARGUMENT;
-  hipLaunchKernelGGL(ragged_partial_derivatives_kernel,
-                     dim3(count, (50 + kRaggedChunk - 1) / kRaggedChunk), dim3(threads),
-                     (kStagedDiffDoubles + np_max) * 8, stream, el, list, 50, u, inv_jac,
-                     scratch_du, dtab);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(gh_mixed_pointwise_kernel, dim3(count), dim3(threads), 0, stream, el, list,
-                     u, scratch_du, params, dt);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  int rc = launch_ragged_gh_state(count, list, el, np_max, u, params, state, stream);
+  if (rc != SXD_OK) return rc;
+  rc = launch_ragged_gh_volume(classes, list, el, u, params, inv_jac, dt, state, nullptr, nullptr,
+                               stream);
+  if (rc != SXD_OK) return rc;
   // with external faces: a sweep over the external faces, then one over the
   // internal ones (the order in which the corrections reach dt)
   if (ghost != nullptr) {
-    const int rc = launch_mixed_gh_face_passes(count, list, el, nbr, kf, km, u, params, inv_jac,
-                                               dt, threads, ghost, kFacesExternal, stream);
+    rc = launch_mixed_gh_face_passes(count, list, el, nbr, kf, km, u, params, inv_jac, dt, threads,
+                                     ghost, kFacesExternal, stream);
     if (rc != SXD_OK) return rc;
     return launch_mixed_gh_face_passes(count, list, el, nbr, kf, km, u, params, inv_jac, dt,
                                        threads, ghost, kFacesInternal, stream);

@@ -15,9 +15,11 @@
 // its face (projection_matrix_child_to_parent) and lifts it (dg::lift_flux),
 // one mortar after another.
 //
-// Here every element's packages stay in HBM and the receiver gathers the
-// partner's package through a per-record index table (the partner's
-// oriented offsets, inverted on the host), so no data is reordered:
+// Two organisations.  Where every mortar is local, mortar_faces.hip takes each
+// mortar from the fields to both sides' lifted corrections in one workgroup.
+// Here, around an exchange of boundary messages, the packages stay in HBM between the steps and the
+// receiver gathers the partner's package through a per-record index table (the
+// partner's oriented offsets, inverted on the host), so no data is reordered:
 //   1. mortar_package_kernel: one workgroup per face, the package of every
 //      face point and |n| (SW 13 values, GH 10 pairs x 13 + 4 speeds);
 //      mortar_direct_kernel instead for a face whose single mortar differs
@@ -776,7 +778,7 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
   std::vector<int32_t> gather, proj;
   std::vector<MortarMessage> messages;
   std::vector<MortarRecvKey> keys;
-  int64_t face_pts = 0, proj_pts = 0, rec_pts = 0, recv_pts = 0;
+  int64_t face_pts = 0, proj_pts = 0, rec_pts = 0, recv_pts = 0, corr_pts = 0;
   int64_t msg_bytes[2] = {0, 0};
   int dim_begin[4] = {0, 0, 0, 0};
   for (int i = 0; i < kept; ++i) {
@@ -814,6 +816,8 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
     }
     m.rec_off = rec_pts;
     rec_pts += km;
+    m.corr_off = corr_pts;
+    corr_pts += r.na * r.nb;
     // my mortar point k reads the partner's point offsets[k]: the partner's
     // oriented offsets map its points to mine, mine map mine to its
     const std::vector<int32_t> g = oriented_offsets(r.ka, r.kb, r.dir / 2, r.o);
@@ -932,6 +936,37 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
     else if (recs[i].partner > i)
       pairs.push_back(i);
   }
+  // one workgroup per mortar (mortar_faces.hip), in classes of decreasing LDS
+  // size: 1, 2, 4 or 8 and more workgroups per CU.  Every mortar fits: faces
+  // have at most 193 points and mortars at most 20 x 20, so a side's staged
+  // values are at most 13 x 20 x 20 doubles, the face packages 13 x 386, and all
+  // of it with the matrices 145 KB.
+  std::vector<MortarCorrection> corrections;
+  if (keys.empty()) {
+    auto lds = [&](bool gh, int32_t i) {
+      return mortar_corrections_lds_bytes(gh, recs[i], recs[recs[i].partner]);
+    };
+    std::stable_sort(pairs.begin(), pairs.end(),
+                     [&](int32_t x, int32_t y) { return lds(true, x) > lds(true, y); });
+    auto per_cu = [&](int32_t i) {
+      const int fit = 160 * 1024 / lds(true, i);
+      return fit >= 8 ? 8 : fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
+    };
+    for (int i = 0; i < static_cast<int>(pairs.size());) {
+      MortarClass c{i, 0, {0, 0}};
+      while (i < static_cast<int>(pairs.size()) && per_cu(pairs[i]) == per_cu(pairs[c.begin])) {
+        c.lds_bytes[0] = std::max(c.lds_bytes[0], lds(false, pairs[i]));
+        c.lds_bytes[1] = std::max(c.lds_bytes[1], lds(true, pairs[i]));
+        ++c.count;
+        ++i;
+      }
+      plan->classes.push_back(c);
+    }
+    corrections.resize(6 * static_cast<size_t>(num_owned));
+    for (const MortarFace& f : faces)
+      corrections[6 * static_cast<size_t>(f.e) + f.dir] = {recs[f.rec_begin].corr_off,
+                                                           f.rec_count, 0};
+  }
   int kf = 0, km = 0, tmp_max = 1, mat_max = 0;
   for (const MortarRecord& m : recs) {
     kf = std::max(kf, m.na * m.nb);
@@ -956,6 +991,7 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
   plan->face_points = face_pts;
   plan->projected_points = proj_pts;
   plan->record_points = rec_pts;
+  plan->corr_points = corr_pts;
   for (int d = 0; d < 4; ++d) plan->dim_begin[d] = dim_begin[d];
   plan->kf = kf;
   plan->km = km;
@@ -979,6 +1015,7 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
   upload(&plan->d_direct, direct);
   upload(&plan->d_pairs, pairs);
   upload(&plan->d_remote_records, remote_records);
+  upload(&plan->d_corrections, corrections);
   upload(&plan->d_messages, messages);
   upload(&plan->d_keys, keys);
   if (rc != SXD_OK) {
@@ -997,6 +1034,7 @@ void destroy_mortar_plan(MortarPlan* plan) {
   if (plan->d_direct != nullptr) (void)hipFree(plan->d_direct);
   if (plan->d_pairs != nullptr) (void)hipFree(plan->d_pairs);
   if (plan->d_remote_records != nullptr) (void)hipFree(plan->d_remote_records);
+  if (plan->d_corrections != nullptr) (void)hipFree(plan->d_corrections);
   if (plan->d_messages != nullptr) (void)hipFree(plan->d_messages);
   if (plan->d_keys != nullptr) (void)hipFree(plan->d_keys);
   *plan = MortarPlan{};
@@ -1131,14 +1169,6 @@ int launch_mortar_corrections(bool gh, const MortarPlan& plan, const MixedElemen
                               double* dt, double* work, hipStream_t stream) {
   const int rc = launch_mortar_boundary_terms(gh, plan, work, stream);
   return rc != SXD_OK ? rc : launch_mortar_lift(gh, plan, el, dt, work, stream);
-}
-
-int launch_mortar_faces(bool gh, const MortarPlan& plan, const MixedElement* el, const double* u,
-                        const double* params, const double* inv_jac, double* dt, double* work,
-                        hipStream_t stream) {
-  if (plan.num_remote > 0) return SXD_ERR_UNSUPPORTED;
-  const int rc = launch_mortar_packages(gh, plan, el, u, params, inv_jac, work, stream);
-  return rc != SXD_OK ? rc : launch_mortar_corrections(gh, plan, el, dt, work, stream);
 }
 
 int launch_mortar_pack(bool gh, const MortarPlan& plan, double* work, void* send, int64_t step,

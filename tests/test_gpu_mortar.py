@@ -236,3 +236,41 @@ def test_boundary_message_checks():
 def directory_offset(group):
     """Byte offset of the group's first message (from its directory)."""
     return int(group[8:16].cpu().numpy().view(np.int64)[0])
+
+
+# The one-workgroup mortar kernel and the volume kernels' size classes at the
+# edges of their ranges: 20 x 20 mortars between 9 x 20 and 20 x 9 faces (conforming and
+# 2:1), the smallest elements, elements of every size class, and point counts
+# of one thread round and one point more (8^3 = 512, 513 = 9 x 19 x 3).
+EDGE_EXTENTS = {
+    "longest": [(9, 20, 9), (20, 9, 9)],
+    "smallest": [(2, 2, 2), (2, 3, 2), (20, 2, 2)],
+    "classes": [(3, 3, 3), (6, 7, 7), (8, 8, 8), (9, 19, 3), (9, 9, 9), (11, 12, 10), (13, 13, 13)],
+}
+
+
+@pytest.mark.parametrize("refine", [{}, {0: (0, 1)}, {1: (2,), 2: (0, 1, 2)}])
+@pytest.mark.parametrize("pattern", sorted(EDGE_EXTENTS))
+def test_mortar_corrections_route_edges(pattern, refine):
+    print(f"mortar edges {pattern} {refine}", flush=True)
+    rng = np.random.default_rng(len(pattern) + len(refine))
+    total = sum(1 << len(refine.get(c, ())) for c in range(4))
+    choices = EDGE_EXTENTS[pattern]
+    ext = [choices[i % len(choices)] for i in range(total)]
+    turns = [wl.ROTATIONS[i] for i in rng.integers(0, len(wl.ROTATIONS), size=total)]
+    if pattern == "longest":
+        turns = None  # faces stay within 193 points
+    brick = wl.MortarBrick((3.0, -4.0, -4.0), (11.0, 4.0, 4.0), (2, 2, 1), refine, ext, turns)
+    inv = brick.inverse_jacobian()
+    inv = inv + 1e-2 * rng.standard_normal(inv.shape)
+    u = brick.ragged([wl.gh_kerr_schild(brick.element_coordinates(e)[None])[0]
+                      for e in range(brick.num_elements)])
+    u = u * (1.0 + 1e-4 * rng.standard_normal(u.shape))
+    gammas = brick.ragged([np.stack([np.ones(n), -np.ones(n), np.ones(n)]) for n in brick.points])
+    domain = dg.MortarDomain.from_brick(brick)
+    ref = ol.gh_rhs_mortars(brick.extents, brick.records, u, gammas, inv)
+    assert np.array_equal(host(domain.gh_rhs(dev(u), dev(gammas), dev(inv))), ref)
+    su = rng.uniform(-1, 1, 5 * brick.total_points)
+    g2 = rng.uniform(0.2, 1.5, brick.total_points)
+    ref = ol.sw_rhs_mortars(brick.extents, brick.records, su, g2, inv)
+    assert np.array_equal(host(domain.scalar_wave_rhs(dev(su), dev(g2), dev(inv))), ref)
