@@ -693,18 +693,18 @@ int create_mixed_domain(sxd_domain** domain, int num_elements, const int32_t* ex
     d->buckets.emplace_back(i, j - i);
     i = j;
   }
-  // classes of the volume kernels, whose LDS a launch reserves for its largest
-  // element: up to 300, 600, 1000 and more points (12, 24, 40 KB and more of
-  // fields)
-  auto size_class = [&](int i) {
-    const int np = el[list[i]].np;
-    return np > 1000 ? 3 : np > 600 ? 2 : np > 300 ? 1 : 0;
-  };
+  // classes of the GH pair kernel, whose LDS a launch reserves for its largest
+  // element: four workgroups per CU of up to 910 points, fewer and larger ones
+  // beyond (1000 elements of extents 4 .. 12: 748 us in these two classes, 794 in
+  // four, 824 in one)
+  auto size_class = [&](int i) { return el[list[i]].np > 910 ? 1 : 0; };
   for (int i = 0; i < num_elements;) {
-    int j = i;
-    while (j < num_elements && size_class(j) == size_class(i)) ++j;
-    d->classes.push_back({i, j - i, el[list[i]].np});
-    i = j;
+    RaggedClass c{i, 0, el[list[i]].np, 0};
+    for (; i < num_elements && size_class(i) == size_class(c.begin); ++i, ++c.count) {
+      const int32_t* n = el[list[i]].n;
+      c.d_doubles = std::max(c.d_doubles, n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    }
+    d->classes.push_back(c);
   }
   d->mixed = true;
   d->has_boundary = has_boundary;
@@ -1065,8 +1065,8 @@ int run_mixed(sxd_domain* d, Scratch& sc, bool gh, int kernel, const double* u,
     return launch_mixed_rhs(gh, d->classes, d->d_list, d->d_el, d->d_nbr, d->kf, d->km, u, params,
                             inv_jac, dt, scratch, threads, stream, ghost, bc_kind);
   for (const auto& b : d->buckets) {
-    const int rc = launch_mixed_rhs(gh, {{0, b.second, d->np_max}}, d->d_buckets + b.first,
-                                    d->d_el, d->d_nbr, d->kf, d->km, u, params, inv_jac, dt,
+    const int rc = launch_mixed_rhs(gh, {{0, b.second, d->np_max, kStagedDiffDoubles}},
+                                    d->d_buckets + b.first, d->d_el, d->d_nbr, d->kf, d->km, u, params, inv_jac, dt,
                                     scratch, threads, stream, ghost, bc_kind);
     if (rc != SXD_OK) return rc;
   }

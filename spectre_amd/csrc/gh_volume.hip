@@ -320,6 +320,29 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
         else if (c == 1) dpi[a] = s;
         else dphi[a + 3 * (c - 2)] = s;
       }
+    // corrections of the point's faces, loaded together with its state: a
+    // face's first mortar here, further ones where they are added
+    bool on[3] = {false, false, false};
+    int mortars[3];
+    const double* from[3];
+    double first[3][5];
+    if constexpr (RAGGED) {
+      if (table != nullptr) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const int at = d == 0 ? i : d == 1 ? j : k, nd = d == 0 ? n0 : d == 1 ? n1 : n2;
+          on[d] = at == 0 || at == nd - 1;
+          if (!on[d]) continue;
+          const int nf = d == 0 ? nf0 : d == 1 ? nf1 : nf2;
+          const MortarCorrection lower = table[6 * e + 2 * d], upper = table[6 * e + 2 * d + 1];
+          mortars[d] = at == 0 ? lower.count : upper.count;
+          from[d] = corr + 50 * (at == 0 ? lower.off : upper.off) +
+                    face_index(n0, n1, d, i, j, k);
+#pragma unroll
+          for (int c = 0; c < 5; ++c) first[d][c] = from[d][comp[c] * nf];
+        }
+      }
+    }
     const double gamma1 = (ga + np)[p], gamma2 = (ga + 2 * np)[p];
     GhPointState st;
     st.lapse = (se + kLapse * np)[p];
@@ -355,15 +378,18 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
     }
     if constexpr (RAGGED) {
       if (table != nullptr) {
-        for (int d = 0; d < 3; ++d) {
-          const int at = d == 0 ? i : d == 1 ? j : k, nd = d == 0 ? n0 : d == 1 ? n1 : n2;
-          if (at != 0 && at != nd - 1) continue;
-          const int nf = d == 0 ? nf0 : d == 1 ? nf1 : nf2;
-          const MortarCorrection t = table[6 * e + 2 * d + (at == 0 ? 0 : 1)];
-          const double* from = corr + 50 * t.off + face_index(n0, n1, d, i, j, k);
-          for (int q = 0; q < t.count; ++q, from += 50 * nf)
 #pragma unroll
-            for (int c = 0; c < 5; ++c) out[c] = out[c] + from[comp[c] * nf];
+        for (int d = 0; d < 3; ++d) {
+          if (!on[d]) continue;
+          const double* src = from[d];
+#pragma unroll
+          for (int c = 0; c < 5; ++c) out[c] = out[c] + first[d][c];
+          const int nf = d == 0 ? nf0 : d == 1 ? nf1 : nf2;
+          for (int q = 1; q < mortars[d]; ++q) {
+            src += 50 * nf;
+#pragma unroll
+            for (int c = 0; c < 5; ++c) out[c] = out[c] + src[comp[c] * nf];
+          }
         }
       }
     }
@@ -465,11 +491,11 @@ int launch_ragged_gh_volume(const std::vector<RaggedClass>& classes, const int32
   if (state == nullptr) return SXD_ERR_INVALID_ARGUMENT;
   const void* kernel = reinterpret_cast<const void*>(&gh_pair_kernel<true, false>);
   for (const RaggedClass& c : classes) {
-    const int lds = (kPairStride * c.np_max + kStagedDiffDoubles) * 8;
+    const int lds = (kPairStride * c.np_max + c.d_doubles) * 8;
     if (!allow_lds(kernel, lds)) return SXD_ERR_UNSUPPORTED;
     const int blocks = (c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10;
     hipLaunchKernelGGL((gh_pair_kernel<true, false>), dim3(blocks),
-                       dim3(c.np_max > 768 ? 384 : c.np_max > 128 ? 256 : 128), lds, stream,
+                       dim3(c.np_max > 910 ? 512 : c.np_max > 128 ? 256 : 128), lds, stream,
                        c.count, 0, 0, 0, el, list + c.begin, nullptr, u, gammas, inv_jac, state,
                        nullptr, nullptr, dt, dtab, table, corr);
     if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;

@@ -117,9 +117,9 @@ const double* device_mortar_matrices();
 // LDS bytes of the face kernel for faces of <= kf and mortars of <= km points.
 int mixed_face_lds_bytes(int kf, int km);
 // Elements of similar size in a work list: [begin, begin + count), at most
-// np_max points each.
+// np_max points and d_doubles entries of their three D matrices each.
 struct RaggedClass {
-  int begin, count, np_max;
+  int begin, count, np_max, d_doubles;
 };
 // Volume terms and mortar-coupled boundary corrections of the elements in
 // `list` (all of its classes; face kernels: one workgroup each, `threads`
@@ -193,10 +193,26 @@ struct MortarCorrection {
   int64_t off;
   int32_t count, pad;
 };
-// Mortars launched together: [begin, begin + count) of d_pairs, and the largest
-// LDS of one of them (ScalarWave, GH).
+// A local mortar as mortar_faces.hip takes it: everything of its two sides in
+// one block, so that a workgroup starts with one load instead of a chain
+// through the record, face and element tables.
+struct MortarSide {
+  int64_t off;               // point offset of the element
+  int64_t pt_off, rec_off;   // face points, record points
+  int64_t corr_off;          // lifted corrections
+  int32_t np, nf, na, nb, ka, kb;
+  int32_t base, step_a, step_b;  // volume index of face point (a, b): base + a step_a + b step_b
+  int32_t mat_a, mat_b;      // matrix offsets in the Full table, -1 - offset in the half one
+  int32_t dim, side;         // the face
+  int32_t extent;            // the element's extent normal to the face
+};
+struct MortarJob {
+  MortarSide side[2];
+};
+// Mortars launched together: [begin, begin + count) of d_jobs, and the largest
+// LDS of one of them.
 struct MortarClass {
-  int begin, count, lds_bytes[2];
+  int begin, count, lds_bytes;
 };
 // Boundary messages (the BoundaryMessage of
 // Evolution/DiscontinuousGalerkin/Messages/BoundaryMessage.hpp for DG mortar
@@ -249,7 +265,8 @@ struct MortarPlan {
   int64_t face_points = 0, projected_points = 0, record_points = 0, remote_points = 0;
   // plans without remote mortars: the lifted corrections of mortar_faces.hip
   int64_t corr_points = 0;
-  std::vector<MortarClass> classes;
+  std::vector<MortarClass> classes[2];  // ScalarWave, GH
+  MortarJob* d_jobs = nullptr;
   MortarCorrection* d_corrections = nullptr;  // per element and direction
   int64_t message_bytes[2] = {0, 0};  // the whole send buffer, per system
   std::vector<MortarPeer> peers;      // outgoing groups, ascending rank

@@ -85,10 +85,9 @@ __device__ __forceinline__ void logical_derivs(const double* sc, const MixedElem
 // face's mortars in order), so that dt is written once.  The five fields of a
 // point lie next to each other in LDS, so that a pencil step reads them at one
 // address.  Dynamic LDS: 5 Np_max doubles, then the D matrices.  Bound by HBM
-// (20 doubles per point and the corrections); its LDS is sized by a class of
-// elements of similar size and its workgroups are as large as the class
-// allows, since 1000 elements are four per CU: extents 4 .. 12 took 138 us with
-// one LDS size for all and 128 threads.
+// (20 doubles per point and the corrections).  1000 elements are four workgroups
+// per CU, so the workgroups are large: extents 4 .. 12 take 25 us with 512
+// threads, against 138 with 128 and D read through the caches.
 __global__ void __launch_bounds__(512)
 sw_ragged_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __restrict__ list,
                         const double* __restrict__ u, const double* __restrict__ gamma2,
@@ -117,6 +116,27 @@ sw_ragged_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __re
   for (unsigned p = threadIdx.x; p < static_cast<unsigned>(np); p += blockDim.x) {
     const int row = p / n0, k = row / n1;
     const int i = p - row * n0, j = row - k * n1;
+    // corrections of the point's faces, in flight during the sums: a face's
+    // first mortar here, further ones where they are added
+    bool on[3] = {false, false, false};
+    int mortars[3];
+    const double* from[3];
+    double first[3][5];
+    if (table != nullptr) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int at = d == 0 ? i : d == 1 ? j : k, nd = d == 0 ? n0 : d == 1 ? n1 : n2;
+        on[d] = at == 0 || at == nd - 1;
+        if (!on[d]) continue;
+        const int nf = d == 0 ? n1 * n2 : d == 1 ? n0 * n2 : n0 * n1;
+        const int f = d == 0 ? j + n1 * k : d == 1 ? i + n0 * k : i + n0 * j;
+        const MortarCorrection lower = table[6 * e + 2 * d], upper = table[6 * e + 2 * d + 1];
+        mortars[d] = at == 0 ? lower.count : upper.count;
+        from[d] = corr + 5 * (at == 0 ? lower.off : upper.off) + f;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) first[d][c] = from[d][c * nf];
+      }
+    }
     double der[5][3];
     auto sums = [&](int d, int n, const double* w, const double* x, int step) {
 #pragma unroll
@@ -148,16 +168,18 @@ sw_ragged_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __re
     }
     sw_time_derivative(out, up, dup, g2[p]);
     if (table != nullptr) {
-      for (int d = 0; d < 3; ++d) {
-        const int at = d == 0 ? i : d == 1 ? j : k, nd = d == 0 ? n0 : d == 1 ? n1 : n2;
-        if (at != 0 && at != nd - 1) continue;
-        const int nf = d == 0 ? n1 * n2 : d == 1 ? n0 * n2 : n0 * n1;
-        const int f = d == 0 ? j + n1 * k : d == 1 ? i + n0 * k : i + n0 * j;
-        const MortarCorrection t = table[6 * e + 2 * d + (at == 0 ? 0 : 1)];
-        const double* from = corr + 5 * t.off + f;
-        for (int q = 0; q < t.count; ++q, from += 5 * nf)
 #pragma unroll
-          for (int c = 0; c < 5; ++c) out[c] = out[c] + from[c * nf];
+      for (int d = 0; d < 3; ++d) {
+        if (!on[d]) continue;
+        const double* src = from[d];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) out[c] = out[c] + first[d][c];
+        const int nf = d == 0 ? n1 * n2 : d == 1 ? n0 * n2 : n0 * n1;
+        for (int q = 1; q < mortars[d]; ++q) {
+          src += 5 * nf;
+#pragma unroll
+          for (int c = 0; c < 5; ++c) out[c] = out[c] + src[c * nf];
+        }
       }
     }
 #pragma unroll
@@ -1261,16 +1283,22 @@ int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32
                             const double* corr, hipStream_t stream) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
+  // one launch for all sizes: a workgroup per element is too few for the
+  // occupancy that smaller LDS allows to outweigh a launch's last round
+  // (1000 elements of extents 4 .. 12: 60 us in four classes, 25 us in one)
+  RaggedClass all{classes.front().begin, 0, 0, 0};
   for (const RaggedClass& c : classes) {
-    const int lds = (5 * c.np_max + kStagedDiffDoubles) * 8;
-    if (!allow_lds(reinterpret_cast<const void*>(&sw_ragged_volume_kernel), lds))
-      return SXD_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(sw_ragged_volume_kernel, dim3(c.count),
-                       dim3(c.np_max > 256 ? 512 : c.np_max > 128 ? 256 : 128), lds, stream, el,
-                       list + c.begin, u, gamma2, inv_jac, dt, dtab, table, corr);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    all.count += c.count;
+    all.np_max = std::max(all.np_max, c.np_max);
+    all.d_doubles = std::max(all.d_doubles, c.d_doubles);
   }
-  return SXD_OK;
+  const int lds = (5 * all.np_max + all.d_doubles) * 8;
+  if (!allow_lds(reinterpret_cast<const void*>(&sw_ragged_volume_kernel), lds))
+    return SXD_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(sw_ragged_volume_kernel, dim3(all.count),
+                     dim3(all.np_max > 256 ? 512 : all.np_max > 128 ? 256 : 128), lds, stream, el,
+                     list + all.begin, u, gamma2, inv_jac, dt, dtab, table, corr);
+  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 
 int launch_mixed_gh_volume_du(int count, const int32_t* list, const MixedElement* el, int np_max,

@@ -936,32 +936,78 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
     else if (recs[i].partner > i)
       pairs.push_back(i);
   }
-  // one workgroup per mortar (mortar_faces.hip), in classes of decreasing LDS
-  // size: 1, 2, 4 or 8 and more workgroups per CU.  Every mortar fits: faces
+  // one workgroup per mortar (mortar_faces.hip), in order of decreasing LDS
+  // size.  Every mortar fits: faces
   // have at most 193 points and mortars at most 20 x 20, so a side's staged
   // values are at most 13 x 20 x 20 doubles, the face packages 13 x 386, and all
   // of it with the matrices 145 KB.
   std::vector<MortarCorrection> corrections;
+  std::vector<MortarJob> jobs;
   if (keys.empty()) {
     auto lds = [&](bool gh, int32_t i) {
       return mortar_corrections_lds_bytes(gh, recs[i], recs[recs[i].partner]);
     };
     std::stable_sort(pairs.begin(), pairs.end(),
                      [&](int32_t x, int32_t y) { return lds(true, x) > lds(true, y); });
-    auto per_cu = [&](int32_t i) {
-      const int fit = 160 * 1024 / lds(true, i);
-      return fit >= 8 ? 8 : fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
-    };
-    for (int i = 0; i < static_cast<int>(pairs.size());) {
-      MortarClass c{i, 0, {0, 0}};
-      while (i < static_cast<int>(pairs.size()) && per_cu(pairs[i]) == per_cu(pairs[c.begin])) {
-        c.lds_bytes[0] = std::max(c.lds_bytes[0], lds(false, pairs[i]));
-        c.lds_bytes[1] = std::max(c.lds_bytes[1], lds(true, pairs[i]));
-        ++c.count;
-        ++i;
+    // GH: classes of 1, 2, 4 and 8 workgroups per CU (one class for all took 869
+    // instead of 794 us on 1000 elements of extents 4 .. 12, a class per number of
+    // workgroups 815).  ScalarWave has a tenth of the workgroups, too few for
+    // occupancy to outweigh a launch's last round: one class (12 RHS 1399 us,
+    // against 1523 with two).
+    for (int sys = 0; sys < 2; ++sys) {
+      auto tier = [&](int32_t i) {
+        const int fit = 160 * 1024 / lds(true, i);
+        return sys == 0 ? 0 : fit >= 8 ? 8 : fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
+      };
+      for (int i = 0; i < static_cast<int>(pairs.size());) {
+        MortarClass c{i, 0, 0};
+        for (; i < static_cast<int>(pairs.size()) && tier(pairs[i]) == tier(pairs[c.begin]);
+             ++i, ++c.count)
+          c.lds_bytes = std::max(c.lds_bytes, lds(sys == 1, pairs[i]));
+        plan->classes[sys].push_back(c);
       }
-      plan->classes.push_back(c);
     }
+    std::vector<int64_t> offsets(num_owned);
+    std::vector<const int32_t*> own_ext(num_owned);
+    for (int e = 0, at = 0; e < num_elements; ++e) {
+      if (local[e] < 0) continue;
+      own_ext[at] = extents + 3 * e;
+      if (at + 1 < num_owned)
+        offsets[at + 1] = offsets[at] + static_cast<int64_t>(extents[3 * e]) *
+                                            extents[3 * e + 1] * extents[3 * e + 2];
+      ++at;
+    }
+    auto side_of = [&](const MortarRecord& r) {
+      const MortarFace& f = faces[r.face];
+      const int32_t* n = own_ext[f.e];
+      const int d = f.dir / 2, upper = f.dir % 2;
+      MortarSide s{};
+      s.off = offsets[f.e];
+      s.pt_off = f.pt_off;
+      s.rec_off = r.rec_off;
+      s.corr_off = r.corr_off;
+      s.np = n[0] * n[1] * n[2];
+      s.nf = f.nf;
+      s.na = r.na;
+      s.nb = r.nb;
+      s.ka = r.ka;
+      s.kb = r.kb;
+      s.base = upper * (n[d] - 1) * (d == 0 ? 1 : d == 1 ? n[0] : n[0] * n[1]);
+      s.step_a = d == 0 ? n[0] : 1;
+      s.step_b = d == 2 ? n[0] : n[0] * n[1];
+      auto matrix = [&](int nf, int nm, int size) {
+        const int at = mortar_table_offset(nf, nm);
+        return size == kChildFull ? at
+               : -1 - (size == kChildUpperHalf ? at : kPackedMortarSize + at);
+      };
+      s.mat_a = matrix(r.na, r.ka, r.size_a);
+      s.mat_b = matrix(r.nb, r.kb, r.size_b);
+      s.dim = d;
+      s.side = upper;
+      s.extent = n[d];
+      return s;
+    };
+    for (const int32_t i : pairs) jobs.push_back({{side_of(recs[i]), side_of(recs[recs[i].partner])}});
     corrections.resize(6 * static_cast<size_t>(num_owned));
     for (const MortarFace& f : faces)
       corrections[6 * static_cast<size_t>(f.e) + f.dir] = {recs[f.rec_begin].corr_off,
@@ -1015,6 +1061,7 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
   upload(&plan->d_direct, direct);
   upload(&plan->d_pairs, pairs);
   upload(&plan->d_remote_records, remote_records);
+  upload(&plan->d_jobs, jobs);
   upload(&plan->d_corrections, corrections);
   upload(&plan->d_messages, messages);
   upload(&plan->d_keys, keys);
@@ -1034,6 +1081,7 @@ void destroy_mortar_plan(MortarPlan* plan) {
   if (plan->d_direct != nullptr) (void)hipFree(plan->d_direct);
   if (plan->d_pairs != nullptr) (void)hipFree(plan->d_pairs);
   if (plan->d_remote_records != nullptr) (void)hipFree(plan->d_remote_records);
+  if (plan->d_jobs != nullptr) (void)hipFree(plan->d_jobs);
   if (plan->d_corrections != nullptr) (void)hipFree(plan->d_corrections);
   if (plan->d_messages != nullptr) (void)hipFree(plan->d_messages);
   if (plan->d_keys != nullptr) (void)hipFree(plan->d_keys);

@@ -17,8 +17,10 @@
 //   3. per mortar point and group of outputs: dimension-b interpolation of the
 //      3 or 4 values the group needs, boundary terms of both sides;
 //   4. dimension-a projection back; 5. dimension-b projection, lift, write.
-// A mortar's LDS is laid out by its own extents; the mortars are launched in
+// A mortar's LDS is laid out by its own extents; GH mortars are launched in
 // classes of similar LDS size, since a launch reserves its largest for all.
+// What bounds it is latency: the phases of a workgroup are short and 12 to 18
+// waves per CU hide them only in part (vector units busy 40 %, LDS 30 %).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,11 +36,13 @@ namespace {
 
 constexpr int kPk = 13;  // packaged values of a point and pair
 
-__host__ __device__ inline bool projects_a(const MortarRecord& r) {
-  return r.size_a != kChildFull || r.na != r.ka;
+// A dimension is the identity where the mortar covers all of it (matrix in the
+// Full table) with the face's extent.
+__host__ __device__ inline bool projects_a(const MortarSide& r) {
+  return r.mat_a < 0 || r.na != r.ka;
 }
-__host__ __device__ inline bool projects_b(const MortarRecord& r) {
-  return r.size_b != kChildFull || r.nb != r.kb;
+__host__ __device__ inline bool projects_b(const MortarSide& r) {
+  return r.mat_b < 0 || r.nb != r.kb;
 }
 
 // LDS of one side (doubles): the face package where dimension a is projected,
@@ -47,21 +51,30 @@ __host__ __device__ inline bool projects_b(const MortarRecord& r) {
 // face, per projected dimension).
 struct SideLds {
   int face, staged, mat_a, mat_b, mag;
-  __host__ __device__ SideLds(const MortarRecord& r, bool gh) {
-    const int fwd = kPk * r.ka * r.nb, back = 5 * r.na * r.kb;
-    face = projects_a(r) ? kPk * r.na * r.nb : 0;
+  __host__ __device__ SideLds(bool proj_a, bool proj_b, int na, int nb, int ka, int kb, bool gh) {
+    const int fwd = kPk * ka * nb, back = 5 * na * kb;
+    face = proj_a ? kPk * na * nb : 0;
     staged = fwd > back ? fwd : back;
-    mat_a = projects_a(r) ? 2 * r.na * r.ka : 0;
-    mat_b = projects_b(r) ? 2 * r.nb * r.kb : 0;
-    mag = gh ? 0 : r.na * r.nb;
+    mat_a = proj_a ? 2 * na * ka : 0;
+    mat_b = proj_b ? 2 * nb * kb : 0;
+    mag = gh ? 0 : na * nb;
   }
+  __host__ __device__ SideLds(const MortarSide& r, bool gh)
+      : SideLds(projects_a(r), projects_b(r), r.na, r.nb, r.ka, r.kb, gh) {}
 };
 
 // The corrections of both sides lie over the face packages.
-__host__ __device__ inline int corrections_doubles(const MortarRecord& r, const SideLds& a,
-                                                   const SideLds& b) {
-  const int faces = a.face + b.face, bc = 10 * r.ka * r.kb;
+__host__ __device__ inline int corrections_doubles(int km, const SideLds& a, const SideLds& b) {
+  const int faces = a.face + b.face, bc = 10 * km;
   return faces > bc ? faces : bc;
+}
+
+// x / n for x < 8000 and n <= 20 with one multiplication.
+__device__ __forceinline__ unsigned divisor(int n) {
+  return ((1u << 20) + static_cast<unsigned>(n) - 1) / static_cast<unsigned>(n);
+}
+__device__ __forceinline__ int divide(int x, unsigned m) {
+  return static_cast<int>((static_cast<unsigned>(x) * m) >> 20);
 }
 
 __device__ __forceinline__ int volume_index(const MixedElement& m, int d, int side, int a,
@@ -133,7 +146,7 @@ gh_mortar_sides_kernel(const MixedElement* __restrict__ el, const MortarFace* __
     const int km = r.ka * r.kb;
     const double* src = s_lam;
     __syncthreads();
-    if (projects_a(r)) {
+    if (r.size_a != kChildFull || r.na != r.ka) {
       const double* Ma = matrix_block(full, half, r.na, r.ka, r.size_a);
       for (int x = threadIdx.x; x < 4 * r.ka * r.nb; x += blockDim.x) {
         const int c = x / (r.ka * r.nb), y = x % (r.ka * r.nb), lb = y / r.ka, ra = y % r.ka;
@@ -150,7 +163,7 @@ gh_mortar_sides_kernel(const MixedElement* __restrict__ el, const MortarFace* __
       const int c = x / km, k = x % km, rb = k / r.ka, ra = k % r.ka;
       const double* v = src + c * r.ka * r.nb + ra;
       double s;
-      if (projects_b(r)) {
+      if (r.size_b != kChildFull || r.nb != r.kb) {
         s = Mb[rb * r.nb] * v[0];
         for (int l = 1; l < r.nb; ++l) s = fma(Mb[rb * r.nb + l], v[r.ka * l], s);
       } else {
@@ -175,6 +188,7 @@ __device__ __forceinline__ void mortar_values(double v[4], const double* staged,
   }
   double w = row[0];
   v[0] = w * at[O0], v[1] = w * at[O1], v[2] = w * at[O2], v[3] = w * at[O3];
+#pragma unroll 2
   for (int l = 1; l < nb; ++l) {
     at += kPk * ka;
     w = row[l];
@@ -195,20 +209,18 @@ __device__ __forceinline__ void boundary_terms(double bc[5], const double in[13]
     sw_boundary_terms(bc, in, ex);
 }
 
-// Grid: GH 10 workgroups per mortar of `list` (its pairs next to each other on
-// one XCD), padded to a multiple of 8 mortars; ScalarWave one per mortar.
-// `list` holds one record of each mortar.  corr: [NC][nf] per record at NC
-// corr_off, the lifted corrections of the record's own face.
+// Grid: GH 10 workgroups per job, one per symmetric pair (next to each other on
+// one XCD, padded to a multiple of 8 jobs); ScalarWave one workgroup per job.
+// corr: [NC][nf] per side at NC corr_off, the lifted corrections of the side's
+// own face.
 template <bool GH>
 __global__ void __launch_bounds__(256)
-mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
-                          const MortarFace* __restrict__ faces,
-                          const MortarRecord* __restrict__ recs,
-                          const int32_t* __restrict__ list, const int32_t* __restrict__ gather,
-                          const double* __restrict__ u, const double* __restrict__ params,
-                          const double* __restrict__ inv_jac, const double* __restrict__ sides,
-                          const double* __restrict__ speeds, double* __restrict__ corr,
-                          const double* __restrict__ full, const double* __restrict__ half) {
+mortar_corrections_kernel(int count, const MortarJob* __restrict__ jobs,
+                          const int32_t* __restrict__ gather, const double* __restrict__ u,
+                          const double* __restrict__ params, const double* __restrict__ inv_jac,
+                          const double* __restrict__ sides, const double* __restrict__ speeds,
+                          double* __restrict__ corr, const double* __restrict__ full,
+                          const double* __restrict__ half) {
   constexpr int NC = GH ? 50 : 5;
   extern __shared__ double s_lds[];
   int at = blockIdx.x, pr = 0;
@@ -218,18 +230,15 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
     pr = slot % 10;
     if (at >= count) return;
   }
-  const int comp[5] = {pr, GH ? 10 + pr : 1, GH ? 20 + 3 * pr : 2, GH ? 21 + 3 * pr : 3,
-                       GH ? 22 + 3 * pr : 4};
-  const MortarRecord r0 = recs[list[at]];
-  const MortarRecord r1 = recs[r0.partner];
-  const MortarFace f0 = faces[r0.face], f1 = faces[r1.face];
+  const MortarSide& r0 = jobs[at].side[0];
+  const MortarSide& r1 = jobs[at].side[1];
   const SideLds l0(r0, GH), l1(r1, GH);
-  const int nf0 = f0.nf, nf1 = f1.nf, km = r0.ka * r0.kb;
+  const int nf0 = r0.nf, nf1 = r1.nf, km = r0.ka * r0.kb;
   double* s_face0 = s_lds;
   double* s_face1 = s_face0 + l0.face;
   double* s_bc0 = s_lds;
   double* s_bc1 = s_bc0 + 5 * km;
-  double* s_st0 = s_lds + corrections_doubles(r0, l0, l1);
+  double* s_st0 = s_lds + corrections_doubles(km, l0, l1);
   double* s_st1 = s_st0 + l0.staged;
   double* s_ma0 = s_st1 + l1.staged;
   double* s_mb0 = s_ma0 + l0.mat_a;
@@ -238,29 +247,32 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
   double* s_mag0 = s_mb1 + l1.mat_b;
   double* s_mag1 = s_mag0 + l0.mag;
   const int t = threadIdx.x, T = blockDim.x;
+  const unsigned by_na0 = divisor(r0.na), by_na1 = divisor(r1.na);
+  const unsigned by_ka0 = divisor(r0.ka), by_ka1 = divisor(r1.ka);
   {
-    const double* a0 = matrix_block(full, half, r0.na, r0.ka, r0.size_a);
-    const double* b0 = matrix_block(full, half, r0.nb, r0.kb, r0.size_b);
-    const double* a1 = matrix_block(full, half, r1.na, r1.ka, r1.size_a);
-    const double* b1 = matrix_block(full, half, r1.nb, r1.kb, r1.size_b);
+    auto block = [&](int mat) { return mat >= 0 ? full + mat : half + (-1 - mat); };
+    const double* a0 = block(r0.mat_a);
+    const double* b0 = block(r0.mat_b);
+    const double* a1 = block(r1.mat_a);
+    const double* b1 = block(r1.mat_b);
     for (int x = t; x < l0.mat_a; x += T) s_ma0[x] = a0[x];
     for (int x = t; x < l0.mat_b; x += T) s_mb0[x] = b0[x];
     for (int x = t; x < l1.mat_a; x += T) s_ma1[x] = a1[x];
     for (int x = t; x < l1.mat_b; x += T) s_mb1[x] = b1[x];
   }
+  const int comp[5] = {pr, GH ? 10 + pr : 1, GH ? 20 + 3 * pr : 2, GH ? 21 + 3 * pr : 3,
+                       GH ? 22 + 3 * pr : 4};
   // 1. packages
   for (int x = t; x < nf0 + nf1; x += T) {
     const bool second = x >= nf0;
-    const MortarFace& fr = second ? f1 : f0;
+    const MortarSide& r = second ? r1 : r0;
     const int f = second ? x - nf0 : x;
-    const int nf = second ? nf1 : nf0, na = second ? r1.na : r0.na;
-    const MixedElement m = el[fr.e];
-    const int d = fr.dir >> 1, side = fr.dir & 1;
-    const int np = m.np;
-    const int p = volume_index(m, d, side, f % na, f / na);
+    const int nf = second ? nf1 : nf0, np = r.np;
+    const int b = divide(f, second ? by_na1 : by_na0), a = f - b * r.na;
+    const int p = r.base + a * r.step_a + b * r.step_b;
     double pk[kPk];
     if constexpr (GH) {
-      const double* sd = sides + 12 * fr.pt_off + f;
+      const double* sd = sides + 12 * r.pt_off + f;
       GhFaceSide s;
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
@@ -270,7 +282,7 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
 #pragma unroll
       for (int c = 0; c < 4; ++c) s.lam[c] = sd[(6 + c) * nf];
       s.gamma2 = sd[10 * nf];
-      const double* ue = u + 50 * m.off + p;
+      const double* ue = u + 50 * r.off + p;
       double phi[3];
 #pragma unroll
       for (int i = 0; i < 3; ++i) phi[i] = ue[comp[2 + i] * np];
@@ -279,13 +291,13 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
       double n[3], up[5], mag;
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        n[i] = inv_jac[9 * m.off + ij3(d, i) * np + p];
-        if (side == 0) n[i] = n[i] * -1.0;
+        n[i] = inv_jac[9 * r.off + ij3(r.dim, i) * np + p];
+        if (r.side == 0) n[i] = n[i] * -1.0;
       }
 #pragma unroll
-      for (int c = 0; c < 5; ++c) up[c] = u[5 * m.off + c * np + p];
+      for (int c = 0; c < 5; ++c) up[c] = u[5 * r.off + c * np + p];
       flat_normalize(n, &mag);
-      sw_package(pk, up, params[m.off + p], n);
+      sw_package(pk, up, params[r.off + p], n);
       (second ? s_mag1 : s_mag0)[f] = mag;
     }
     double* out = (second ? (l1.face > 0 ? s_face1 : s_st1) : (l0.face > 0 ? s_face0 : s_st0)) +
@@ -299,15 +311,16 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
   if (l0.face + l1.face > 0) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const MortarRecord& r = s == 0 ? r0 : r1;
+      const MortarSide& r = s == 0 ? r0 : r1;
       if ((s == 0 ? l0.face : l1.face) == 0) continue;
       const double* in = s == 0 ? s_face0 : s_face1;
       const double* M = s == 0 ? s_ma0 : s_ma1;
       double* out = s == 0 ? s_st0 : s_st1;
       const int half_ka = (r.ka + 1) / 2, items = half_ka * r.nb;
+      const unsigned by_half = divisor(half_ka);
       for (int x = t; x < 3 * items; x += T) {
-        const int g = x / items, y = x - g * items;
-        const int lb = y / half_ka, ra = 2 * (y - lb * half_ka);
+        const int g = (x >= items) + (x >= 2 * items), y = x - g * items;
+        const int lb = divide(y, by_half), ra = 2 * (y - lb * half_ka);
         const bool two = ra + 1 < r.ka;
         const double* v = in + kPk * r.na * lb + 4 * g;
         const double* w0 = M + ra * r.na;
@@ -318,7 +331,8 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
           s0[c] = w0[0] * v[c];
           s1[c] = w1[0] * v[c];
         }
-        for (int l = 1; l < r.na; ++l) {
+  #pragma unroll 2
+      for (int l = 1; l < r.na; ++l) {
           v += kPk;
           const double a = w0[l], b = w1[l];
 #pragma unroll
@@ -341,10 +355,10 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
   // 3. boundary terms: groups 0..2 the Phi_g output (values 1 + g, 6 + g,
   // 9 + g), group 3 the g and Pi outputs (values 0, 4, 5, 12)
   for (int x = t; x < 4 * km; x += T) {
-    const int g = x / km, k = x - g * km;
+    const int g = (x >= km) + (x >= 2 * km) + (x >= 3 * km), k = x - g * km;
     const int q = gather[r0.rec_off + k];
-    const int rb0 = k / r0.ka, ra0 = k - rb0 * r0.ka;
-    const int rb1 = q / r1.ka, ra1 = q - rb1 * r1.ka;
+    const int rb0 = divide(k, by_ka0), ra0 = k - rb0 * r0.ka;
+    const int rb1 = divide(q, by_ka1), ra1 = q - rb1 * r1.ka;
     const double* row0 = l0.mat_b > 0 ? s_mb0 + rb0 * r0.nb : nullptr;
     const double* row1 = l1.mat_b > 0 ? s_mb1 + rb1 * r1.nb : nullptr;
     double lam0[4] = {0, 0, 0, 0}, lam1[4] = {0, 0, 0, 0};
@@ -387,12 +401,13 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
       const bool second = x >= items0;
       const int y = second ? x - items0 : x;
       const int na = second ? r1.na : r0.na, ka = second ? r1.ka : r0.ka;
-      const int lb = y / na, ra = y - lb * na;
+      const int lb = divide(y, second ? by_na1 : by_na0), ra = y - lb * na;
       const double* v = (second ? s_bc1 : s_bc0) + 5 * ka * lb;
       const double* w = (second ? s_ma1 : s_ma0) + na * ka + ra * ka;
       double s[5];
 #pragma unroll
       for (int c = 0; c < 5; ++c) s[c] = w[0] * v[c];
+#pragma unroll 2
       for (int l = 1; l < ka; ++l) {
         v += 5;
         const double a = w[l];
@@ -408,17 +423,19 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
   // 5. dimension b back to the face, and lift
   for (int x = t; x < nf0 + nf1; x += T) {
     const bool second = x >= nf0;
+    const MortarSide& r = second ? r1 : r0;
     const int f = second ? x - nf0 : x;
-    const int nf = second ? nf1 : nf0, na = second ? r1.na : r0.na;
-    const int nb = second ? r1.nb : r0.nb, kb = second ? r1.kb : r0.kb;
-    const int fb = f / na, fa = f - fb * na;
-    const double* v = (second ? (l1.mat_a > 0 ? s_st1 : s_bc1) : (l0.mat_a > 0 ? s_st0 : s_bc0)) +
-                      5 * fa;
+    const int nf = second ? nf1 : nf0, na = r.na;
+    const int fb = divide(f, second ? by_na1 : by_na0), fa = f - fb * na;
+    const double* v =
+        (second ? (l1.mat_a > 0 ? s_st1 : s_bc1) : (l0.mat_a > 0 ? s_st0 : s_bc0)) + 5 * fa;
     double s[5];
     if ((second ? l1.mat_b : l0.mat_b) > 0) {
+      const int nb = r.nb, kb = r.kb;
       const double* w = (second ? s_mb1 : s_mb0) + nb * kb + fb * kb;
 #pragma unroll
       for (int c = 0; c < 5; ++c) s[c] = w[0] * v[c];
+#pragma unroll 2
       for (int l = 1; l < kb; ++l) {
         v += 5 * na;
         const double a = w[l];
@@ -429,17 +446,13 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
 #pragma unroll
       for (int c = 0; c < 5; ++c) s[c] = v[5 * na * fb + c];
     }
-    const MortarFace& fr = second ? f1 : f0;
-    const MixedElement& m = el[fr.e];
-    const int d = fr.dir >> 1;
-    const int nd = d == 0 ? m.n[0] : (d == 1 ? m.n[1] : m.n[2]);
     double mag;
     if constexpr (GH)
-      mag = sides[12 * fr.pt_off + 11 * nf + f];
+      mag = sides[12 * r.pt_off + 11 * nf + f];
     else
       mag = (second ? s_mag1 : s_mag0)[f];
-    const double fac = lift_factor(nd, mag);
-    double* out = corr + NC * (second ? r1.corr_off : r0.corr_off) + f;
+    const double fac = lift_factor(r.extent, mag);
+    double* out = corr + NC * r.corr_off + f;
 #pragma unroll
     for (int c = 0; c < 5; ++c) out[comp[c] * nf] = s[c] * fac;
   }
@@ -448,9 +461,13 @@ mortar_corrections_kernel(int count, const MixedElement* __restrict__ el,
 }  // namespace
 
 int mortar_corrections_lds_bytes(bool gh, const MortarRecord& r, const MortarRecord& partner) {
-  const SideLds a(r, gh), b(partner, gh);
-  return 8 * (corrections_doubles(r, a, b) + a.staged + b.staged + a.mat_a + a.mat_b + b.mat_a +
-              b.mat_b + a.mag + b.mag);
+  auto side = [gh](const MortarRecord& m) {
+    return SideLds(m.size_a != kChildFull || m.na != m.ka, m.size_b != kChildFull || m.nb != m.kb,
+                   m.na, m.nb, m.ka, m.kb, gh);
+  };
+  const SideLds a = side(r), b = side(partner);
+  return 8 * (corrections_doubles(r.ka * r.kb, a, b) + a.staged + b.staged + a.mat_a + a.mat_b +
+              b.mat_a + b.mat_b + a.mag + b.mag);
 }
 
 MortarCorrectionsWork::MortarCorrectionsWork(bool gh, const MortarPlan& plan, double* work) {
@@ -476,21 +493,24 @@ int launch_mortar_lifted_corrections(bool gh, const MortarPlan& plan, const Mixe
                        half, plan.kf);
     if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   }
-  for (const MortarClass& c : plan.classes) {
+  for (const MortarClass& c : plan.classes[gh ? 1 : 0]) {
     const void* kernel = gh ? reinterpret_cast<const void*>(&mortar_corrections_kernel<true>)
                             : reinterpret_cast<const void*>(&mortar_corrections_kernel<false>);
-    const int lds = c.lds_bytes[gh ? 1 : 0];
+    const int lds = c.lds_bytes;
     if (!allow_lds(kernel, lds)) return SXD_ERR_DEVICE;
-    const int32_t* list = plan.d_pairs + c.begin;
-    const int blocks = gh ? (c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10 : c.count;
+    const MortarJob* jobs = plan.d_jobs + c.begin;
+    // threads, measured on 1000 elements of extents 4 .. 12 with 64 / 128 / 192 /
+    // 256: whole GH RHS 1055 / 912 / 864 / 864 us (768 refined and rotated elements
+    // 448 / 403 / 401 / 412), 12 ScalarWave RHS 2155 / 1837 / 1728 / 1673 us
     if (gh)
-      hipLaunchKernelGGL(mortar_corrections_kernel<true>, dim3(blocks), dim3(128), lds, stream,
-                         c.count, el, plan.d_faces, plan.d_records, list, plan.d_gather, u,
-                         params, inv_jac, w.sides, w.speeds, w.corr, full, half);
+      hipLaunchKernelGGL(mortar_corrections_kernel<true>,
+                         dim3((c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10),
+                         dim3(192), lds, stream, c.count, jobs, plan.d_gather, u, params, inv_jac,
+                         w.sides, w.speeds, w.corr, full, half);
     else
-      hipLaunchKernelGGL(mortar_corrections_kernel<false>, dim3(blocks), dim3(128), lds, stream,
-                         c.count, el, plan.d_faces, plan.d_records, list, plan.d_gather, u,
-                         params, inv_jac, nullptr, nullptr, w.corr, full, half);
+      hipLaunchKernelGGL(mortar_corrections_kernel<false>, dim3(c.count), dim3(256), lds,
+                         stream, c.count, jobs, plan.d_gather, u, params, inv_jac, nullptr,
+                         nullptr, w.corr, full, half);
     if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   }
   return SXD_OK;
