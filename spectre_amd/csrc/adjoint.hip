@@ -218,90 +218,12 @@ rk3_adjoint_substep_kernel(int substep, int64_t n, double dt, const double* lam,
 
 // ---------------------------------------------------------------------------
 // Generalized harmonic: adjoint of the RHS linearised at the state u (the RHS
-// is nonlinear), after the partial derivatives of u:
-//  1. point-wise: ubar = (df/du)^T gbar; the adjoint of the inertial
-//     derivatives contracted with the inverse Jacobian into logical-derivative
-//     adjoints xbar[3 c + j], written over du (read first, same point);
-//  2. faces: every face point's transposed lifted UpwindPenalty terms of each
-//     face it lies on, as interior point of its own face and as exterior
-//     point of the neighbour's face, into a per-face work array;
-//  3. transposed differentiation sweeps ubar_c += sum_j D_j^T xbar_cj, then
-//     the face terms.
-__global__ void __launch_bounds__(128)
-gh_adjoint_pointwise_kernel(int64_t total, int np, const double* __restrict__ u,
-                            double* du_xbar, const double* __restrict__ gammas,
-                            const double* __restrict__ inv_jac, const double* __restrict__ gbar,
-                            double* __restrict__ ubar) {
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= total) return;
-  const int64_t e = gid / np;
-  const int p = static_cast<int>(gid % np);
-  double ub[50];
-  const double* up = u + e * 50 * np + p;
-  const double* dup = du_xbar + e * 150 * np + p;
-  const double* gp = gbar + e * 50 * np + p;
-  const double* ga = gammas + e * 3 * np + p;
-  const double gamma1 = ga[np], gamma2 = ga[2 * np];
-  GhVjpPoint pt;
-  gh_time_derivative_vjp(up, np, dup, np, ga[0], gamma1, gamma2, gp, np, ub, &pt);
-  for (int c = 0; c < 50; ++c) ubar[(e * 50 + c) * np + p] = ub[c];
-  // every read of du is done: the logical-derivative adjoints go in its place
-  double ij[9];
-  for (int c = 0; c < 9; ++c) ij[c] = inv_jac[(e * 9 + c) * np + p];
-  for (int c = 0; c < 50; ++c) {
-    double dub[3];
-    for (int i = 0; i < 3; ++i) dub[i] = gh_time_derivative_dubar(pt, gamma1, gamma2, gp, np, 3 * c + i);
-    for (int j = 0; j < 3; ++j) {
-      double s = 0.0;
-      for (int i = 0; i < 3; ++i) s += ij[ij3(j, i)] * dub[i];
-      du_xbar[(e * 150 + 3 * c + j) * np + p] = s;
-    }
-  }
-}
-
-// ubar_c += sum_j D_j^T xbar_cj, then the face terms of the points on the
-// element's faces (contrib: [E][6][50][F], F = largest face, directions in
-// order).  Grid: (E, 50 / kSweepChunk); dynamic LDS: 3 Np doubles, then
-// the three D matrices.
-constexpr int kSweepChunk = 5;
-__global__ void __launch_bounds__(256)
-transposed_sweeps_kernel(int n0, int n1, int n2, int nc, const double* __restrict__ xbar,
-                         double* __restrict__ ubar, const double* __restrict__ dtab,
-                         const double* __restrict__ contrib, int F) {
-  extern __shared__ double s_x[];
-  const int np = n0 * n1 * n2;
-  const int64_t e = blockIdx.x;
-  const int n[3] = {n0, n1, n2};
-  const int stride[3] = {1, n0, n0 * n1};
-  const double* D[3];
-  stage_diff_matrices(dtab, n, s_x + 3 * np, D);  // synchronised by the loop's first barrier
-  const int c_end = min(nc, static_cast<int>(blockIdx.y + 1) * kSweepChunk);
-  for (int c = blockIdx.y * kSweepChunk; c < c_end; ++c) {
-    __syncthreads();
-    for (int x = threadIdx.x; x < 3 * np; x += blockDim.x)
-      s_x[x] = xbar[(e * 3 * nc + 3 * c) * np + x];
-    __syncthreads();
-    for (int p = threadIdx.x; p < np; p += blockDim.x) {
-      const int idx[3] = {p % n0, (p / n0) % n1, p / (n0 * n1)};
-      double acc = ubar[(e * nc + c) * np + p];
-      for (int j = 0; j < 3; ++j) {
-        const int base = p - idx[j] * stride[j];
-        for (int m = 0; m < n[j]; ++m)
-          acc = fma(D[j][m * n[j] + idx[j]], s_x[j * np + base + m * stride[j]], acc);
-      }
-      for (int d = 0; d < 3; ++d) {
-        if (n[d] == 1) continue;
-        const int side = idx[d] == 0 ? 0 : idx[d] == n[d] - 1 ? 1 : -1;
-        if (side < 0) continue;
-        const int a = d == 0 ? idx[1] : idx[0], b = d == 2 ? idx[1] : idx[2];
-        const int f = a + (d == 0 ? n1 : n0) * b;
-        acc += contrib[((e * 6 + 2 * d + side) * nc + c) * F + f];
-      }
-      ubar[(e * nc + c) * np + p] = acc;
-    }
-  }
-}
-
+// is nonlinear): the point-wise adjoint (gh_adjoint_volume.hip); the face points'
+// transposed lifted UpwindPenalty terms of each face they lie on, as interior
+// point of their own face and as exterior point of the neighbour's, into a
+// per-face work array; then the transposed differentiation sweeps
+// (gh_adjoint_volume.hip), which add the face terms.
+//
 // Faces, one thread per (element, face, face point): the point's face terms
 // (its own correction's and the neighbour's, gh_face_pair_vjp) go to its
 // slot of contrib [E][6][50][F] (F = largest face), which the transposed
@@ -386,32 +308,18 @@ int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t*
                           const double* u, const double* gammas, const double* inv_jac,
                           const double* gbar, double* ubar, double* scratch_du,
                           double* scratch_faces, hipStream_t stream) {
-  const double* dtab = device_diff_matrices();
-  if (dtab == nullptr) return SXD_ERR_DEVICE;
-  const int np = ext[0] * ext[1] * ext[2];
-  const int d_doubles = ext[0] * ext[0] + ext[1] * ext[1] + ext[2] * ext[2];
-  const int sweep_lds = (3 * np + d_doubles) * static_cast<int>(sizeof(double));
-  if (sweep_lds > 160 * 1024) return SXD_ERR_UNSUPPORTED;
-  if (!allow_lds(reinterpret_cast<const void*>(&transposed_sweeps_kernel), sweep_lds))
-    return SXD_ERR_DEVICE;
-  const int64_t total = static_cast<int64_t>(num_elements) * np;
-  int rc = launch_partial_derivatives(num_elements, ext, 50, u, inv_jac, scratch_du, nullptr,
-                                      stream);
+  if (!gh_adjoint_supported(ext)) return SXD_ERR_UNSUPPORTED;
+  const int rc = launch_gh_adjoint_points(num_elements, ext, u, gammas, inv_jac, gbar, ubar,
+                                          scratch_du, stream);
   if (rc != SXD_OK) return rc;
-  hipLaunchKernelGGL(gh_adjoint_pointwise_kernel, dim3(static_cast<unsigned>((total + 127) / 128)),
-                     dim3(128), 0, stream, total, np, u, scratch_du, gammas, inv_jac, gbar, ubar);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   const int F = gh_adjoint_face_slots(ext);
   const int64_t faces = static_cast<int64_t>(num_elements) * 6 * F;
   hipLaunchKernelGGL(gh_adjoint_face_kernel, dim3(static_cast<unsigned>((faces + 63) / 64)),
                      dim3(64), 0, stream, faces, F, ext[0], ext[1], ext[2], nbr, u, gammas,
                      inv_jac, gbar, scratch_faces);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(transposed_sweeps_kernel,
-                     dim3(num_elements, (50 + kSweepChunk - 1) / kSweepChunk), dim3(256),
-                     sweep_lds, stream, ext[0], ext[1], ext[2], 50, scratch_du, ubar, dtab,
-                     scratch_faces, F);
-  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+  return launch_gh_adjoint_sweeps(num_elements, ext, gammas, inv_jac, gbar, scratch_du, ubar,
+                                  scratch_faces, F, stream);
 }
 
 int launch_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,

@@ -1654,10 +1654,10 @@ int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u, const double* 
     if (int rc = reserve_scratch(sc, 150 * static_cast<size_t>(d->total_points), 0);
         rc != SXD_OK)
       return finish(rc, __func__);
-    return finish(launch_mixed_gh_adjoint(d->num_elements, d->d_list, d->d_el, d->d_point_el,
-                                          d->total_points, d->d_nbr,
-                                          d->np_max, d->kf, d->km, u, gammas, inv_jac, gbar, ubar,
-                                          sc.du, static_cast<hipStream_t>(stream)),
+    return finish(launch_mixed_gh_adjoint(d->classes, d->d_list, d->d_el, d->d_point_el,
+                                          d->total_points, d->d_nbr, d->kf, d->km, u, gammas,
+                                          inv_jac, gbar, ubar, sc.du,
+                                          static_cast<hipStream_t>(stream)),
                   __func__);
   }
   const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];

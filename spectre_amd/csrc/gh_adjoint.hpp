@@ -25,27 +25,8 @@ namespace sxd {
 
 #define SXD_HD __host__ __device__ inline
 
-// Makes a pointer's value opaque to the optimiser: loads through it after
-// this point are not merged with loads made before it.  A long point-wise
-// adjoint re-reads its inputs (from cache) in each phase instead of keeping
-// every value it read alive in registers across phases.  On the device the
-// pointers are global memory (kernel arguments): the opaque value is a
-// global-space pointer, so the re-reads stay global loads rather than flat
-// ones (which also occupy the LDS counter).
-#if defined(__HIP_DEVICE_COMPILE__)
-#define SXD_REREAD(p)                                                     \
-  do {                                                                    \
-    auto sxd_q_ = (const __attribute__((address_space(1))) double*)(p);   \
-    asm volatile("" : "+v"(sxd_q_));                                      \
-    (p) = (const double*)sxd_q_;                                          \
-  } while (0)
-#else
-#define SXD_REREAD(p) asm volatile("" : "+r"(p))
-#endif
-
 namespace adj {
 SXD_HD int iaa(int i, int a, int b) { return i + 3 * sym4(a, b); }
-SXD_HD int ijaa(int i, int j, int a, int b) { return i + 3 * j + 9 * sym4(a, b); }
 SXD_HD int abb(int a, int b, int c) { return a + 4 * sym4(b, c); }
 SXD_HD double step(double x) { return x < 0.0 ? 0.0 : 1.0; }
 
@@ -121,7 +102,7 @@ SXD_HD void lapse_shift_vjp(const LapseShift& L, double isp_bar[6], double shift
 }  // namespace adj
 
 // Scalars of the linearisation point that the adjoint of the derivative
-// inputs needs (see gh_time_derivative_dubar).
+// inputs needs (see gh_pair_dubar).
 struct GhVjpPoint {
   double lapse, shift[3], isp[6];
 };
@@ -166,14 +147,37 @@ SXD_HD void add_slots(double* s_b, const double* G, double scale) {
 }
 }  // namespace adj
 
+// f is affine in the derivatives, so all that the adjoint with respect to u needs
+// of them are sums over the symmetric pairs, weighted by gbar (w_g, w_Pi,
+// w_Phi,i of pair ab, and s = gamma1 gamma2 w_Pi + (1 + gamma1) w_g):
+//   lapse    sum w_Phi,i (gamma2 dg(i, ab) - dPi(i, ab))
+//   shift_m  sum w_Pi dPi(m, ab) + w_Phi,i dPhi(m, i, ab) + s dg(m, ab)
+//   q(m, n)  sum w_Pi dPhi(m, n, ab), symmetric slots (off-diagonal ones hold
+//            both orders)
+struct GhDerivativeSums {
+  double lapse, shift[3], q[6];
+};
+
+// LDS pointer, and a statement that makes its value opaque to the optimiser: loads
+// after it are not merged with loads made before it.
+using LdsField = const __attribute__((address_space(3))) double*;
+#define SXD_REREAD_LDS(p) asm volatile("" : "+v"(p))
+// The same for a pointer to global memory (a kernel argument): the opaque value
+// is a global-space pointer, so that loads stay global rather than flat ones.
+#define SXD_REREAD(p)                                                     \
+  do {                                                                    \
+    auto sxd_q_ = (const __attribute__((address_space(1))) double*)(p);   \
+    asm volatile("" : "+v"(sxd_q_));                                      \
+    (p) = (const double*)sxd_q_;                                          \
+  } while (0)
+
 // Adjoint of the point-wise GH time derivative dt = f(u, du; gamma0..2) with
-// respect to u: ubar[50] is OVERWRITTEN with (df/du)^T gbar.  u, du and gbar
-// are read through strides (su, sdu, sg: the distance between components, 1
-// for packed arrays or Np for a Variables block in memory).  Layouts as
-// gh_time_derivative: u = (g, Pi, Phi), du = (d g at 3 p + i, d Pi at
-// 30 + 3 p + i, d Phi at 60 + i + 3 j + 9 p).  The adjoint with respect to du
-// (f is affine in du) is gh_time_derivative_dubar(pt, ...), from the
-// scalars returned in *pt.
+// respect to u: ubar[50] is OVERWRITTEN with (df/du)^T gbar.  u = (g, Pi, Phi) is
+// the point's column of an LDS block with su doubles between components: each
+// phase below reads it again instead of keeping it in registers, and one wave
+// per SIMD (all its registers are in use) hides no global latency.  gbar is read
+// through the stride sg.  The adjoint with respect to du is the caller's, from
+// the scalars returned in *pt.
 //
 // The quadratic terms of dt Pi are written as traces of 4x4 products so that
 // their adjoints come in closed form and few intermediates are alive at once:
@@ -186,16 +190,15 @@ SXD_HD void add_slots(double* s_b, const double* G, double scale) {
 //    2 sum_{de, n} Psi_n(mu, de) (P_n ig)(nu, de)  =  2 sum_n (Psi_n ig P_n)(mu, nu)
 //   -2 sum_{al, de} (C_mu ig)(al, de) (C_nu ig)(de, al) = -2 tr(C_mu ig C_nu ig)
 // each symmetric in (mu, nu).
-SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, int sdu,
-                                   double gamma0, double gamma1, double gamma2,
-                                   const double* gbar, int sg, double* ubar, GhVjpPoint* pt) {
+__device__ __forceinline__ void gh_time_derivative_vjp(LdsField u, int su,
+                                                       const GhDerivativeSums& sums,
+                                                       double gamma0, double gamma1,
+                                                       double gamma2, const double* gbar, int sg,
+                                                       double* ubar, GhVjpPoint* pt) {
   using namespace adj;
 #define G_(a, b) u[sym4(a, b) * su]
 #define PI_(a, b) u[(10 + sym4(a, b)) * su]
 #define PHI_(i, a, b) u[(20 + iaa(i, a, b)) * su]
-#define DG_(i, a, b) du[(3 * sym4(a, b) + (i)) * sdu]
-#define DPI_(i, a, b) du[(30 + 3 * sym4(a, b) + (i)) * sdu]
-#define DPHI_(i, j, a, b) du[(60 + ijaa(i, j, a, b)) * sdu]
 #define GB_(c) gbar[(c) * sg]
   // ---- metric quantities -------------------------------------------------
   LapseShift L;
@@ -245,8 +248,7 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
 #pragma unroll
     for (int b = 0; b < 4; ++b) H[4 * a + b] = (a == b ? 1.0 : 0.5) * GB_(10 + sym4(a, b));
 
-  SXD_REREAD(u);
-  SXD_REREAD(du);
+  SXD_REREAD_LDS(u);
   SXD_REREAD(gbar);
   // ---- Christoffel part: tc, the harmonic-gauge term, -2 tr(C ig C ig) -------
   {
@@ -322,7 +324,7 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
     for (int mu = 0; mu < 4; ++mu)
 #pragma unroll
       for (int nu = mu; nu < 4; ++nu) {
-        const double w = GB_(10 + sym4(mu, nu));
+        const double w = (mu == nu ? 1.0 : 2.0) * H[4 * mu + nu];
         double base;
         if (mu == 0 && nu == 0)
           base = 2.0 * tmp00 * tc[0] - ndgc * G_(0, 0);
@@ -381,8 +383,7 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
 
   // ---- Pi / Phi quadratic terms, and dt Phi -----------------------------------
   {
-    SXD_REREAD(u);
-    SXD_REREAD(du);
+    SXD_REREAD_LDS(u);
     SXD_REREAD(gbar);
     double pion[4];
 #pragma unroll
@@ -433,7 +434,8 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
       }
     };
     {
-      SXD_REREAD(u);
+      SXD_REREAD_LDS(u);
+      SXD_REREAD(gbar);
       // -2 (Pi ig Pi): d/dPi = -4 H Pi ig, d/dig = -2 Pi H Pi
       double Pf[16], Q[16], T[16], U[16];
 #pragma unroll
@@ -449,7 +451,8 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
       add_slots(ig_b, U, -2.0 * lapse);
 #pragma unroll
       for (int n = 0; n < 3; ++n) {
-        SXD_REREAD(u);
+        SXD_REREAD_LDS(u);
+        SXD_REREAD(gbar);
         // 2 tr(H Psi_n ig P_n): d/dPsi_n = 2 H P_n ig, d/dig = 2 Psi_n H P_n,
         // d/dP_n = 2 ig Psi_n H
         double Sf[16], Pn[16];
@@ -471,7 +474,8 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
         mul4(Q, H, T);     // ig Psi_n H
         double pb[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         add_slots(pb, T, 2.0 * lapse);
-        SXD_REREAD(u);
+        SXD_REREAD_LDS(u);
+        SXD_REREAD(gbar);
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -481,59 +485,56 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
           }
       }
     }
+    // the derivative terms, from their sums over the slots
+    lapse_b += sums.lapse;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) shift_b[m] += sums.shift[m];
+#pragma unroll
+    for (int x = 0; x < 6; ++x) {
+      lapse_b -= isp[x] * sums.q[x];
+      isp_b[x] -= lapse * sums.q[x];
+    }
     // slot by slot: the remaining terms of dt Pi (-hptn Pi
-    // - sum_m pion(m+1) Psi_m - sum_{m,n} isp(m, n) dPhi(m, n)
-    // + sum_m shift_m dPi(m)), dt Phi, and the C3 terms
+    // - sum_m pion(m+1) Psi_m), dt Phi, and the C3 terms
     //   dt Phi(i, ab) = S lapse + sum_m shift_m dPhi(m, i, ab),
     //   S = Pi(ab) hphi_i - dPi(i, ab) + gamma2 C3(i, ab)
     //       + sum_n pon[i + 3 (n + 1)] Psi(n, ab),  C3 = dg - Phi;
     //   dt g = dtg + (1 + gamma1) sdc3, dt Pi += gamma12 sdc3,
-    //   sdc3 = sum_m shift_m C3(m) (the dg part of C3's adjoint: dubar)
+    //   sdc3 = sum_m shift_m C3(m) (without derivatives)
     const double gamma12 = gamma1 * gamma2;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int b = a; b < 4; ++b) {
-        SXD_REREAD(u);
-        SXD_REREAD(du);
+        SXD_REREAD_LDS(u);
         SXD_REREAD(gbar);
         double ps[3], psb[3] = {0.0, 0.0, 0.0};
 #pragma unroll
         for (int n = 0; n < 3; ++n) ps[n] = psi_at(n, a, b);
         const double pi_ab = PI_(a, b);
+        const double wpi = (a == b ? 1.0 : 2.0) * H[4 * a + b];
         {
-          const double w = GB_(10 + sym4(a, b));
           double R = -hptn * pi_ab;
 #pragma unroll
-          for (int m = 0; m < 3; ++m) {
-            R += -pion[m + 1] * ps[m];
-#pragma unroll
-            for (int n = 0; n < 3; ++n) R += -isp[sym3(m, n)] * DPHI_(m, n, a, b);
-          }
-          lapse_b += w * R;
-#pragma unroll
-          for (int m = 0; m < 3; ++m) shift_b[m] += w * DPI_(m, a, b);
-          const double Rb = w * lapse;
+          for (int m = 0; m < 3; ++m) R += -pion[m + 1] * ps[m];
+          lapse_b += wpi * R;
+          const double Rb = wpi * lapse;
           hptn_b -= Rb * pi_ab;
           pi_b[sym4(a, b)] -= Rb * hptn;
 #pragma unroll
           for (int m = 0; m < 3; ++m) {
             pion_b[m + 1] -= Rb * ps[m];
             psb[m] -= Rb * pion[m + 1];
-#pragma unroll
-            for (int n = 0; n < 3; ++n) isp_b[sym3(m, n)] -= Rb * DPHI_(m, n, a, b);
           }
         }
         {
 #pragma unroll
           for (int i = 0; i < 3; ++i) {
             const double w = GB_(20 + iaa(i, a, b));
-            double S = pi_ab * hphi[i] - DPI_(i, a, b) + gamma2 * (DG_(i, a, b) - PHI_(i, a, b));
+            double S = pi_ab * hphi[i] - gamma2 * PHI_(i, a, b);
 #pragma unroll
             for (int n = 0; n < 3; ++n) S += pon[i + 3 * (n + 1)] * ps[n];
             lapse_b += w * S;
-#pragma unroll
-            for (int m = 0; m < 3; ++m) shift_b[m] += w * DPHI_(m, i, a, b);
             const double Sb = w * lapse;
             pi_b[sym4(a, b)] += Sb * hphi[i];
             hphi_b[i] += Sb * pi_ab;
@@ -546,17 +547,18 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
           }
           const double wg = GB_(sym4(a, b));
           dtg_b[sym4(a, b)] += wg;
-          const double sb = gamma12 * GB_(10 + sym4(a, b)) + (1.0 + gamma1) * wg;
+          const double sb = gamma12 * wpi + (1.0 + gamma1) * wg;
 #pragma unroll
           for (int m = 0; m < 3; ++m) {
-            shift_b[m] += sb * (DG_(m, a, b) - PHI_(m, a, b));
+            shift_b[m] -= sb * PHI_(m, a, b);
             phi_b[iaa(m, a, b)] -= sb * shift[m];
           }
         }
 #pragma unroll
         for (int n = 0; n < 3; ++n) psi_adjoint(n, a, b, psb[n]);
       }
-    SXD_REREAD(u);
+    SXD_REREAD_LDS(u);
+    SXD_REREAD(gbar);
     // hphi[n] = 0.5 sum_mu nv[mu] pon[n + 3 mu]
 #pragma unroll
     for (int n = 0; n < 3; ++n)
@@ -598,8 +600,7 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
     nv0_b -= nv_b[i + 1] * shift[i];
   }
   lapse_b -= nv0_b / (lapse * lapse);
-  SXD_REREAD(u);
-  SXD_REREAD(du);
+  SXD_REREAD_LDS(u);
   SXD_REREAD(gbar);
   // dtg(a b) = -lapse Pi(a b) + sum_m shift_m Phi(m, a, b)
 #pragma unroll
@@ -638,33 +639,29 @@ SXD_HD void gh_time_derivative_vjp(const double* u, int su, const double* du, in
 #undef G_
 #undef PI_
 #undef PHI_
-#undef DG_
-#undef DPI_
-#undef DPHI_
 #undef GB_
 }
 
-// Adjoint of the point-wise GH time derivative with respect to du component
-// c (layout of gh_time_derivative_vjp).  dt depends on du linearly:
+// Adjoint of the point-wise GH time derivative with respect to the 15 derivatives
+// of one symmetric pair ab, from gbar at the pair (w_g, w_Pi, w_Phi).  dt
+// depends on them linearly:
 //   dt_g(ab)     += (1 + gamma1) sum_n shift_n dg(n, ab)
 //   dt_Pi(ab)    += gamma1 gamma2 sum_n shift_n dg(n, ab) + sum_m shift_m dPi(m, ab)
 //                   - lapse sum_{m,n} isp(m, n) dPhi(m, n, ab)
 //   dt_Phi(i,ab) += lapse (gamma2 dg(i, ab) - dPi(i, ab)) + sum_m shift_m dPhi(m, i, ab)
-SXD_HD double gh_time_derivative_dubar(const GhVjpPoint& pt, double gamma1, double gamma2,
-                                       const double* gbar, int sg, int c) {
-  if (c < 30) {  // dg(n, ab), c = 3 p + n
-    const int p = c / 3, n = c % 3;
-    const double ggb = gbar[p * sg], gpb = gbar[(10 + p) * sg], gfb = gbar[(20 + n + 3 * p) * sg];
-    return gamma2 * gfb * pt.lapse + (gamma1 * gamma2 * gpb + (1.0 + gamma1) * ggb) * pt.shift[n];
+// out[i]: derivative i of the pair's field c (g, Pi, Phi_0..2).
+__device__ __forceinline__ void gh_pair_dubar(double out[3], int c, const GhVjpPoint& pt,
+                                              double gamma1, double gamma2, const double w[5]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (c == 0)
+      out[i] = gamma2 * w[2 + i] * pt.lapse +
+               (gamma1 * gamma2 * w[1] + (1.0 + gamma1) * w[0]) * pt.shift[i];
+    else if (c == 1)
+      out[i] = -w[2 + i] * pt.lapse + w[1] * pt.shift[i];
+    else
+      out[i] = w[c] * pt.shift[i] - w[1] * pt.lapse * pt.isp[sym3(i, c - 2)];
   }
-  if (c < 60) {  // dPi(i, ab), c = 30 + 3 p + i
-    const int p = (c - 30) / 3, i = (c - 30) % 3;
-    return -gbar[(20 + i + 3 * p) * sg] * pt.lapse + gbar[(10 + p) * sg] * pt.shift[i];
-  }
-  // dPhi(m, n, ab), c = 60 + m + 3 n + 9 p
-  const int r = c - 60, m = r % 3, n = (r / 3) % 3, p = r / 9;
-  return gbar[(20 + n + 3 * p) * sg] * pt.shift[m] -
-         gbar[(10 + p) * sg] * pt.lapse * pt.isp[sym3(m, n)];
 }
 
 // One side of a face point: unit normal covector/vector, magnitude and
@@ -907,6 +904,7 @@ SXD_HD void gh_face_pair_vjp(const double* u_p, double gamma1_p, double gamma2_p
   for (int c = 0; c < 10; ++c) ubar_p[c * sb] += gm_b[c];
 }
 
+#undef SXD_REREAD_LDS
 #undef SXD_REREAD
 #undef SXD_HD
 

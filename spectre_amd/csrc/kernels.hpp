@@ -332,15 +332,33 @@ int launch_mortar_pack(bool gh, const MortarPlan& plan, double* work, void* send
 int launch_mortar_unpack(bool gh, const MortarPlan& plan, double* work, const void* recv,
                          int64_t bytes, int count, int64_t step, int32_t* status,
                          hipStream_t stream);
+// Volume part of the GH adjoint (gh_adjoint_volume.hip); work: kGhAdjointDoubles
+// per point, filled by the points launch and read by the sweeps.  contrib: the
+// face terms [E][6][50][F] that the sweeps add.
+constexpr int kGhAdjointDoubles = 30;
+bool gh_adjoint_supported(const int32_t ext[3]);
+int launch_gh_adjoint_points(int num_elements, const int32_t ext[3], const double* u,
+                             const double* gammas, const double* inv_jac, const double* gbar,
+                             double* ubar, double* work, hipStream_t stream);
+int launch_gh_adjoint_sweeps(int num_elements, const int32_t ext[3], const double* gammas,
+                             const double* inv_jac, const double* gbar, const double* work,
+                             double* ubar, const double* contrib, int F, hipStream_t stream);
+int launch_ragged_gh_adjoint_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+                                    const MixedElement* el, const int32_t* point_el,
+                                    int64_t total_points, const double* u, const double* gammas,
+                                    const double* inv_jac, const double* gbar, double* ubar,
+                                    double* work, hipStream_t stream);
 // Adjoint of the GH RHS on a mixed-p domain, linearised at u: ubar =
-// (d dt / d u)^T gbar over the work list; scratch_du = 150 x total points.
+// (d dt / d u)^T gbar over the work list (all of its classes); scratch_du =
+// 150 x total points.
 int mixed_face_adjoint_lds_bytes(int kf, int km);
 // point_el: the element of each of the total_points grid points.
-int launch_mixed_gh_adjoint(int count, const int32_t* list, const MixedElement* el,
-                            const int32_t* point_el, int64_t total_points,
-                            const int32_t* nbr, int np_max, int kf, int km, const double* u,
-                            const double* gammas, const double* inv_jac, const double* gbar,
-                            double* ubar, double* scratch_du, hipStream_t stream);
+int launch_mixed_gh_adjoint(const std::vector<RaggedClass>& classes, const int32_t* list,
+                            const MixedElement* el, const int32_t* point_el,
+                            int64_t total_points, const int32_t* nbr, int kf, int km,
+                            const double* u, const double* gammas, const double* inv_jac,
+                            const double* gbar, double* ubar, double* scratch_du,
+                            hipStream_t stream);
 // Adjoint (transpose) of the ScalarWave RHS on a uniform domain (isotropic
 // extents 2..10) and of one RK3 substep.
 bool sw_adjoint_supported(const int32_t ext[3]);

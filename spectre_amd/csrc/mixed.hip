@@ -666,85 +666,9 @@ sw_mixed_face_kernel(const MixedElement* __restrict__ el, const int32_t* __restr
 
 // ---------------------------------------------------------------------------
 // Generalized harmonic adjoint on mixed-p domains (the RHS linearised at u):
-// the kernels of the uniform adjoint with per-element extents, and a face
+// the volume kernels of gh_adjoint_volume.hip with per-element extents, and a face
 // kernel that transposes the mortar coupling.
 //
-// Point-wise adjoint, one thread per grid point (point_el gives its
-// element): ubar = (df/du)^T gbar, and the logical-derivative adjoints xbar
-// written over du (read first, same point).
-__global__ void __launch_bounds__(128)
-gh_mixed_adjoint_pointwise_kernel(int64_t total, const MixedElement* __restrict__ el,
-                                  const int32_t* __restrict__ point_el,
-                                  const double* __restrict__ u, double* du_xbar,
-                                  const double* __restrict__ gammas,
-                                  const double* __restrict__ inv_jac,
-                                  const double* __restrict__ gbar, double* __restrict__ ubar) {
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= total) return;
-  const MixedElement m = el[point_el[gid]];
-  const int np = m.np;
-  const int p = static_cast<int>(gid - m.off);
-  const double* gp = gbar + 50 * m.off + p;
-  const double* ga = gammas + 3 * m.off + p;
-  const double gamma1 = ga[np], gamma2 = ga[2 * np];
-  double ub[50];
-  GhVjpPoint pt;
-  gh_time_derivative_vjp(u + 50 * m.off + p, np, du_xbar + 150 * m.off + p, np, ga[0], gamma1,
-                         gamma2, gp, np, ub, &pt);
-#pragma unroll
-  for (int c = 0; c < 50; ++c) ubar[50 * m.off + c * np + p] = ub[c];
-  double ij[9];
-#pragma unroll
-  for (int c = 0; c < 9; ++c) ij[c] = inv_jac[9 * m.off + c * np + p];
-  for (int c = 0; c < 50; ++c) {
-    double dub[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      dub[i] = gh_time_derivative_dubar(pt, gamma1, gamma2, gp, np, 3 * c + i);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      double s = 0.0;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) s += ij[ij3(j, i)] * dub[i];
-      du_xbar[150 * m.off + (3 * c + j) * np + p] = s;
-    }
-  }
-}
-
-// ubar_c += sum_j D_j^T xbar_cj per element.  Grid: (list length, component
-// chunks of kRaggedChunk); dynamic LDS: the element's D matrices
-// (kStagedDiffDoubles), then 3 Np_max doubles.
-__global__ void __launch_bounds__(256)
-ragged_transposed_sweeps_kernel(const MixedElement* __restrict__ el,
-                                const int32_t* __restrict__ list, int nc,
-                                const double* __restrict__ xbar, double* __restrict__ ubar,
-                                const double* __restrict__ dtab) {
-  extern __shared__ double s_lds[];
-  double* s_x = s_lds + kStagedDiffDoubles;
-  const MixedElement m = el[list[blockIdx.x]];
-  const int np = m.np;
-  const int stride[3] = {1, m.n[0], m.n[0] * m.n[1]};
-  const double* D[3];
-  stage_diff_matrices(dtab, m.n, s_lds, D);  // synchronised by the loop's first barrier
-  const int c_end = min(nc, static_cast<int>(blockIdx.y + 1) * kRaggedChunk);
-  for (int c = blockIdx.y * kRaggedChunk; c < c_end; ++c) {
-    __syncthreads();
-    for (int x = threadIdx.x; x < 3 * np; x += blockDim.x)
-      s_x[x] = xbar[3 * nc * m.off + 3 * c * np + x];
-    __syncthreads();
-    for (int p = threadIdx.x; p < np; p += blockDim.x) {
-      const int idx[3] = {p % m.n[0], (p / m.n[0]) % m.n[1], p / (m.n[0] * m.n[1])};
-      double acc = ubar[nc * m.off + c * np + p];
-      for (int j = 0; j < 3; ++j) {
-        const int base = p - idx[j] * stride[j];
-        for (int l = 0; l < m.n[j]; ++l)
-          acc = fma(D[j][l * m.n[j] + idx[j]], s_x[j * np + base + l * stride[j]], acc);
-      }
-      ubar[nc * m.off + c * np + p] = acc;
-    }
-  }
-}
-
 // Transpose of apply_face_matrices: in [NC][oa ob] -> out [NC][ia ib] with
 // Ma [oa][ia] (skipped when ia == oa) and Mb [ob][ib] (skipped when
 // ib == ob), dimension b first, through tmp [NC][oa ib]; work items as in
@@ -1265,8 +1189,6 @@ bool enable_large_lds() {
       hipFuncSetAttribute(reinterpret_cast<const void*>(&gh_mixed_face_adjoint_pass_kernel<false>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
       hipFuncSetAttribute(reinterpret_cast<const void*>(&gh_mixed_face_adjoint_pass_kernel<true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&ragged_transposed_sweeps_kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess)
     return false;
   done[dev] = true;
@@ -1406,34 +1328,26 @@ int mixed_face_adjoint_lds_bytes(int kf, int km) {
   return FaceAdjPassPlan<false>(kf, km).total * 8;
 }
 
-int launch_mixed_gh_adjoint(int count, const int32_t* list, const MixedElement* el,
-                            const int32_t* point_el, int64_t total_points,
-                            const int32_t* nbr, int np_max, int kf, int km, const double* u,
-                            const double* gammas, const double* inv_jac, const double* gbar,
-                            double* ubar, double* scratch_du, hipStream_t stream) {
-  if (count == 0) return SXD_OK;
-  const double* dtab = device_diff_matrices();
+int launch_mixed_gh_adjoint(const std::vector<RaggedClass>& classes, const int32_t* list,
+                            const MixedElement* el, const int32_t* point_el,
+                            int64_t total_points, const int32_t* nbr, int kf, int km,
+                            const double* u, const double* gammas, const double* inv_jac,
+                            const double* gbar, double* ubar, double* scratch_du,
+                            hipStream_t stream) {
   const double* mtab = device_mortar_matrices();
-  if (dtab == nullptr || mtab == nullptr) return SXD_ERR_DEVICE;
-  if (mixed_face_adjoint_lds_bytes(kf, km) > 160 * 1024 ||
-      (kStagedDiffDoubles + 3 * np_max) * 8 > 160 * 1024)
-    return SXD_ERR_UNSUPPORTED;
+  if (mtab == nullptr) return SXD_ERR_DEVICE;
+  int count = 0;
+  for (const RaggedClass& c : classes) {
+    count += c.count;
+    if ((kStagedDiffDoubles + 3 * c.np_max) * 8 > 160 * 1024) return SXD_ERR_UNSUPPORTED;
+  }
+  if (mixed_face_adjoint_lds_bytes(kf, km) > 160 * 1024) return SXD_ERR_UNSUPPORTED;
   if (scratch_du == nullptr) return SXD_ERR_INVALID_ARGUMENT;
   if (!enable_large_lds()) return SXD_ERR_DEVICE;
-  const dim3 chunks(count, (50 + kRaggedChunk - 1) / kRaggedChunk);
-  hipLaunchKernelGGL(ragged_partial_derivatives_kernel, chunks, dim3(256),
-                     (kStagedDiffDoubles + np_max) * 8, stream, el, list, 50, u, inv_jac,
-                     scratch_du, dtab);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(gh_mixed_adjoint_pointwise_kernel,
-                     dim3(static_cast<unsigned>((total_points + 127) / 128)), dim3(128), 0, stream,
-                     total_points, el, point_el, u, scratch_du, gammas, inv_jac, gbar, ubar);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(ragged_transposed_sweeps_kernel, chunks, dim3(256),
-                     (kStagedDiffDoubles + 3 * np_max) * 8, stream, el, list, 50, scratch_du, ubar,
-                     dtab);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  // faces: the derivative work array is free again and holds the side
+  const int rc = launch_ragged_gh_adjoint_volume(classes, list, el, point_el, total_points, u,
+                                                 gammas, inv_jac, gbar, ubar, scratch_du, stream);
+  if (rc != SXD_OK) return rc;
+  // faces: the work array is free again and holds the side
   // adjoints (110 doubles per point) and the side values of the current
   // dimension's face points (12 per point), under the 150 it has
   const int lds_split = FaceAdjPassPlan<false>(kf, km).total * 8;
