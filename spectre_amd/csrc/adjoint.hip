@@ -262,7 +262,6 @@ gh_adjoint_face_kernel(int64_t total, int F, int n0, int n1, int n2,
     if (s == 1) nq_row[i] = nq_row[i] * -1.0;
   }
   double* out = contrib + (e * 6 + dir) * 50 * static_cast<int64_t>(F) + f;
-  for (int c = 0; c < 50; ++c) out[c * F] = 0.0;
   // this element's face (d, s) at p and the neighbour's face (d, 1 - s) at
   // q: each point is the other's exterior
   gh_face_pair_vjp(u + e * 50 * np + p, gap[np], gap[2 * np], np_row, u + en * 50 * np + q,
@@ -306,11 +305,11 @@ int gh_adjoint_face_slots(const int32_t ext[3]) {
 
 int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t* nbr,
                           const double* u, const double* gammas, const double* inv_jac,
-                          const double* gbar, double* ubar, double* scratch_du,
+                          const double* gbar, double* ubar, double* work,
                           double* scratch_faces, hipStream_t stream) {
   if (!gh_adjoint_supported(ext)) return SXD_ERR_UNSUPPORTED;
   const int rc = launch_gh_adjoint_points(num_elements, ext, u, gammas, inv_jac, gbar, ubar,
-                                          scratch_du, stream);
+                                          work, stream);
   if (rc != SXD_OK) return rc;
   const int F = gh_adjoint_face_slots(ext);
   const int64_t faces = static_cast<int64_t>(num_elements) * 6 * F;
@@ -318,7 +317,7 @@ int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t*
                      dim3(64), 0, stream, faces, F, ext[0], ext[1], ext[2], nbr, u, gammas,
                      inv_jac, gbar, scratch_faces);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  return launch_gh_adjoint_sweeps(num_elements, ext, gammas, inv_jac, gbar, scratch_du, ubar,
+  return launch_gh_adjoint_sweeps(num_elements, ext, gammas, inv_jac, gbar, work, ubar,
                                   scratch_faces, F, stream);
 }
 

@@ -23,6 +23,8 @@ namespace sxd {
 // derivative array `du` and the per-point / per-face-slot temporaries.
 // Grown on demand (hipFree, then hipMalloc: a growth waits for the device),
 // or, when `fixed`, a caller-provided block that is never reallocated.
+constexpr int kAdjointBlock = 2;  // index in Scratch::block
+
 struct Scratch {
   // Held while a call enqueues its kernels: calls of several threads on one
   // stream take their turns, so that none of them writes the work arrays
@@ -30,9 +32,10 @@ struct Scratch {
   std::mutex enqueue;
   double* du = nullptr;
   double* temps = nullptr;
-  // Work arrays of one size per domain and system, so that they never move:
-  // the GH pair kernels' and the lifted corrections of mortar domains.
-  double* block[2] = {nullptr, nullptr};
+  // Work arrays of one size per domain, so that they never move:
+  // the ScalarWave corrections of mortar domains, the GH states and corrections,
+  // and the GH adjoint's.
+  double* block[3] = {nullptr, nullptr, nullptr};
   size_t du_doubles = 0, temps_doubles = 0;
   bool fixed = false;
   size_t fixed_doubles = 0;  // capacity of a fixed block
@@ -124,7 +127,7 @@ struct Scratch {
     }
     side = nullptr;
     fork = join = nullptr;
-    du = temps = block[0] = block[1] = nullptr;
+    du = temps = block[0] = block[1] = block[2] = nullptr;
     du_doubles = temps_doubles = 0;
   }
 };
@@ -1636,6 +1639,32 @@ int sxd_scalar_wave_rhs_adjoint(const sxd_domain* domain, const double* gbar, co
                 __func__);
 }
 
+namespace {
+// Face contributions, point-wise adjoint, then the transposed sweeps, which
+// add the contributions.
+int run_gh_adjoint_mixed(sxd_domain* d, Scratch& sc, const double* u, const double* gammas,
+                         const double* inv_jac, const double* gbar, double* ubar,
+                         hipStream_t stream) {
+  if (!d->conforming_plan || mixed_face_adjoint_lds_bytes(d->kf, d->km) > 160 * 1024 ||
+      (kStagedDiffDoubles + 3 * d->np_max) * 8 > 160 * 1024)
+    return SXD_ERR_UNSUPPORTED;
+  const size_t volume = kGhAdjointDoubles * static_cast<size_t>(d->total_points);
+  const GhAdjointFacesWork size(d->plan, nullptr);
+  if (int rc = sc.reserve_block(kAdjointBlock, size.doubles + volume); rc != SXD_OK) return rc;
+  const GhAdjointFacesWork w(d->plan, sc.block[kAdjointBlock]);
+  double* work = w.contrib + w.doubles;
+  int rc = launch_gh_adjoint_faces(d->plan, d->d_el, u, gammas, inv_jac, gbar, w.contrib, stream);
+  if (rc == SXD_OK)
+    rc = launch_ragged_gh_adjoint_points(d->classes, d->d_list, d->d_el, d->d_point_el,
+                                         d->total_points, u, gammas, inv_jac, gbar, ubar, work,
+                                         stream);
+  if (rc == SXD_OK)
+    rc = launch_ragged_gh_adjoint_sweeps(d->classes, d->d_list, d->d_el, gammas, inv_jac, gbar,
+                                         work, ubar, d->plan.d_corrections, w.contrib, stream);
+  return rc;
+}
+}  // namespace
+
 int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u, const double* gammas,
                        const double* inv_jac, const double* gbar, double* ubar, void* stream) {
   if (int rc = check_periodic(domain); rc != SXD_OK) return rc;
@@ -1650,23 +1679,19 @@ int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u, const double* 
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
   std::lock_guard<std::mutex> enqueue(sc.enqueue);
-  if (d->mixed) {
-    if (int rc = reserve_scratch(sc, 150 * static_cast<size_t>(d->total_points), 0);
-        rc != SXD_OK)
-      return finish(rc, __func__);
-    return finish(launch_mixed_gh_adjoint(d->classes, d->d_list, d->d_el, d->d_point_el,
-                                          d->total_points, d->d_nbr, d->kf, d->km, u, gammas,
-                                          inv_jac, gbar, ubar, sc.du,
-                                          static_cast<hipStream_t>(stream)),
+  if (d->mixed)
+    return finish(run_gh_adjoint_mixed(d, sc, u, gammas, inv_jac, gbar, ubar,
+                                       static_cast<hipStream_t>(stream)),
                   __func__);
-  }
   const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];
-  const size_t face_doubles = 300 * static_cast<size_t>(gh_adjoint_face_slots(d->ext));
-  if (int rc = reserve_scratch(sc, 150 * np * d->num_elements, face_doubles * d->num_elements);
-      rc != SXD_OK)
+  const size_t volume = kGhAdjointDoubles * np * d->num_elements;
+  const size_t faces = 300 * static_cast<size_t>(gh_adjoint_face_slots(d->ext)) * d->num_elements;
+  if (int rc = sc.reserve_block(kAdjointBlock, volume + faces); rc != SXD_OK)
     return finish(rc, __func__);
+  double* work = sc.block[kAdjointBlock];
   return finish(launch_gh_rhs_adjoint(d->num_elements, d->ext, d->d_nbr, u, gammas, inv_jac, gbar,
-                                      ubar, sc.du, sc.temps, static_cast<hipStream_t>(stream)),
+                                      ubar, work, work + volume,
+                                      static_cast<hipStream_t>(stream)),
                 __func__);
 }
 

@@ -727,20 +727,20 @@ SXD_HD void gh_side_vjp(const GhSideFwd& s, double gamma1, const double n_b_in[3
   adj::lapse_shift_vjp(s.L, isp_b, shift_b, lapse_b, gbar);
 }
 
-// Packaged fields of pair pr at one point (UpwindPenalty dg_package_data,
-// layout of gh_package_seed); u read with stride su.
+// Packaged fields of a pair at one point (UpwindPenalty dg_package_data,
+// layout of gh_package_seed) from its fields (g, Pi, Phi_0..2).
 SXD_HD void gh_package_fwd(const double n[3], const double nv[3], const double lam[4],
-                           double gamma2, const double* u, int su, int pr, double pk[13]) {
-  const double g = u[pr * su], pi = u[(10 + pr) * su];
-  const double* phi = u + (20 + 3 * pr) * su;
+                           double gamma2, const double fields[5], double pk[13]) {
+  const double g = fields[0], pi = fields[1];
+  const double* phi = fields + 2;
   const double g2g = gamma2 * g;
   double ndphi = 0.0;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) ndphi += nv[i] * phi[i * su];
+  for (int i = 0; i < 3; ++i) ndphi += nv[i] * phi[i];
   pk[4] = lam[2] * ((pi + ndphi) - g2g);
   pk[5] = lam[3] * ((pi - ndphi) - g2g);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) pk[1 + i] = lam[1] * (phi[i * su] - n[i] * ndphi);
+  for (int i = 0; i < 3; ++i) pk[1 + i] = lam[1] * (phi[i] - n[i] * ndphi);
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     pk[6 + d] = pk[4] * n[d];
@@ -797,20 +797,19 @@ SXD_HD void gh_package_seed(const double lam[4], const double bi[5], const doubl
   }
 }
 
-// Reverse of the package of pair pr at one point with unit normal n, normal
-// vector nv, speeds lam and gamma2: consumes the package adjoint B and ADDS
-// to the point's ubar (components g, Pi, Phi of pair pr, stride sb) and to
-// the adjoints of n, nv and lam.  u is read with stride su.
+// Reverse of the package of a pair at one point with unit normal n, normal
+// vector nv, speeds lam and gamma2: consumes the package adjoint B, writes the
+// adjoint of the pair's fields (g, Pi, Phi_0..2, given in `fields`) to out and
+// ADDS to the adjoints of n, nv and lam.
 SXD_HD void gh_package_vjp(const double n[3], const double nv[3], const double lam[4],
-                           double gamma2, const double* u, int su, int pr, double B[13],
-                           double* ubar, int sb, double n_b[3], double nv_b[3],
-                           double lam_b[4]) {
-  const double g = u[pr * su], pi = u[(10 + pr) * su];
-  const double* phi = u + (20 + 3 * pr) * su;
+                           double gamma2, const double fields[5], double B[13], double out[5],
+                           double n_b[3], double nv_b[3], double lam_b[4]) {
+  const double g = fields[0], pi = fields[1];
+  const double* phi = fields + 2;
   const double g2g = gamma2 * g;
   double ndphi = 0.0;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) ndphi += nv[i] * phi[i * su];
+  for (int i = 0; i < 3; ++i) ndphi += nv[i] * phi[i];
   const double pk4 = lam[2] * ((pi + ndphi) - g2g), pk5 = lam[3] * ((pi - ndphi) - g2g);
   double g2g_b = 0.0, ndphi_b = 0.0, pi_b = 0.0, g_b = 0.0, phi_b[3] = {0, 0, 0};
   // pk12 = g2g lam0; pk0 = lam0 g
@@ -827,7 +826,7 @@ SXD_HD void gh_package_vjp(const double n[3], const double nv[3], const double l
   // pk1+i = lam1 (phi_i - n_i ndphi)
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    lam_b[1] += B[1 + i] * (phi[i * su] - n[i] * ndphi);
+    lam_b[1] += B[1 + i] * (phi[i] - n[i] * ndphi);
     const double ib = B[1 + i] * lam[1];
     phi_b[i] += ib;
     n_b[i] -= ib * ndphi;
@@ -843,14 +842,14 @@ SXD_HD void gh_package_vjp(const double n[3], const double nv[3], const double l
   // ndphi = nv . phi; g2g = gamma2 g
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    nv_b[i] += ndphi_b * phi[i * su];
+    nv_b[i] += ndphi_b * phi[i];
     phi_b[i] += ndphi_b * nv[i];
   }
   g_b += g2g_b * gamma2;
-  ubar[pr * sb] += g_b;
-  ubar[(10 + pr) * sb] += pi_b;
+  out[0] = g_b;
+  out[1] = pi_b;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) ubar[(20 + 3 * pr + i) * sb] += phi_b[i];
+  for (int i = 0; i < 3; ++i) out[2 + i] = phi_b[i];
 }
 
 // Adjoint of the lifted GH UpwindPenalty corrections of one face point pair,
@@ -863,8 +862,8 @@ SXD_HD void gh_package_vjp(const double n[3], const double nv[3], const double l
 // unnormalised normal covector at p pointing out of p's element (the
 // inverse-Jacobian row, sign applied) and n_q the one at q, as the forward
 // uses them.  Given gbar_p and gbar_q, the adjoints of dt at p and q (50
-// components, stride sg), ADDS d/du_p of <gbar_p, dt(p)> + <gbar_q, dt(q)>
-// to ubar_p (50 components, stride sb).  u_p and u_q are read with stride su.
+// components, stride sg), writes d/du_p of <gbar_p, dt(p)> + <gbar_q, dt(q)>
+// to ubar_p (50 components, stride sb; OVERWRITTEN).  u_p and u_q are read with stride su.
 SXD_HD void gh_face_pair_vjp(const double* u_p, double gamma1_p, double gamma2_p,
                              const double n_p[3], const double* u_q, double gamma1_q,
                              double gamma2_q, const double n_q[3], int n_perp, int su,
@@ -877,11 +876,18 @@ SXD_HD void gh_face_pair_vjp(const double* u_p, double gamma1_p, double gamma2_p
   const double lift = -0.5 * static_cast<double>(n_perp * (n_perp - 1));
   const double fac_p = lift * sp.mag, fac_q = lift * sq.mag;
   double n_b[3] = {0, 0, 0}, nv_b[3] = {0, 0, 0}, lam_b[4] = {0, 0, 0, 0}, fac_b = 0.0;
+  double gm_b[10];
+#pragma unroll
   for (int pr = 0; pr < 10; ++pr) {
     const int comp[5] = {pr, 10 + pr, 20 + 3 * pr, 21 + 3 * pr, 22 + 3 * pr};
-    double pkp[13], pkq[13];
-    gh_package_fwd(sp.n, sp.nv, sp.lam, gamma2_p, u_p, su, pr, pkp);
-    gh_package_fwd(sq.n, sq.nv, sq.lam, gamma2_q, u_q, su, pr, pkq);
+    double pkp[13], pkq[13], fp[5], fq[5], out[5];
+#pragma unroll
+    for (int c = 0; c < 5; ++c) {
+      fp[c] = u_p[comp[c] * su];
+      fq[c] = u_q[comp[c] * su];
+    }
+    gh_package_fwd(sp.n, sp.nv, sp.lam, gamma2_p, fp, pkp);
+    gh_package_fwd(sq.n, sq.nv, sq.lam, gamma2_q, fq, pkq);
     // correction at p (p interior): its value feeds fac_p's adjoint
     double bc[5];
     gh_boundary_fwd(pkp, sp.lam, pkq, sq.lam, bc);
@@ -895,13 +901,15 @@ SXD_HD void gh_face_pair_vjp(const double* u_p, double gamma1_p, double gamma2_p
     // p's package: interior of the correction at p, exterior of the one at q
     double B[13];
     gh_package_seed(sp.lam, bp_b, bq_b, B);
-    gh_package_vjp(sp.n, sp.nv, sp.lam, gamma2_p, u_p, su, pr, B, ubar_p, sb, n_b, nv_b, lam_b);
+    gh_package_vjp(sp.n, sp.nv, sp.lam, gamma2_p, fp, B, out, n_b, nv_b, lam_b);
+    gm_b[pr] = out[0];
+#pragma unroll
+    for (int c = 1; c < 5; ++c) ubar_p[comp[c] * sb] = out[c];
   }
   // fac_p = lift |n_p|; the normals and speeds of p's side depend on g(p)
-  double gm_b[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   gh_side_vjp(sp, gamma1_p, n_b, nv_b, lam_b, fac_b * lift, gm_b);
 #pragma unroll
-  for (int c = 0; c < 10; ++c) ubar_p[c * sb] += gm_b[c];
+  for (int c = 0; c < 10; ++c) ubar_p[c * sb] = gm_b[c];
 }
 
 #undef SXD_REREAD_LDS

@@ -7,7 +7,7 @@
 //     values into ubar) and the scalars that the adjoint of the derivatives needs;
 //   gh_adjoint_sweeps_kernel: one workgroup per (element, pair): the adjoint of
 //     the pair's 15 derivatives from gbar, contracted into logical ones in LDS,
-//     transposed differentiation sweeps, and (uniform domains) the face terms.
+//     transposed differentiation sweeps, and the face terms.
 //
 // 30 doubles per point go through the work array.  The arrangement before wrote
 // 150 derivatives and 150 derivative adjoints per point and read both back, and
@@ -220,7 +220,8 @@ gh_adjoint_point_kernel(int64_t total, int np_uniform, const MixedElement* __res
 
 // S fields of the pair at a time (5, or 1 where their 15 Np derivative adjoints
 // leave fewer than two workgroups per CU).  Dynamic LDS: 3 S Np doubles, then
-// the D matrices.  contrib (uniform domains): face terms [E][6][50][F].
+// the D matrices.  contrib: face terms, [E][6][50][F] (uniform domains) or per
+// record as `table` places them.
 template <bool RAGGED, int S>
 __global__ void __launch_bounds__(512)
 gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* __restrict__ el,
@@ -228,7 +229,7 @@ gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* 
                          const double* __restrict__ inv_jac, const double* __restrict__ gbar,
                          const double* __restrict__ work, double* __restrict__ ubar,
                          const double* __restrict__ dtab, const double* __restrict__ contrib,
-                         int F) {
+                         int F, const MortarCorrection* __restrict__ table) {
   extern __shared__ double s_lds[];
   int64_t at;
   int pr;
@@ -309,6 +310,21 @@ gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* 
 #pragma unroll
           for (int c = 0; c < S; ++c) acc[c] += from[static_cast<int64_t>(comp[c0 + c]) * F];
         }
+      } else {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const int at_d = d == 0 ? i : d == 1 ? j : k, nd = n[d];
+          if (at_d != 0 && at_d != nd - 1) continue;
+          const int nf = d == 0 ? m.n1 * m.n2 : d == 1 ? m.n0 * m.n2 : m.n0 * m.n1;
+          const int f = d == 0 ? j + m.n1 * k : d == 1 ? i + m.n0 * k : i + m.n0 * j;
+          const MortarCorrection lower = table[6 * m.e + 2 * d];
+          const MortarCorrection upper = table[6 * m.e + 2 * d + 1];
+          const int mortars = at_d == 0 ? lower.count : upper.count;
+          const double* from = contrib + 50 * (at_d == 0 ? lower.off : upper.off) + f;
+          for (int q = 0; q < mortars; ++q, from += 50 * nf)
+#pragma unroll
+            for (int c = 0; c < S; ++c) acc[c] += from[comp[c0 + c] * nf];
+        }
       }
 #pragma unroll
       for (int c = 0; c < S; ++c) (ube + comp[c0 + c] * np)[p] = acc[c];
@@ -357,7 +373,8 @@ template <bool RAGGED>
 int launch_sweeps(int count, int np, int d_doubles, const int32_t ext[3], const MixedElement* el,
                   const int32_t* list, const double* gammas, const double* inv_jac,
                   const double* gbar, const double* work, double* ubar, const double* dtab,
-                  const double* contrib, int F, hipStream_t stream) {
+                  const double* contrib, int F, const MortarCorrection* table,
+                  hipStream_t stream) {
   const bool five = 2 * (15 * np + d_doubles) <= kLdsDoubles;
   const int lds = ((five ? 15 : 3) * np + d_doubles) * 8;
   const void* kernel = five
@@ -369,11 +386,11 @@ int launch_sweeps(int count, int np, int d_doubles, const int32_t ext[3], const 
   if (five)
     hipLaunchKernelGGL((gh_adjoint_sweeps_kernel<RAGGED, 5>), dim3(blocks), dim3(threads), lds,
                        stream, count, ext[0], ext[1], ext[2], el, list, gammas, inv_jac, gbar,
-                       work, ubar, dtab, contrib, F);
+                       work, ubar, dtab, contrib, F, table);
   else
     hipLaunchKernelGGL((gh_adjoint_sweeps_kernel<RAGGED, 1>), dim3(blocks), dim3(threads), lds,
                        stream, count, ext[0], ext[1], ext[2], el, list, gammas, inv_jac, gbar,
-                       work, ubar, dtab, contrib, F);
+                       work, ubar, dtab, contrib, F, table);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 }  // namespace
@@ -404,10 +421,10 @@ int launch_gh_adjoint_sweeps(int num_elements, const int32_t ext[3], const doubl
   const int np = ext[0] * ext[1] * ext[2];
   const int d_doubles = ext[0] * ext[0] + ext[1] * ext[1] + ext[2] * ext[2];
   return launch_sweeps<false>(num_elements, np, d_doubles, ext, nullptr, nullptr, gammas, inv_jac,
-                              gbar, work, ubar, dtab, contrib, F, stream);
+                              gbar, work, ubar, dtab, contrib, F, nullptr, stream);
 }
 
-int launch_ragged_gh_adjoint_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+int launch_ragged_gh_adjoint_points(const std::vector<RaggedClass>& classes, const int32_t* list,
                                     const MixedElement* el, const int32_t* point_el,
                                     int64_t total_points, const double* u, const double* gammas,
                                     const double* inv_jac, const double* gbar, double* ubar,
@@ -423,10 +440,21 @@ int launch_ragged_gh_adjoint_volume(const std::vector<RaggedClass>& classes, con
   hipLaunchKernelGGL(gh_adjoint_point_kernel<true>,
                      dim3(static_cast<unsigned>((total_points + 63) / 64)), dim3(64), 0, stream,
                      total_points, 0, el, point_el, u, gammas, gbar, work, ubar);
-  if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+}
+
+int launch_ragged_gh_adjoint_sweeps(const std::vector<RaggedClass>& classes, const int32_t* list,
+                                    const MixedElement* el, const double* gammas,
+                                    const double* inv_jac, const double* gbar,
+                                    const double* work, double* ubar,
+                                    const MortarCorrection* table, const double* contrib,
+                                    hipStream_t stream) {
+  const double* dtab = device_diff_matrices();
+  if (dtab == nullptr) return SXD_ERR_DEVICE;
+  const int32_t none[3] = {0, 0, 0};
   for (const RaggedClass& c : classes) {
     const int rc = launch_sweeps<true>(c.count, c.np_max, c.d_doubles, none, el, list + c.begin,
-                                       gammas, inv_jac, gbar, work, ubar, dtab, nullptr, 0,
+                                       gammas, inv_jac, gbar, work, ubar, dtab, contrib, 0, table,
                                        stream);
     if (rc != SXD_OK) return rc;
   }

@@ -210,9 +210,9 @@ struct MortarJob {
   MortarSide side[2];
 };
 // Mortars launched together: [begin, begin + count) of d_jobs, and the largest
-// LDS of one of them.
+// LDS of one of them, for the corrections and for their adjoint.
 struct MortarClass {
-  int begin, count, lds_bytes;
+  int begin, count, lds_bytes, adjoint_lds_bytes;
 };
 // Boundary messages (the BoundaryMessage of
 // Evolution/DiscontinuousGalerkin/Messages/BoundaryMessage.hpp for DG mortar
@@ -307,6 +307,20 @@ struct MortarCorrectionsWork {
   size_t doubles;
   MortarCorrectionsWork(bool gh, const MortarPlan& plan, double* work);
 };
+int launch_gh_mortar_sides(const MortarPlan& plan, const MixedElement* el, const double* u,
+                           const double* params, const double* inv_jac, double* sides,
+                           double* speeds, hipStream_t stream);
+// Face part of the GH adjoint (gh_adjoint_faces.hip): every record's
+// contribution to its element's ubar, [50][nf] at 50 corr_off of work.contrib.
+int gh_adjoint_mortar_lds_bytes(const MortarRecord& r, const MortarRecord& partner);
+struct GhAdjointFacesWork {
+  double *contrib, *side_adj, *sides, *speeds;
+  size_t doubles;
+  GhAdjointFacesWork(const MortarPlan& plan, double* work);
+};
+int launch_gh_adjoint_faces(const MortarPlan& plan, const MixedElement* el, const double* u,
+                            const double* gammas, const double* inv_jac, const double* gbar,
+                            double* work, hipStream_t stream);
 int launch_mortar_lifted_corrections(bool gh, const MortarPlan& plan, const MixedElement* el,
                                      const double* u, const double* params,
                                      const double* inv_jac, double* work, hipStream_t stream);
@@ -343,22 +357,21 @@ int launch_gh_adjoint_points(int num_elements, const int32_t ext[3], const doubl
 int launch_gh_adjoint_sweeps(int num_elements, const int32_t ext[3], const double* gammas,
                              const double* inv_jac, const double* gbar, const double* work,
                              double* ubar, const double* contrib, int F, hipStream_t stream);
-int launch_ragged_gh_adjoint_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
+// The same on a ragged domain, in two steps (point_el: the element of each of the
+// total_points grid points); table, contrib: launch_gh_adjoint_faces' work.
+int launch_ragged_gh_adjoint_points(const std::vector<RaggedClass>& classes, const int32_t* list,
                                     const MixedElement* el, const int32_t* point_el,
                                     int64_t total_points, const double* u, const double* gammas,
                                     const double* inv_jac, const double* gbar, double* ubar,
                                     double* work, hipStream_t stream);
-// Adjoint of the GH RHS on a mixed-p domain, linearised at u: ubar =
-// (d dt / d u)^T gbar over the work list (all of its classes); scratch_du =
-// 150 x total points.
+int launch_ragged_gh_adjoint_sweeps(const std::vector<RaggedClass>& classes, const int32_t* list,
+                                    const MixedElement* el, const double* gammas,
+                                    const double* inv_jac, const double* gbar,
+                                    const double* work, double* ubar,
+                                    const MortarCorrection* table, const double* contrib,
+                                    hipStream_t stream);
+// Largest LDS of the face kernel the mixed-p adjoint's size limit stems from.
 int mixed_face_adjoint_lds_bytes(int kf, int km);
-// point_el: the element of each of the total_points grid points.
-int launch_mixed_gh_adjoint(const std::vector<RaggedClass>& classes, const int32_t* list,
-                            const MixedElement* el, const int32_t* point_el,
-                            int64_t total_points, const int32_t* nbr, int kf, int km,
-                            const double* u, const double* gammas, const double* inv_jac,
-                            const double* gbar, double* ubar, double* scratch_du,
-                            hipStream_t stream);
 // Adjoint (transpose) of the ScalarWave RHS on a uniform domain (isotropic
 // extents 2..10) and of one RK3 substep.
 bool sw_adjoint_supported(const int32_t ext[3]);
@@ -367,12 +380,12 @@ int launch_sw_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t*
                           double* ubar, hipStream_t stream);
 // Adjoint of the GH RHS linearised at u (uniform extents with
 // 3 Np + N0^2 + N1^2 + N2^2 <= 20480):
-// ubar = (d dt / d u)^T gbar; scratch_du: 150 x E x Np doubles; scratch_faces:
-// 300 x E x gh_adjoint_face_slots(ext) doubles.
+// ubar = (d dt / d u)^T gbar; work: kGhAdjointDoubles x E x Np doubles;
+// scratch_faces: 300 x E x gh_adjoint_face_slots(ext) doubles.
 int gh_adjoint_face_slots(const int32_t ext[3]);
 int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t* nbr,
                           const double* u, const double* gammas, const double* inv_jac,
-                          const double* gbar, double* ubar, double* scratch_du,
+                          const double* gbar, double* ubar, double* work,
                           double* scratch_faces, hipStream_t stream);
 int launch_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,
                                const double* a, double* mu, double* lam_out, hipStream_t stream);

@@ -35,7 +35,6 @@
 #include <vector>
 
 #include "device_common.hpp"
-#include "gh_adjoint.hpp"
 #include "gh_point.hpp"
 #include "kernels.hpp"
 #include "sw_point.hpp"
@@ -665,111 +664,6 @@ sw_mixed_face_kernel(const MixedElement* __restrict__ el, const int32_t* __restr
 }
 
 // ---------------------------------------------------------------------------
-// Generalized harmonic adjoint on mixed-p domains (the RHS linearised at u):
-// the volume kernels of gh_adjoint_volume.hip with per-element extents, and a face
-// kernel that transposes the mortar coupling.
-//
-// Transpose of apply_face_matrices: in [NC][oa ob] -> out [NC][ia ib] with
-// Ma [oa][ia] (skipped when ia == oa) and Mb [ob][ib] (skipped when
-// ib == ob), dimension b first, through tmp [NC][oa ib]; work items as in
-// apply_face_matrices.  Includes the barriers between the steps.
-template <int NC, int G>
-__device__ void apply_face_matrices_t(int oa, int ob, int ia, int ib, const double* Ma,
-                                      const double* Mb, const double* in, double* tmp,
-                                      double* out) {
-  constexpr int NG = (NC + G - 1) / G;
-  const int t = threadIdx.x, T = blockDim.x;
-  const double* src = in;
-  if (ib != ob) {
-    for (int x = t; x < G * oa * ib; x += T) {
-      const int g = x / (oa * ib), y = x % (oa * ib), lb = y / oa, ra = y % oa;
-      const double* v = in + g * NG * oa * ob + ra;
-      double acc[NG];
-#pragma unroll
-      for (int c = 0; c < NG; ++c) acc[c] = g * NG + c < NC ? Mb[lb] * v[c * oa * ob] : 0.0;
-      for (int r = 1; r < ob; ++r) {
-        const double m = Mb[r * ib + lb];
-#pragma unroll
-        for (int c = 0; c < NG; ++c)
-          if (g * NG + c < NC) acc[c] = fma(m, v[c * oa * ob + oa * r], acc[c]);
-      }
-#pragma unroll
-      for (int c = 0; c < NG; ++c)
-        if (g * NG + c < NC) tmp[(g * NG + c) * oa * ib + y] = acc[c];
-    }
-    __syncthreads();
-    src = tmp;
-  }
-  for (int x = t; x < G * ia * ib; x += T) {
-    const int g = x / (ia * ib), y = x % (ia * ib), lb = y / ia, la = y % ia;
-    const double* v = src + g * NG * oa * ib + oa * lb;
-    double acc[NG];
-    if (ia == oa) {
-#pragma unroll
-      for (int c = 0; c < NG; ++c) acc[c] = g * NG + c < NC ? v[c * oa * ib + la] : 0.0;
-    } else {
-#pragma unroll
-      for (int c = 0; c < NG; ++c) acc[c] = g * NG + c < NC ? Ma[la] * v[c * oa * ib] : 0.0;
-      for (int r = 1; r < oa; ++r) {
-        const double m = Ma[r * ia + la];
-#pragma unroll
-        for (int c = 0; c < NG; ++c)
-          if (g * NG + c < NC) acc[c] = fma(m, v[c * oa * ib + r], acc[c]);
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < NG; ++c)
-      if (g * NG + c < NC) out[(g * NG + c) * ia * ib + y] = acc[c];
-  }
-  __syncthreads();
-}
-
-// Side values of face point f of element m's face (d, side); the raw normal
-// is negated when `flip`.
-__device__ void face_side_adjoint(const MixedElement& m, int d, int side, bool flip, int f,
-                                  const double* __restrict__ u, const double* __restrict__ params,
-                                  const double* __restrict__ inv_jac, GhSideFwd& s, int* point) {
-  const int na = d == 0 ? m.n[1] : m.n[0];
-  const int p = face_point(m, d, side, f % na, f / na);
-  double n[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    n[i] = inv_jac[9 * m.off + ij3(d, i) * m.np + p];
-    if (flip) n[i] = n[i] * -1.0;
-  }
-  gh_side_forward(s, u + 50 * m.off + p, m.np, params[3 * m.off + m.np + p], n);
-  *point = p;
-}
-
-// Side values of every face point of the faces normal to dimension d, both
-// sides of every element of the list, as face_side_adjoint forms them (the
-// normal taken outward): n, nv, lam[4], gamma2, |n| at sides[12 (off + p)].
-// Grid: (list length, 2 sides).
-__global__ void __launch_bounds__(128)
-gh_mixed_face_sides_kernel(int d, const MixedElement* __restrict__ el,
-                           const int32_t* __restrict__ list, const double* __restrict__ u,
-                           const double* __restrict__ params,
-                           const double* __restrict__ inv_jac, double* __restrict__ sides) {
-  const int side = blockIdx.y;
-  const MixedElement m = el[list[blockIdx.x]];
-  const int na = d == 0 ? m.n[1] : m.n[0], nb = d == 2 ? m.n[1] : m.n[2];
-  for (int f = threadIdx.x; f < na * nb; f += blockDim.x) {
-    GhSideFwd s;
-    int p;
-    face_side_adjoint(m, d, side, side == 0, f, u, params, inv_jac, s, &p);
-    double* o = sides + 12 * (m.off + p);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      o[i] = s.n[i];
-      o[3 + i] = s.nv[i];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) o[6 + k] = s.lam[k];
-    o[10] = params[3 * m.off + 2 * m.np + p];
-    o[11] = s.mag;
-  }
-}
-
 // GH faces, one pass per workgroup: grid (list length, 2 sides, 10 pairs) for
 // the faces normal to dimension d, so every (face, pair) runs concurrently.
 // Each workgroup packages its pair on both face meshes together with the
@@ -954,219 +848,6 @@ gh_mixed_face_pass_kernel(int d, const MixedElement* __restrict__ el,
   }
 }
 
-// GH face adjoint, one pass per workgroup: grid (list length, 2 sides, 10
-// pairs) for the faces normal to dimension d, as gh_mixed_face_pass_kernel.
-// Workgroup (e, side, pr) adds to e's points on face (d, side) the adjoint,
-// for pair pr, of e's own lifted correction and of the neighbour's (in which
-// e is the exterior side): the forward is recomputed up to the mortar
-// corrections, then
-//   seeds   gbar * lift factor on both faces (the neighbour's with its own),
-//   P^T     each seed projected back onto the mortar (transposed projection),
-//   weights the adjoint of e's package on the mortar, interior for its own
-//           correction and exterior for the neighbour's, from the upwind
-//           weights of the mortar speeds,
-//   I^T     transposed interpolation onto e's face,
-//   package reverse at e's face points into ubar (the pair's components).
-// The adjoints of e's normals, speeds and |n| from this pair go to side_adj
-// (11 per pair at each face point, indexed by the point's volume index);
-// gh_mixed_side_adjoint_kernel sums them over the pairs and takes them to g.
-// Dynamic LDS: FaceAdjPassPlan(kf, km).total doubles.
-// kFusedNb as in FacePassPlan: without a mortar buffer for the neighbour side.
-template <bool kFusedNb>
-struct FaceAdjPassPlan {
-  int side, mag_nb, face, tmp, m_own, m_nb, total;
-  __host__ __device__ FaceAdjPassPlan(int kf, int km) {
-    side = 0;                // own face point: n, nv, lam, gamma2, |n|
-    mag_nb = side + 12 * kf;  // |n| of the neighbour's face points
-    face = mag_nb + kf;       // 17 per face point (speeds, package); then
-                              // corrections, seeds, package adjoint
-    tmp = face + 17 * kf;
-    m_own = tmp + 17 * km;   // own speeds, package; then corrections, seeds on
-                             // the mortar, package adjoint (all in place)
-    m_nb = m_own + 17 * km;  // the neighbour side on the mortar
-    total = m_nb + (kFusedNb ? 0 : 17 * km);
-  }
-};
-
-template <bool kFusedNb>
-__global__ void __launch_bounds__(256, 3)
-gh_mixed_face_adjoint_pass_kernel(int d, const MixedElement* __restrict__ el,
-                                  const int32_t* __restrict__ list,
-                                  const int32_t* __restrict__ nbr, const double* __restrict__ u,
-                                  const double* __restrict__ params,
-                                  const double* __restrict__ inv_jac,
-                                  const double* __restrict__ gbar, double* __restrict__ ubar,
-                                  double* __restrict__ side_adj,
-                                  const double* __restrict__ sides,
-                                  const double* __restrict__ mortar_tab, int kf, int km) {
-  extern __shared__ double sm[];
-  const FaceAdjPassPlan<kFusedNb> L(kf, km);
-  const int t = threadIdx.x, T = blockDim.x;
-  const int side = blockIdx.y, pr = blockIdx.z;
-  const int e = list[blockIdx.x];
-  const MixedElement m = el[e];
-  const MixedElement mn = el[nbr[6 * e + 2 * d + side]];
-  const int na = d == 0 ? m.n[1] : m.n[0], nb = d == 2 ? m.n[1] : m.n[2];
-  const int ma = d == 0 ? mn.n[1] : mn.n[0], mb = d == 2 ? mn.n[1] : mn.n[2];
-  const int ka = max(na, ma), kb = max(nb, mb);
-  const int nf = na * nb, mf = ma * mb, kmf = ka * kb;
-  const double* Ia_own = mortar_tab + mortar_table_offset(na, ka);
-  const double* Ib_own = mortar_tab + mortar_table_offset(nb, kb);
-  const double* Ia_nb = mortar_tab + mortar_table_offset(ma, ka);
-  const double* Ib_nb = mortar_tab + mortar_table_offset(mb, kb);
-  const double* Pa = Ia_own + na * ka;  // projection block follows the interpolation
-  const double* Pb = Ib_own + nb * kb;
-  const double* Pa_nb = Ia_nb + ma * ka;
-  const double* Pb_nb = Ib_nb + mb * kb;
-  const double lift_own = lift_factor(ext_at(m, d), 1.0), lift_nb = lift_factor(ext_at(mn, d), 1.0);
-  const int comp[5] = {pr, 10 + pr, 20 + 3 * pr, 21 + 3 * pr, 22 + 3 * pr};
-  double* face = sm + L.face;
-  // own side: side values (gh_mixed_face_sides_kernel), speeds and package
-  // of the pair
-  for (int f = t; f < nf; f += T) {
-    const int p = face_point(m, d, side, f % na, f / na);
-    const double* sv = sides + 12 * (m.off + p);
-    double* o = sm + L.side + 12 * f;
-#pragma unroll
-    for (int c = 0; c < 12; ++c) o[c] = sv[c];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) face[k * nf + f] = o[6 + k];
-    double pk[13];
-    gh_package_fwd(o, o + 3, o + 6, o[10], u + 50 * m.off + p, m.np, pr, pk);
-#pragma unroll
-    for (int c = 0; c < 13; ++c) face[(4 + c) * nf + f] = pk[c];
-  }
-  __syncthreads();
-  apply_face_matrices<17, 2>(na, nb, ka, kb, Ia_own, Ib_own, face, sm + L.tmp, sm + L.m_own);
-  for (int f = t; f < mf; f += T) {
-    const int q = face_point(mn, d, 1 - side, f % ma, f / ma);
-    double sv[12];
-#pragma unroll
-    for (int c = 0; c < 12; ++c) sv[c] = sides[12 * (mn.off + q) + c];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) face[k * mf + f] = sv[6 + k];
-    sm[L.mag_nb + f] = sv[11];
-    double pk[13];
-    gh_package_fwd(sv, sv + 3, sv + 6, sv[10], u + 50 * mn.off + q, mn.np, pr, pk);
-#pragma unroll
-    for (int c = 0; c < 13; ++c) face[(4 + c) * mf + f] = pk[c];
-  }
-  __syncthreads();
-  // the neighbour side on the mortar (as apply_face_matrices; with kFusedNb
-  // its dimension-b sums are formed per mortar point below), and e's
-  // corrections there, over e's package slots
-  const double* src_nb = face;
-  if constexpr (!kFusedNb) {
-    apply_face_matrices<17, 2>(ma, mb, ka, kb, Ia_nb, Ib_nb, face, sm + L.tmp, sm + L.m_nb);
-  } else if (ma != ka) {
-    face_matrix_a<17, 2>(ma, mb, ka, Ia_nb, face, sm + L.tmp);
-    __syncthreads();
-    src_nb = sm + L.tmp;
-  }
-  for (int k = t; k < kmf; k += T) {
-    double in[13], li[4], nbv[17], bc[5];  // nbv: neighbour speeds, package
-#pragma unroll
-    for (int c = 0; c < 4; ++c) li[c] = sm[L.m_own + c * kmf + k];
-#pragma unroll
-    for (int c = 0; c < 13; ++c) in[c] = sm[L.m_own + (4 + c) * kmf + k];
-    if constexpr (!kFusedNb) {
-#pragma unroll
-      for (int c = 0; c < 17; ++c) nbv[c] = sm[L.m_nb + c * kmf + k];
-    } else {
-      face_matrix_b_point<17>(mb, ka, kb, Ib_nb, src_nb, k % ka, k / ka, nbv);
-    }
-    gh_boundary_fwd(in, li, nbv + 4, nbv, bc);
-#pragma unroll
-    for (int c = 0; c < 5; ++c) sm[L.m_own + (4 + c) * kmf + k] = bc[c];
-  }
-  __syncthreads();
-  apply_face_matrices<5, 1>(ka, kb, na, nb, Pa, Pb, sm + L.m_own + 4 * kmf, sm + L.tmp, face);
-  // seeds on both faces; the pair's part of the |n| adjoint of e's lift factor
-  double* seed_own = face + 5 * kf;
-  double* seed_nb = face + 10 * kf;
-  for (int f = t; f < nf; f += T) {
-    const int p = face_point(m, d, side, f % na, f / na);
-    const double fac = lift_own * sm[L.side + 12 * f + 11];
-    double fac_b = 0.0;
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      const double gb = gbar[50 * m.off + comp[c] * m.np + p];
-      fac_b += gb * face[c * nf + f];
-      seed_own[c * nf + f] = gb * fac;
-    }
-    side_adj[110 * (m.off + p) + 11 * pr + 10] = lift_own * fac_b;
-  }
-  for (int f = t; f < mf; f += T) {
-    const int q = face_point(mn, d, 1 - side, f % ma, f / ma);
-    const double fac = lift_nb * sm[L.mag_nb + f];
-#pragma unroll
-    for (int c = 0; c < 5; ++c)
-      seed_nb[c * mf + f] = gbar[50 * mn.off + comp[c] * mn.np + q] * fac;
-  }
-  __syncthreads();
-  apply_face_matrices_t<5, 1>(na, nb, ka, kb, Pa, Pb, seed_own, sm + L.tmp,
-                              sm + L.m_own + 4 * kmf);
-  apply_face_matrices_t<5, 1>(ma, mb, ka, kb, Pa_nb, Pb_nb, seed_nb, sm + L.tmp,
-                        sm + L.m_own + 9 * kmf);
-  for (int k = t; k < kmf; k += T) {
-    double li[4], bi[5], bx[5], B[13];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) li[c] = sm[L.m_own + c * kmf + k];
-#pragma unroll
-    for (int c = 0; c < 5; ++c) {
-      bi[c] = sm[L.m_own + (4 + c) * kmf + k];
-      bx[c] = sm[L.m_own + (9 + c) * kmf + k];
-    }
-    gh_package_seed(li, bi, bx, B);
-#pragma unroll
-    for (int c = 0; c < 13; ++c) sm[L.m_own + c * kmf + k] = B[c];
-  }
-  __syncthreads();
-  apply_face_matrices_t<13, 2>(ka, kb, na, nb, Ia_own, Ib_own, sm + L.m_own, sm + L.tmp, face);
-  for (int f = t; f < nf; f += T) {
-    const double* o = sm + L.side + 12 * f;
-    const int p = face_point(m, d, side, f % na, f / na);
-    double B[13], a[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int c = 0; c < 13; ++c) B[c] = face[c * nf + f];
-    gh_package_vjp(o, o + 3, o + 6, o[10], u + 50 * m.off + p, m.np, pr, B,
-                   ubar + 50 * m.off + p, m.np, a, a + 3, a + 6);
-    double* out = side_adj + 110 * (m.off + p) + 11 * pr;
-#pragma unroll
-    for (int c = 0; c < 10; ++c) out[c] = a[c];
-  }
-}
-
-// The adjoints of e's normals, speeds and |n| on the faces normal to
-// dimension d, summed over the ten pairs in order, into g.  Grid: (list
-// length, 2 sides).
-__global__ void __launch_bounds__(256)
-gh_mixed_side_adjoint_kernel(int d, const MixedElement* __restrict__ el,
-                             const int32_t* __restrict__ list, const double* __restrict__ u,
-                             const double* __restrict__ params,
-                             const double* __restrict__ inv_jac,
-                             const double* __restrict__ side_adj, double* __restrict__ ubar) {
-  const int side = blockIdx.y;
-  const MixedElement m = el[list[blockIdx.x]];
-  const int na = d == 0 ? m.n[1] : m.n[0], nb = d == 2 ? m.n[1] : m.n[2];
-  for (int f = threadIdx.x; f < na * nb; f += blockDim.x) {
-    GhSideFwd s;
-    int p;
-    face_side_adjoint(m, d, side, side == 0, f, u, params, inv_jac, s, &p);
-    const double* in = side_adj + 110 * (m.off + p);
-    double a[11];
-#pragma unroll
-    for (int c = 0; c < 11; ++c) a[c] = in[c];
-    for (int pr = 1; pr < 10; ++pr)
-#pragma unroll
-      for (int c = 0; c < 11; ++c) a[c] += in[11 * pr + c];
-    double gm_b[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    gh_side_vjp(s, params[3 * m.off + m.np + p], a, a + 3, a + 6, a[10], gm_b);
-#pragma unroll
-    for (int c = 0; c < 10; ++c) ubar[50 * m.off + c * m.np + p] += gm_b[c];
-  }
-}
-
 // Dynamic LDS beyond the default 64 KiB has to be enabled per kernel; done
 // once per device (before any graph capture of these launches).
 bool enable_large_lds() {
@@ -1185,10 +866,6 @@ bool enable_large_lds() {
       hipFuncSetAttribute(reinterpret_cast<const void*>(&gh_mixed_face_pass_kernel<false>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
       hipFuncSetAttribute(reinterpret_cast<const void*>(&gh_mixed_face_pass_kernel<true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gh_mixed_face_adjoint_pass_kernel<false>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess ||
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gh_mixed_face_adjoint_pass_kernel<true>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, lds_max) != hipSuccess)
     return false;
   done[dev] = true;
@@ -1324,54 +1001,6 @@ int launch_mixed_gh_face_passes(int count, const int32_t* list, const MixedEleme
   return SXD_OK;
 }
 
-int mixed_face_adjoint_lds_bytes(int kf, int km) {
-  return FaceAdjPassPlan<false>(kf, km).total * 8;
-}
-
-int launch_mixed_gh_adjoint(const std::vector<RaggedClass>& classes, const int32_t* list,
-                            const MixedElement* el, const int32_t* point_el,
-                            int64_t total_points, const int32_t* nbr, int kf, int km,
-                            const double* u, const double* gammas, const double* inv_jac,
-                            const double* gbar, double* ubar, double* scratch_du,
-                            hipStream_t stream) {
-  const double* mtab = device_mortar_matrices();
-  if (mtab == nullptr) return SXD_ERR_DEVICE;
-  int count = 0;
-  for (const RaggedClass& c : classes) {
-    count += c.count;
-    if ((kStagedDiffDoubles + 3 * c.np_max) * 8 > 160 * 1024) return SXD_ERR_UNSUPPORTED;
-  }
-  if (mixed_face_adjoint_lds_bytes(kf, km) > 160 * 1024) return SXD_ERR_UNSUPPORTED;
-  if (scratch_du == nullptr) return SXD_ERR_INVALID_ARGUMENT;
-  if (!enable_large_lds()) return SXD_ERR_DEVICE;
-  const int rc = launch_ragged_gh_adjoint_volume(classes, list, el, point_el, total_points, u,
-                                                 gammas, inv_jac, gbar, ubar, scratch_du, stream);
-  if (rc != SXD_OK) return rc;
-  // faces: the work array is free again and holds the side
-  // adjoints (110 doubles per point) and the side values of the current
-  // dimension's face points (12 per point), under the 150 it has
-  const int lds_split = FaceAdjPassPlan<false>(kf, km).total * 8;
-  const int lds_fused = FaceAdjPassPlan<true>(kf, km).total * 8;
-  const bool fused_nb = 160 * 1024 / lds_fused > 160 * 1024 / lds_split;
-  double* sides = scratch_du + 110 * total_points;
-  for (int d = 0; d < 3; ++d) {
-    hipLaunchKernelGGL(gh_mixed_face_sides_kernel, dim3(count, 2), dim3(128), 0, stream, d, el,
-                       list, u, gammas, inv_jac, sides);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-    if (fused_nb)
-      hipLaunchKernelGGL(gh_mixed_face_adjoint_pass_kernel<true>, dim3(count, 2, 10), dim3(256),
-                         lds_fused, stream, d, el, list, nbr, u, gammas, inv_jac, gbar, ubar,
-                         scratch_du, sides, mtab, kf, km);
-    else
-      hipLaunchKernelGGL(gh_mixed_face_adjoint_pass_kernel<false>, dim3(count, 2, 10),
-                         dim3(256), lds_split, stream, d, el, list, nbr, u, gammas, inv_jac,
-                         gbar, ubar, scratch_du, sides, mtab, kf, km);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-    hipLaunchKernelGGL(gh_mixed_side_adjoint_kernel, dim3(count, 2), dim3(128), 0, stream, d, el,
-                       list, u, gammas, inv_jac, scratch_du, ubar);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  }
-  return SXD_OK;
-}
+int mixed_face_adjoint_lds_bytes(int kf, int km) { return (30 * kf + 51 * km) * 8; }
 
 }  // namespace sxd

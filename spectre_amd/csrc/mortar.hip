@@ -960,10 +960,14 @@ int build_mortar_plan(int num_elements, const int32_t* extents, int num_records,
         return sys == 0 ? 0 : fit >= 8 ? 8 : fit >= 4 ? 4 : fit >= 2 ? 2 : 1;
       };
       for (int i = 0; i < static_cast<int>(pairs.size());) {
-        MortarClass c{i, 0, 0};
+        MortarClass c{i, 0, 0, 0};
         for (; i < static_cast<int>(pairs.size()) && tier(pairs[i]) == tier(pairs[c.begin]);
-             ++i, ++c.count)
+             ++i, ++c.count) {
           c.lds_bytes = std::max(c.lds_bytes, lds(sys == 1, pairs[i]));
+          c.adjoint_lds_bytes =
+              std::max(c.adjoint_lds_bytes,
+                       gh_adjoint_mortar_lds_bytes(recs[pairs[i]], recs[recs[pairs[i]].partner]));
+        }
         plan->classes[sys].push_back(c);
       }
     }

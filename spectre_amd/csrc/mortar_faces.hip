@@ -29,53 +29,10 @@
 #include "device_common.hpp"
 #include "gh_point.hpp"
 #include "kernels.hpp"
-#include "sw_point.hpp"
+#include "mortar_side.hpp"
 
 namespace sxd {
 namespace {
-
-constexpr int kPk = 13;  // packaged values of a point and pair
-
-// A dimension is the identity where the mortar covers all of it (matrix in the
-// Full table) with the face's extent.
-__host__ __device__ inline bool projects_a(const MortarSide& r) {
-  return r.mat_a < 0 || r.na != r.ka;
-}
-__host__ __device__ inline bool projects_b(const MortarSide& r) {
-  return r.mat_b < 0 || r.nb != r.kb;
-}
-
-// LDS of one side (doubles): the face package where dimension a is projected,
-// the staged values (dimension a done; later the corrections with dimension a
-// projected back), and the side's matrices (face to mortar, then mortar to
-// face, per projected dimension).
-struct SideLds {
-  int face, staged, mat_a, mat_b, mag;
-  __host__ __device__ SideLds(bool proj_a, bool proj_b, int na, int nb, int ka, int kb, bool gh) {
-    const int fwd = kPk * ka * nb, back = 5 * na * kb;
-    face = proj_a ? kPk * na * nb : 0;
-    staged = fwd > back ? fwd : back;
-    mat_a = proj_a ? 2 * na * ka : 0;
-    mat_b = proj_b ? 2 * nb * kb : 0;
-    mag = gh ? 0 : na * nb;
-  }
-  __host__ __device__ SideLds(const MortarSide& r, bool gh)
-      : SideLds(projects_a(r), projects_b(r), r.na, r.nb, r.ka, r.kb, gh) {}
-};
-
-// The corrections of both sides lie over the face packages.
-__host__ __device__ inline int corrections_doubles(int km, const SideLds& a, const SideLds& b) {
-  const int faces = a.face + b.face, bc = 10 * km;
-  return faces > bc ? faces : bc;
-}
-
-// x / n for x < 8000 and n <= 20 with one multiplication.
-__device__ __forceinline__ unsigned divisor(int n) {
-  return ((1u << 20) + static_cast<unsigned>(n) - 1) / static_cast<unsigned>(n);
-}
-__device__ __forceinline__ int divide(int x, unsigned m) {
-  return static_cast<int>((static_cast<unsigned>(x) * m) >> 20);
-}
 
 __device__ __forceinline__ int volume_index(const MixedElement& m, int d, int side, int a,
                                             int b) {
@@ -174,41 +131,6 @@ gh_mortar_sides_kernel(const MixedElement* __restrict__ el, const MortarFace* __
   }
 }
 
-// v[j] of the packaged values OFF[j] at mortar point (ra, rb) of a side:
-// dimension b of the interpolation (row: the matrix row of rb, null for the
-// identity) from the staged values.
-template <int O0, int O1, int O2, int O3>
-__device__ __forceinline__ void mortar_values(double v[4], const double* staged, const double* row,
-                                              int nb, int ka, int ra, int rb) {
-  const double* at = staged + kPk * ra;
-  if (row == nullptr) {
-    at += kPk * ka * rb;
-    v[0] = at[O0], v[1] = at[O1], v[2] = at[O2], v[3] = at[O3];
-    return;
-  }
-  double w = row[0];
-  v[0] = w * at[O0], v[1] = w * at[O1], v[2] = w * at[O2], v[3] = w * at[O3];
-#pragma unroll 2
-  for (int l = 1; l < nb; ++l) {
-    at += kPk * ka;
-    w = row[l];
-    v[0] = fma(w, at[O0], v[0]);
-    v[1] = fma(w, at[O1], v[1]);
-    v[2] = fma(w, at[O2], v[2]);
-    v[3] = fma(w, at[O3], v[3]);
-  }
-}
-
-template <bool GH>
-__device__ __forceinline__ void boundary_terms(double bc[5], const double in[13],
-                                               const double lam_in[4], const double ex[13],
-                                               const double lam_ex[4]) {
-  if constexpr (GH)
-    gh_boundary_terms_pair(bc, in, lam_in, ex, lam_ex);
-  else
-    sw_boundary_terms(bc, in, ex);
-}
-
 // Grid: GH 10 workgroups per job, one per symmetric pair (next to each other on
 // one XCD, padded to a multiple of 8 jobs); ScalarWave one workgroup per job.
 // corr: [NC][nf] per side at NC corr_off, the lifted corrections of the side's
@@ -233,228 +155,31 @@ mortar_corrections_kernel(int count, const MortarJob* __restrict__ jobs,
   const MortarSide& r0 = jobs[at].side[0];
   const MortarSide& r1 = jobs[at].side[1];
   const SideLds l0(r0, GH), l1(r1, GH);
-  const int nf0 = r0.nf, nf1 = r1.nf, km = r0.ka * r0.kb;
-  double* s_face0 = s_lds;
-  double* s_face1 = s_face0 + l0.face;
-  double* s_bc0 = s_lds;
-  double* s_bc1 = s_bc0 + 5 * km;
-  double* s_st0 = s_lds + corrections_doubles(km, l0, l1);
-  double* s_st1 = s_st0 + l0.staged;
-  double* s_ma0 = s_st1 + l1.staged;
-  double* s_mb0 = s_ma0 + l0.mat_a;
-  double* s_ma1 = s_mb0 + l0.mat_b;
-  double* s_mb1 = s_ma1 + l1.mat_a;
-  double* s_mag0 = s_mb1 + l1.mat_b;
-  double* s_mag1 = s_mag0 + l0.mag;
-  const int t = threadIdx.x, T = blockDim.x;
-  const unsigned by_na0 = divisor(r0.na), by_na1 = divisor(r1.na);
-  const unsigned by_ka0 = divisor(r0.ka), by_ka1 = divisor(r1.ka);
-  {
-    auto block = [&](int mat) { return mat >= 0 ? full + mat : half + (-1 - mat); };
-    const double* a0 = block(r0.mat_a);
-    const double* b0 = block(r0.mat_b);
-    const double* a1 = block(r1.mat_a);
-    const double* b1 = block(r1.mat_b);
-    for (int x = t; x < l0.mat_a; x += T) s_ma0[x] = a0[x];
-    for (int x = t; x < l0.mat_b; x += T) s_mb0[x] = b0[x];
-    for (int x = t; x < l1.mat_a; x += T) s_ma1[x] = a1[x];
-    for (int x = t; x < l1.mat_b; x += T) s_mb1[x] = b1[x];
-  }
+  const int km = r0.ka * r0.kb;
+  const MortarLds sh(s_lds, km, l0, l1, corrections_doubles(km, l0, l1), l0.staged + l1.staged);
   const int comp[5] = {pr, GH ? 10 + pr : 1, GH ? 20 + 3 * pr : 2, GH ? 21 + 3 * pr : 3,
                        GH ? 22 + 3 * pr : 4};
-  // 1. packages
-  for (int x = t; x < nf0 + nf1; x += T) {
-    const bool second = x >= nf0;
-    const MortarSide& r = second ? r1 : r0;
-    const int f = second ? x - nf0 : x;
-    const int nf = second ? nf1 : nf0, np = r.np;
-    const int b = divide(f, second ? by_na1 : by_na0), a = f - b * r.na;
-    const int p = r.base + a * r.step_a + b * r.step_b;
-    double pk[kPk];
-    if constexpr (GH) {
-      const double* sd = sides + 12 * r.pt_off + f;
-      GhFaceSide s;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        s.n[i] = sd[i * nf];
-        s.nv[i] = sd[(3 + i) * nf];
-      }
-#pragma unroll
-      for (int c = 0; c < 4; ++c) s.lam[c] = sd[(6 + c) * nf];
-      s.gamma2 = sd[10 * nf];
-      const double* ue = u + 50 * r.off + p;
-      double phi[3];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) phi[i] = ue[comp[2 + i] * np];
-      gh_package_pair(pk, ue[comp[0] * np], ue[comp[1] * np], phi, s);
-    } else {
-      double n[3], up[5], mag;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        n[i] = inv_jac[9 * r.off + ij3(r.dim, i) * np + p];
-        if (r.side == 0) n[i] = n[i] * -1.0;
-      }
-#pragma unroll
-      for (int c = 0; c < 5; ++c) up[c] = u[5 * r.off + c * np + p];
-      flat_normalize(n, &mag);
-      sw_package(pk, up, params[r.off + p], n);
-      (second ? s_mag1 : s_mag0)[f] = mag;
-    }
-    double* out = (second ? (l1.face > 0 ? s_face1 : s_st1) : (l0.face > 0 ? s_face0 : s_st0)) +
-                  kPk * f;
-#pragma unroll
-    for (int c = 0; c < kPk; ++c) out[c] = pk[c];
-  }
-  __syncthreads();
-  // 2. dimension a onto the mortar: a work item is two output points of one
-  // line for 5 of the 13 values (groups from 0, 4 and 8)
-  if (l0.face + l1.face > 0) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const MortarSide& r = s == 0 ? r0 : r1;
-      if ((s == 0 ? l0.face : l1.face) == 0) continue;
-      const double* in = s == 0 ? s_face0 : s_face1;
-      const double* M = s == 0 ? s_ma0 : s_ma1;
-      double* out = s == 0 ? s_st0 : s_st1;
-      const int half_ka = (r.ka + 1) / 2, items = half_ka * r.nb;
-      const unsigned by_half = divisor(half_ka);
-      for (int x = t; x < 3 * items; x += T) {
-        const int g = (x >= items) + (x >= 2 * items), y = x - g * items;
-        const int lb = divide(y, by_half), ra = 2 * (y - lb * half_ka);
-        const bool two = ra + 1 < r.ka;
-        const double* v = in + kPk * r.na * lb + 4 * g;
-        const double* w0 = M + ra * r.na;
-        const double* w1 = two ? w0 + r.na : w0;
-        double s0[5], s1[5];
-#pragma unroll
-        for (int c = 0; c < 5; ++c) {
-          s0[c] = w0[0] * v[c];
-          s1[c] = w1[0] * v[c];
-        }
-  #pragma unroll 2
-      for (int l = 1; l < r.na; ++l) {
-          v += kPk;
-          const double a = w0[l], b = w1[l];
-#pragma unroll
-          for (int c = 0; c < 5; ++c) {
-            s0[c] = fma(a, v[c], s0[c]);
-            s1[c] = fma(b, v[c], s1[c]);
-          }
-        }
-        double* o = out + kPk * (r.ka * lb + ra) + 4 * g;
-#pragma unroll
-        for (int c = 0; c < 5; ++c) o[c] = s0[c];
-        if (two) {
-#pragma unroll
-          for (int c = 0; c < 5; ++c) o[kPk + c] = s1[c];
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // 3. boundary terms: groups 0..2 the Phi_g output (values 1 + g, 6 + g,
-  // 9 + g), group 3 the g and Pi outputs (values 0, 4, 5, 12)
-  for (int x = t; x < 4 * km; x += T) {
-    const int g = (x >= km) + (x >= 2 * km) + (x >= 3 * km), k = x - g * km;
-    const int q = gather[r0.rec_off + k];
-    const int rb0 = divide(k, by_ka0), ra0 = k - rb0 * r0.ka;
-    const int rb1 = divide(q, by_ka1), ra1 = q - rb1 * r1.ka;
-    const double* row0 = l0.mat_b > 0 ? s_mb0 + rb0 * r0.nb : nullptr;
-    const double* row1 = l1.mat_b > 0 ? s_mb1 + rb1 * r1.nb : nullptr;
-    double lam0[4] = {0, 0, 0, 0}, lam1[4] = {0, 0, 0, 0};
-    if constexpr (GH) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        lam0[c] = speeds[4 * r0.rec_off + c * km + k];
-        lam1[c] = speeds[4 * r1.rec_off + c * km + q];
-      }
-    }
-    double p0[13], p1[13], bc[5], v[4];
-    if (g < 3) {
-      mortar_values<1, 6, 9, 9>(v, s_st0 + g, row0, r0.nb, r0.ka, ra0, rb0);
-      p0[1] = v[0], p0[6] = v[1], p0[9] = v[2];
-      mortar_values<1, 6, 9, 9>(v, s_st1 + g, row1, r1.nb, r1.ka, ra1, rb1);
-      p1[1] = v[0], p1[6] = v[1], p1[9] = v[2];
-      boundary_terms<GH>(bc, p0, lam0, p1, lam1);
-      s_bc0[5 * k + 2 + g] = bc[2];
-      boundary_terms<GH>(bc, p1, lam1, p0, lam0);
-      s_bc1[5 * q + 2 + g] = bc[2];
-    } else {
-      mortar_values<0, 4, 5, 12>(v, s_st0, row0, r0.nb, r0.ka, ra0, rb0);
-      p0[0] = v[0], p0[4] = v[1], p0[5] = v[2], p0[12] = v[3];
-      mortar_values<0, 4, 5, 12>(v, s_st1, row1, r1.nb, r1.ka, ra1, rb1);
-      p1[0] = v[0], p1[4] = v[1], p1[5] = v[2], p1[12] = v[3];
-      boundary_terms<GH>(bc, p0, lam0, p1, lam1);
-      s_bc0[5 * k] = bc[0];
-      s_bc0[5 * k + 1] = bc[1];
-      boundary_terms<GH>(bc, p1, lam1, p0, lam0);
-      s_bc1[5 * q] = bc[0];
-      s_bc1[5 * q + 1] = bc[1];
-    }
-  }
-  __syncthreads();
-  // 4. dimension a back to the face, both sides' lines as one list
-  if (l0.mat_a + l1.mat_a > 0) {
-    const int items0 = l0.mat_a > 0 ? r0.na * r0.kb : 0;
-    const int items1 = l1.mat_a > 0 ? r1.na * r1.kb : 0;
-    for (int x = t; x < items0 + items1; x += T) {
-      const bool second = x >= items0;
-      const int y = second ? x - items0 : x;
-      const int na = second ? r1.na : r0.na, ka = second ? r1.ka : r0.ka;
-      const int lb = divide(y, second ? by_na1 : by_na0), ra = y - lb * na;
-      const double* v = (second ? s_bc1 : s_bc0) + 5 * ka * lb;
-      const double* w = (second ? s_ma1 : s_ma0) + na * ka + ra * ka;
-      double s[5];
-#pragma unroll
-      for (int c = 0; c < 5; ++c) s[c] = w[0] * v[c];
-#pragma unroll 2
-      for (int l = 1; l < ka; ++l) {
-        v += 5;
-        const double a = w[l];
-#pragma unroll
-        for (int c = 0; c < 5; ++c) s[c] = fma(a, v[c], s[c]);
-      }
-      double* o = (second ? s_st1 : s_st0) + 5 * y;
-#pragma unroll
-      for (int c = 0; c < 5; ++c) o[c] = s[c];
-    }
-    __syncthreads();
-  }
+  mortar_terms<GH>(r0, r1, l0, l1, sh, comp, gather, u, params, inv_jac, sides, speeds, full,
+                   half);
   // 5. dimension b back to the face, and lift
-  for (int x = t; x < nf0 + nf1; x += T) {
-    const bool second = x >= nf0;
+  const unsigned by_na0 = divisor(r0.na), by_na1 = divisor(r1.na);
+  for (int x = threadIdx.x; x < r0.nf + r1.nf; x += blockDim.x) {
+    const bool second = x >= r0.nf;
     const MortarSide& r = second ? r1 : r0;
-    const int f = second ? x - nf0 : x;
-    const int nf = second ? nf1 : nf0, na = r.na;
-    const int fb = divide(f, second ? by_na1 : by_na0), fa = f - fb * na;
-    const double* v =
-        (second ? (l1.mat_a > 0 ? s_st1 : s_bc1) : (l0.mat_a > 0 ? s_st0 : s_bc0)) + 5 * fa;
-    double s[5];
-    if ((second ? l1.mat_b : l0.mat_b) > 0) {
-      const int nb = r.nb, kb = r.kb;
-      const double* w = (second ? s_mb1 : s_mb0) + nb * kb + fb * kb;
-#pragma unroll
-      for (int c = 0; c < 5; ++c) s[c] = w[0] * v[c];
-#pragma unroll 2
-      for (int l = 1; l < kb; ++l) {
-        v += 5 * na;
-        const double a = w[l];
-#pragma unroll
-        for (int c = 0; c < 5; ++c) s[c] = fma(a, v[c], s[c]);
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 5; ++c) s[c] = v[5 * na * fb + c];
-    }
+    const int f = second ? x - r0.nf : x, nf = r.nf;
+    const int fb = divide(f, second ? by_na1 : by_na0), fa = f - fb * r.na;
+    double v[5];
+    mortar_face_value(v, r, second ? l1.mat_a > 0 : l0.mat_a > 0,
+                      second ? l1.mat_b > 0 : l0.mat_b > 0, sh, second, fa, fb);
     double mag;
     if constexpr (GH)
       mag = sides[12 * r.pt_off + 11 * nf + f];
     else
-      mag = (second ? s_mag1 : s_mag0)[f];
+      mag = sh.mag(second)[f];
     const double fac = lift_factor(r.extent, mag);
     double* out = corr + NC * r.corr_off + f;
 #pragma unroll
-    for (int c = 0; c < 5; ++c) out[comp[c] * nf] = s[c] * fac;
+    for (int c = 0; c < 5; ++c) out[comp[c] * nf] = v[c] * fac;
   }
 }
 
@@ -478,6 +203,18 @@ MortarCorrectionsWork::MortarCorrectionsWork(bool gh, const MortarPlan& plan, do
             (gh ? 12 * plan.face_points + 4 * plan.record_points : 0);
 }
 
+int launch_gh_mortar_sides(const MortarPlan& plan, const MixedElement* el, const double* u,
+                           const double* params, const double* inv_jac, double* sides,
+                           double* speeds, hipStream_t stream) {
+  const double* full = device_mortar_matrices();
+  const double* half = device_half_mortar_matrices();
+  if (full == nullptr || half == nullptr) return SXD_ERR_DEVICE;
+  hipLaunchKernelGGL(gh_mortar_sides_kernel, dim3(plan.num_faces), dim3(128),
+                     8 * 4 * (plan.kf + plan.tmp_max), stream, el, plan.d_faces, plan.d_records, u,
+                     params, inv_jac, sides, speeds, full, half, plan.kf);
+  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+}
+
 int launch_mortar_lifted_corrections(bool gh, const MortarPlan& plan, const MixedElement* el,
                                      const double* u, const double* params,
                                      const double* inv_jac, double* work, hipStream_t stream) {
@@ -487,11 +224,8 @@ int launch_mortar_lifted_corrections(bool gh, const MortarPlan& plan, const Mixe
   if (work == nullptr || plan.num_remote > 0) return SXD_ERR_INVALID_ARGUMENT;
   const MortarCorrectionsWork w(gh, plan, work);
   if (gh) {
-    const int lds = 8 * 4 * (plan.kf + plan.tmp_max);
-    hipLaunchKernelGGL(gh_mortar_sides_kernel, dim3(plan.num_faces), dim3(128), lds, stream, el,
-                       plan.d_faces, plan.d_records, u, params, inv_jac, w.sides, w.speeds, full,
-                       half, plan.kf);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    const int rc = launch_gh_mortar_sides(plan, el, u, params, inv_jac, w.sides, w.speeds, stream);
+    if (rc != SXD_OK) return rc;
   }
   for (const MortarClass& c : plan.classes[gh ? 1 : 0]) {
     const void* kernel = gh ? reinterpret_cast<const void*>(&mortar_corrections_kernel<true>)

@@ -1,9 +1,9 @@
-"""The volume kernels of the GH adjoint at the edges of their routes, against
+"""The kernels of the GH adjoint at the edges of their routes, against
 the oracle's reverse-mode tape: elements whose 15 derivative adjoints per point
 still leave two workgroups per CU and ones where they do not (8 x 9 x 9, 10 x 9 x
 9), elements whose five fields exceed the LDS (16^3), the smallest and flat
 ones, several point rounds per thread, and ragged elements of both size
-classes."""
+classes, whose mortars reach the largest LDS (extents 12 and 13)."""
 import numpy as np
 import pytest
 import torch
@@ -45,7 +45,8 @@ def test_gh_adjoint_volume_edges(elements, extents):
     check(dg.Domain.from_brick(brick), u, gammas, inv, gbar, ref)
 
 
-@pytest.mark.parametrize("elements,lowest,highest", [((1, 1, 2), 2, 4), ((1, 2, 1), 8, 11)])
+@pytest.mark.parametrize("elements,lowest,highest", [((1, 1, 2), 2, 4), ((1, 2, 1), 8, 11),
+                                                     ((1, 1, 2), 12, 13)])
 def test_gh_adjoint_volume_ragged_edges(elements, lowest, highest):
     print(f"gh adjoint ragged {elements} {lowest}..{highest}", flush=True)
     brick, u, gammas, inv, _ = wl.gh_adjoint_workload_mixed(seed=5, elements=elements,
