@@ -584,6 +584,18 @@ int sxd_rk3_substep(int substep, int64_t n, double dt, const double* u0,
                     const double* uk, const double* lk, double* out,
                     void* stream);
 
+/* One Rk3HesthavenSsp step (three right-hand sides and substeps) of `system`
+ * on a domain without external faces, with its stage inputs:
+ *   u1 = u + dt L(u), u2 = 0.25 (3 u + u1 + dt L(u1)),
+ *   out = (1/3) (u + 2 u2 + 2 dt L(u2))
+ * out may be u, or NULL to stop after the stage inputs.  u, u1, u2 and the
+ * work array l are distinct fields, except that u2 may be l if the stage
+ * inputs are not needed (their contents are then unspecified).  params is gamma2
+ * (ScalarWave) or gammas (GH). */
+int sxd_rk3_step(const sxd_domain* domain, int system, double dt,
+                 const double* u, const double* params, const double* inv_jac,
+                 double* u1, double* u2, double* l, double* out, void* stream);
+
 /* ---- Adjoints (no counterpart in the reference) ------------------------- */
 
 /* Transpose of the ScalarWave DG RHS of sxd_scalar_wave_rhs, which is linear

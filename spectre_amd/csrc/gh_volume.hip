@@ -26,6 +26,7 @@
 #include "device_common.hpp"
 #include "gh_point.hpp"
 #include "kernels.hpp"
+#include "rk3.hpp"
 
 namespace sxd {
 namespace {
@@ -179,7 +180,7 @@ __host__ __device__ inline int pair_lds_doubles(int n0, int n1, int n2, bool fac
 // corrections are added before those of the internal faces.
 // RAGGED: with a table of lifted corrections (launch_ragged_gh_volume) those of
 // the faces a point lies on are added, each face's mortars in order.
-template <bool RAGGED, bool FACES>
+template <bool RAGGED, bool FACES, bool UPDATE>
 __global__ void __launch_bounds__(512)
 gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __restrict__ el,
                const int32_t* __restrict__ list, const int32_t* __restrict__ nbr,
@@ -187,7 +188,8 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
                const double* __restrict__ inv_jac, const double* __restrict__ state,
                const double* __restrict__ sides, const double* __restrict__ ghost,
                double* __restrict__ dt, const double* __restrict__ dtab,
-               const MortarCorrection* __restrict__ table, const double* __restrict__ corr) {
+               const MortarCorrection* __restrict__ table, const double* __restrict__ corr,
+               Rk3Update update) {
   extern __shared__ double s_lds[];
   int64_t e, off;
   int pr;
@@ -393,6 +395,21 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
         }
       }
     }
+    if constexpr (UPDATE) {
+      // the fields are read from the LDS once more: held in registers since the
+      // point-wise terms they would cost a wavefront per SIMD
+      asm volatile("" ::: "memory");
+      const PairFields uk = pair_fields(s_u + kPairStride * p);
+      const double h = rk3_step_size(update);
+      const double* u0 = update.u0 + 50 * off;
+      double first_u[5];
+#pragma unroll
+      for (int c = 0; c < 5; ++c)
+        first_u[c] = update.substep == 0 ? uk.v[c] : (u0 + comp[c] * np)[p];
+#pragma unroll
+      for (int c = 0; c < 5; ++c)
+        out[c] = rk3_value(update.substep, h, first_u[c], uk.v[c], out[c]);
+    }
     double* dte = dt + 50 * off;
 #pragma unroll
     for (int c = 0; c < 5; ++c) (dte + comp[c] * np)[p] = out[c];
@@ -452,22 +469,24 @@ bool gh_pairs_supported(const int32_t ext[3]) {
 
 int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* nbr,
                         const double* u, const double* gammas, const double* inv_jac, double* dt,
-                        double* work, const double* ghost, hipStream_t stream) {
+                        double* work, const double* ghost, hipStream_t stream,
+                        const Rk3Update& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   const int np = ext[0] * ext[1] * ext[2];
   const int64_t total = static_cast<int64_t>(num_elements) * np;
   const int lds = pair_lds_doubles(ext[0], ext[1], ext[2], true) * 8;
-  if (!allow_lds(reinterpret_cast<const void*>(&gh_pair_kernel<false, true>), lds))
-    return SXD_ERR_UNSUPPORTED;
+  const auto pair_kernel = up.substep < 0 ? &gh_pair_kernel<false, true, false>
+                                          : &gh_pair_kernel<false, true, true>;
+  if (!allow_lds(reinterpret_cast<const void*>(pair_kernel), lds)) return SXD_ERR_UNSUPPORTED;
   double* sides = work + kGhStateDoubles * total;
   hipLaunchKernelGGL(gh_state_kernel<false>, dim3(static_cast<unsigned>((total + 127) / 128)),
                      dim3(128), 0, stream, total, ext[0], ext[1], ext[2], nullptr, nullptr, u,
                      gammas, inv_jac, work, sides);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL((gh_pair_kernel<false, true>), dim3(10 * num_elements),
-                     dim3(pair_threads(np)), lds, stream, num_elements, ext[0], ext[1], ext[2],
-                     nullptr, nullptr, nbr, u, gammas, inv_jac, work, sides, ghost, dt, dtab, nullptr, nullptr);
+  hipLaunchKernelGGL(pair_kernel, dim3(10 * num_elements), dim3(pair_threads(np)), lds, stream, num_elements, ext[0], ext[1], ext[2],
+                     nullptr, nullptr, nbr, u, gammas, inv_jac, work, sides, ghost, dt, dtab, nullptr,
+                     nullptr, up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 
@@ -485,19 +504,20 @@ int launch_ragged_gh_volume(const std::vector<RaggedClass>& classes, const int32
                             const MixedElement* el, const double* u, const double* gammas,
                             const double* inv_jac, double* dt, const double* state,
                             const MortarCorrection* table, const double* corr,
-                            hipStream_t stream) {
+                            hipStream_t stream, const Rk3Update& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   if (state == nullptr) return SXD_ERR_INVALID_ARGUMENT;
-  const void* kernel = reinterpret_cast<const void*>(&gh_pair_kernel<true, false>);
+  const auto pair_kernel = up.substep < 0 ? &gh_pair_kernel<true, false, false>
+                                          : &gh_pair_kernel<true, false, true>;
   for (const RaggedClass& c : classes) {
     const int lds = (kPairStride * c.np_max + c.d_doubles) * 8;
-    if (!allow_lds(kernel, lds)) return SXD_ERR_UNSUPPORTED;
+    if (!allow_lds(reinterpret_cast<const void*>(pair_kernel), lds)) return SXD_ERR_UNSUPPORTED;
     const int blocks = (c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10;
-    hipLaunchKernelGGL((gh_pair_kernel<true, false>), dim3(blocks),
+    hipLaunchKernelGGL(pair_kernel, dim3(blocks),
                        dim3(c.np_max > 910 ? 512 : c.np_max > 128 ? 256 : 128), lds, stream,
                        c.count, 0, 0, 0, el, list + c.begin, nullptr, u, gammas, inv_jac, state,
-                       nullptr, nullptr, dt, dtab, table, corr);
+                       nullptr, nullptr, dt, dtab, table, corr, up);
     if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   }
   return SXD_OK;

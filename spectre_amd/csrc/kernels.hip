@@ -15,6 +15,7 @@
 #include "device_common.hpp"
 #include "gh_point.hpp"
 #include "kernels.hpp"
+#include "rk3.hpp"
 #include "sw_point.hpp"
 
 namespace sxd {
@@ -617,12 +618,12 @@ int launch_face_passes(bool gh, int num_elements, const int32_t ext[3], const in
 // its 15 derivatives from the LDS pencils, the volume terms, then the lifted
 // UpwindPenalty corrections of the faces it lies on (xi, eta, zeta order),
 // reading the neighbour's trace directly from HBM, and writes dt once.
-template <int N, bool GHOST>
+template <int N, bool GHOST, bool UPDATE>
 __global__ void __launch_bounds__((N * N * N + 63) / 64 * 64)
 sw_rhs_fused_kernel(const int32_t* __restrict__ nbr, const double* __restrict__ u,
                     const double* __restrict__ gamma2, const double* __restrict__ inv_jac,
                     double* __restrict__ dt, const double* __restrict__ dtab,
-                    const double* __restrict__ ghost, int bc_kind) {
+                    const double* __restrict__ ghost, int bc_kind, Rk3Update update) {
   constexpr int NP = N * N * N;
   __shared__ double s_u[5 * NP];
   const int64_t e = xcd_local_element(blockIdx.x, gridDim.x);
@@ -721,6 +722,7 @@ sw_rhs_fused_kernel(const int32_t* __restrict__ nbr, const double* __restrict__ 
 #pragma unroll
     for (int c = 0; c < 5; ++c) dtp[c] = dtp[c] + bc[c] * fac;
   }
+  if constexpr (UPDATE) rk3_apply<5>(dtp, update, up, (e * 5) * NP + t, NP);
 #pragma unroll
   for (int c = 0; c < 5; ++c) dt[(e * 5 + c) * NP + t] = dtp[c];
 }
@@ -748,14 +750,15 @@ template <int N>
 static int launch_sw_fused_n(int num_elements, const int32_t* nbr, const double* u,
                              const double* gamma2, const double* inv_jac, double* dt,
                              const double* dtab, const double* ghost, int bc_kind,
-                             hipStream_t stream) {
+                             hipStream_t stream, const Rk3Update& up) {
   constexpr int threads = (N * N * N + 63) / 64 * 64;
   if (ghost != nullptr || bc_kind != kSwBcGhostArray) {
-    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, true>), dim3(num_elements), dim3(threads), 0,
-                       stream, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind);
+    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, true, false>), dim3(num_elements), dim3(threads), 0,
+                       stream, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, up);
   } else {
-    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, false>), dim3(num_elements), dim3(threads), 0,
-                       stream, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind);
+    hipLaunchKernelGGL((up.substep < 0 ? &sw_rhs_fused_kernel<N, false, false>
+                                       : &sw_rhs_fused_kernel<N, false, true>),
+                       dim3(num_elements), dim3(threads), 0, stream, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, up);
   }
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
@@ -767,21 +770,21 @@ bool sw_fused_supported(const int32_t ext[3]) {
 int launch_sw_rhs(int num_elements, const int32_t ext[3], const int32_t* nbr,
                   const double* u, const double* gamma2, const double* inv_jac, double* dt,
                   bool fused, double* scratch_du, const double* ghost, int bc_kind,
-                  hipStream_t stream) {
+                  hipStream_t stream, const Rk3Update& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   if (fused) {
     if (!sw_fused_supported(ext)) return SXD_ERR_UNSUPPORTED;
     switch (ext[0]) {
-      case 2: return launch_sw_fused_n<2>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 3: return launch_sw_fused_n<3>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 4: return launch_sw_fused_n<4>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 5: return launch_sw_fused_n<5>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 6: return launch_sw_fused_n<6>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 7: return launch_sw_fused_n<7>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 8: return launch_sw_fused_n<8>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 9: return launch_sw_fused_n<9>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
-      case 10: return launch_sw_fused_n<10>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream);
+      case 2: return launch_sw_fused_n<2>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 3: return launch_sw_fused_n<3>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 4: return launch_sw_fused_n<4>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 5: return launch_sw_fused_n<5>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 6: return launch_sw_fused_n<6>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 7: return launch_sw_fused_n<7>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 8: return launch_sw_fused_n<8>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 9: return launch_sw_fused_n<9>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+      case 10: return launch_sw_fused_n<10>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
       default: return SXD_ERR_UNSUPPORTED;
     }
   }
@@ -899,51 +902,18 @@ int launch_gh_rhs_bjorhus(int num_elements, bool physical, const int32_t ext[3],
 // ---------------------------------------------------------------------------
 // Rk3HesthavenSsp::update_u (Time/TimeSteppers/Rk3HesthavenSsp.cpp:55-81).
 __global__ void __launch_bounds__(256)
-rk3_substep_kernel(int substep, int64_t n, double dt, const double* __restrict__ u0,
-                   const double* __restrict__ uk, const double* __restrict__ lk,
-                   double* __restrict__ out) {
+rk3_substep_kernel(int64_t n, Rk3Update up, const double* __restrict__ uk,
+                   const double* __restrict__ lk, double* __restrict__ out) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  if (substep == 0) {
-    out[i] = u0[i] + dt * lk[i];
-  } else if (substep == 1) {
-    out[i] = 0.25 * (3.0 * u0[i] + uk[i] + dt * lk[i]);
-  } else {
-    out[i] = (1.0 / 3.0) * (u0[i] + 2.0 * uk[i] + 2.0 * dt * lk[i]);
-  }
+  out[i] = rk3_value(up.substep, rk3_step_size(up), up.u0[i], uk[i], lk[i]);
 }
 
-// The same update with the step size read from device memory at run time
-// (for graphs that are replayed with changing step sizes).
-__global__ void __launch_bounds__(256)
-rk3_substep_dt_kernel(int substep, int64_t n, const double* __restrict__ dt_ptr,
-                      const double* __restrict__ u0, const double* __restrict__ uk,
-                      const double* __restrict__ lk, double* __restrict__ out) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double dt = *dt_ptr;
-  if (substep == 0) {
-    out[i] = u0[i] + dt * lk[i];
-  } else if (substep == 1) {
-    out[i] = 0.25 * (3.0 * u0[i] + uk[i] + dt * lk[i]);
-  } else {
-    out[i] = (1.0 / 3.0) * (u0[i] + 2.0 * uk[i] + 2.0 * dt * lk[i]);
-  }
-}
-
-int launch_rk3_substep_dt(int substep, int64_t n, const double* dt, const double* u0,
-                          const double* uk, const double* lk, double* out, hipStream_t stream) {
-  if (n == 0) return SXD_OK;
-  hipLaunchKernelGGL(rk3_substep_dt_kernel, dim3(static_cast<unsigned>((n + 255) / 256)),
-                     dim3(256), 0, stream, substep, n, dt, u0, uk, lk, out);
-  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
-}
-
-int launch_rk3_substep(int substep, int64_t n, double dt, const double* u0, const double* uk,
-                       const double* lk, double* out, hipStream_t stream) {
+int launch_rk3_substep(int64_t n, const Rk3Update& up, const double* uk, const double* lk,
+                       double* out, hipStream_t stream) {
   if (n == 0) return SXD_OK;
   hipLaunchKernelGGL(rk3_substep_kernel, dim3(static_cast<unsigned>((n + 255) / 256)),
-                     dim3(256), 0, stream, substep, n, dt, u0, uk, lk, out);
+                     dim3(256), 0, stream, n, up, uk, lk, out);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 

@@ -69,6 +69,16 @@ constexpr int kSwBcCpsrSommerfeld = 3, kSwBcCpsrFirstOrderBt = 4, kSwBcCpsrSecon
 // GH constraint-preserving Bjorhus (a time-derivative condition, no upwind
 // term on the external faces).
 constexpr int kGhBcBjorhus = 10;
+// A substep of Rk3HesthavenSsp applied where a kernel would store the time
+// derivative of its state uk: `dt` then receives the substep's result (it may
+// be u0, not uk).  substep < 0: none.  The step size is *dt_ptr, or dt if that
+// is null (graphs are replayed with changing step sizes).
+struct Rk3Update {
+  int substep = -1;
+  const double* u0 = nullptr;  // read for substeps 1 and 2 (substep 0: uk is u0)
+  double dt = 0.0;
+  const double* dt_ptr = nullptr;
+};
 // fused: one launch per RHS (requires sw_fused_supported); otherwise the
 // composite path, which needs scratch_du [E][15][Np].  Faces whose neighbour
 // index is negative take their exterior state by bc_kind: kSwBcGhostArray
@@ -78,7 +88,7 @@ constexpr int kGhBcBjorhus = 10;
 int launch_sw_rhs(int num_elements, const int32_t ext[3], const int32_t* nbr,
                   const double* u, const double* gamma2, const double* inv_jac, double* dt,
                   bool fused, double* scratch_du, const double* ghost, int bc_kind,
-                  hipStream_t stream);
+                  hipStream_t stream, const Rk3Update& up = {});  // up: fused, no external faces
 // ghost: as for launch_sw_rhs, with [E][50][Np].
 int launch_gh_rhs_composite(int num_elements, const int32_t ext[3], const int32_t* nbr,
                             const double* u, const double* gammas, const double* inv_jac,
@@ -95,7 +105,8 @@ bool gh_pairs_faster(int num_elements, const int32_t ext[3]);
 // ghost: as for launch_gh_rhs_composite.
 int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* nbr,
                         const double* u, const double* gammas, const double* inv_jac, double* dt,
-                        double* work, const double* ghost, hipStream_t stream);
+                        double* work, const double* ghost, hipStream_t stream,
+                        const Rk3Update& up = {});
 // Derivative engines of the fused GH kernel.
 constexpr int kGhFusedValu = 0;  // LDS pencils on the vector ALUs
 constexpr int kGhFusedMfma = 1;  // v_mfma_f64_16x16x4f64 tiles
@@ -150,11 +161,11 @@ int launch_ragged_gh_volume(const std::vector<RaggedClass>& classes, const int32
                             const MixedElement* el, const double* u, const double* gammas,
                             const double* inv_jac, double* dt, const double* state,
                             const MortarCorrection* table, const double* corr,
-                            hipStream_t stream);
+                            hipStream_t stream, const Rk3Update& up = {});
 int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
                             const MixedElement* el, const double* u, const double* gamma2,
                             const double* inv_jac, double* dt, const MortarCorrection* table,
-                            const double* corr, hipStream_t stream);
+                            const double* corr, hipStream_t stream, const Rk3Update& up = {});
 // The GH face corrections alone of launch_mixed_rhs, one launch per dimension,
 // for the faces that `phase` selects (kFacesAll, kFacesExternal with the ghost
 // state, kFacesInternal).
@@ -389,10 +400,8 @@ int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t*
                           double* scratch_faces, hipStream_t stream);
 int launch_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,
                                const double* a, double* mu, double* lam_out, hipStream_t stream);
-int launch_rk3_substep_dt(int substep, int64_t n, const double* dt, const double* u0,
-                          const double* uk, const double* lk, double* out, hipStream_t stream);
-int launch_rk3_substep(int substep, int64_t n, double dt, const double* u0, const double* uk,
-                       const double* lk, double* out, hipStream_t stream);
+int launch_rk3_substep(int64_t n, const Rk3Update& up, const double* uk, const double* lk,
+                       double* out, hipStream_t stream);
 // Flux systems (divergence.hip).  Strong (weak = false; jac = inverse
 // Jacobian) or weak (jac = det J times the inverse Jacobian) divergence of
 // fluxes [E][3 nc][Np] (block i + 3 c = F^i_c).  terms = false: out = div.

@@ -37,6 +37,7 @@
 #include "device_common.hpp"
 #include "gh_point.hpp"
 #include "kernels.hpp"
+#include "rk3.hpp"
 #include "sw_point.hpp"
 
 namespace sxd {
@@ -93,7 +94,7 @@ sw_ragged_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __re
                         const double* __restrict__ inv_jac, double* __restrict__ dt,
                         const double* __restrict__ dtab,
                         const MortarCorrection* __restrict__ table,
-                        const double* __restrict__ corr) {
+                        const double* __restrict__ corr, Rk3Update update) {
   extern __shared__ double s_lds[];
   const int e = list[blockIdx.x];
   const MixedElement m = el[e];
@@ -181,6 +182,7 @@ sw_ragged_volume_kernel(const MixedElement* __restrict__ el, const int32_t* __re
         }
       }
     }
+    if (update.substep >= 0) rk3_apply<5>(out, update, up, 5 * m.off + p, np);
 #pragma unroll
     for (int c = 0; c < 5; ++c) (dte + c * np)[p] = out[c];
   }
@@ -879,7 +881,7 @@ int mixed_face_lds_bytes(int kf, int km) { return FacePlan(kf, km, 13).total * 8
 int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32_t* list,
                             const MixedElement* el, const double* u, const double* gamma2,
                             const double* inv_jac, double* dt, const MortarCorrection* table,
-                            const double* corr, hipStream_t stream) {
+                            const double* corr, hipStream_t stream, const Rk3Update& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   // one launch for all sizes: a workgroup per element is too few for the
@@ -896,7 +898,7 @@ int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32
     return SXD_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(sw_ragged_volume_kernel, dim3(all.count),
                      dim3(all.np_max > 256 ? 512 : all.np_max > 128 ? 256 : 128), lds, stream, el,
-                     list + all.begin, u, gamma2, inv_jac, dt, dtab, table, corr);
+                     list + all.begin, u, gamma2, inv_jac, dt, dtab, table, corr, up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 

@@ -292,6 +292,14 @@ PYBIND11_MODULE(_Pybindings, m) {
     check(sxd_gh_rhs_adjoint(handle(h), a, b, c, g, o, current_stream(u)));
     return out;
   });
+  m.def("rk3_step", [](uintptr_t h, int system, double dt, py::object u, py::object params,
+                       py::object inv_jac, py::object u1, py::object u2, py::object l,
+                       py::object out) {
+    const double *a = SXD_CPTR(u), *b = SXD_CPTR(params), *c = SXD_CPTR(inv_jac);
+    double *s1 = SXD_PTR(u1), *s2 = SXD_PTR(u2), *w = SXD_PTR(l);
+    double* o = out.is_none() ? nullptr : SXD_PTR(out);
+    check(sxd_rk3_step(handle(h), system, dt, a, b, c, s1, s2, w, o, current_stream(u)));
+  });
   m.def("rk3_substep", [](int substep, double dt, py::object u0, py::object uk, py::object lk,
                           py::object out) {
     const int64_t n = out.attr("numel")().cast<int64_t>();

@@ -23,12 +23,10 @@ import torch
 
 from . import _Pybindings as _pyb
 from . import dg
+from ._lib import SYSTEMS as _SYSTEMS
 
 
-def _rhs(domain, system):
-    """RHS callable fn(u, params, inv_jac, out) of `system` on `domain`."""
-    call = _pyb.scalar_wave_rhs if system == "scalar_wave" else _pyb.gh_rhs
-    return lambda u, params, inv_jac, out: call(domain.handle, u, params, inv_jac, out)
+_SCALAR_WAVE, _GH = _SYSTEMS["scalar_wave"], _SYSTEMS["gh"]
 
 
 def _sw_rhs_adjoint(domain):
@@ -73,11 +71,10 @@ class ScalarWaveEvolution(torch.autograd.Function):
         u = u0.detach().clone()
         stage, l = torch.empty_like(u), torch.empty_like(u)
         checkpoints = []
-        rhs = _rhs(domain, "scalar_wave")
         for n in range(steps):
             if n % checkpoint_every == 0:
                 checkpoints.append(u.clone())
-            rk3_step(domain, rhs, u, gamma2, inv_jac, dt, stage, l)
+            _pyb.rk3_step(domain.handle, _SCALAR_WAVE, dt, u, gamma2, inv_jac, stage, l, l, u)
         ctx.domain, ctx.dt, ctx.steps = domain, dt, steps
         ctx.checkpoint_every, ctx.recompute = checkpoint_every, recompute
         ctx.checkpoints = checkpoints
@@ -100,8 +97,8 @@ class ScalarWaveEvolution(torch.autograd.Function):
                 states = []
                 for _ in range(first, last):
                     states.append(u.clone())
-                    rk3_step(domain, _rhs(domain, "scalar_wave"), u, gamma2, inv_jac, dt,
-                             stage, l)
+                    _pyb.rk3_step(domain.handle, _SCALAR_WAVE, dt, u, gamma2, inv_jac, stage, l,
+                                  l, u)
             for _ in range(last - first):
                 rk3_step_adjoint(_sw_rhs_adjoint(domain), lam3, gamma2, inv_jac, dt, a, lam, mu)
                 lam3, mu = mu, lam3
@@ -124,6 +121,15 @@ def rk3_step_states(rhs, u, params, inv_jac, dt, l, complete=True):
     return u0, u1, u2
 
 
+def _gh_step_stages(domain, u, gammas, inv_jac, dt, l, complete=True):
+    """rk3_step_states of the GH RHS on `domain`, the substeps applied by its
+    kernels."""
+    u0 = u.clone() if complete else u
+    u1, u2 = torch.empty_like(u), torch.empty_like(u)
+    _pyb.rk3_step(domain.handle, _GH, dt, u, gammas, inv_jac, u1, u2, l, u if complete else None)
+    return u0, u1, u2
+
+
 class GhEvolution(torch.autograd.Function):
     """u_final after `steps` RK3 steps of the GH DG RHS on `domain`.
 
@@ -143,14 +149,14 @@ class GhEvolution(torch.autograd.Function):
         l = torch.empty_like(u)
         checkpoints, last_stages = [], []
         last_first = (max(steps - 1, 0) // checkpoint_every) * checkpoint_every
-        rhs = _rhs(domain, "gh")
         for n in range(steps):
             if n % checkpoint_every == 0:
                 checkpoints.append(u.clone())
             if n >= last_first:
-                last_stages.append(rk3_step_states(rhs, u, gammas, inv_jac, dt, l))
+                last_stages.append(_gh_step_stages(domain, u, gammas, inv_jac, dt, l))
             else:
-                rk3_step(domain, rhs, u, gammas, inv_jac, dt, torch.empty_like(u), l)
+                _pyb.rk3_step(domain.handle, _GH, dt, u, gammas, inv_jac, torch.empty_like(u), l, l,
+                              u)
         ctx.domain, ctx.dt, ctx.steps, ctx.k = domain, dt, steps, checkpoint_every
         # overlap the recompute with the adjoint (see backward): on by default
         # for mixed-p domains; the uniform fused RHS kernel fills whole CUs
@@ -188,8 +194,7 @@ class GhEvolution(torch.autograd.Function):
                 l2 = torch.empty_like(u)
                 # the segment's last step is not completed: its result is
                 # the next checkpoint
-                stages = [rk3_step_states(_rhs(twin, "gh"), u, gammas, inv_jac, dt, l2,
-                                          complete=n < last - 1)
+                stages = [_gh_step_stages(twin, u, gammas, inv_jac, dt, l2, complete=n < last - 1)
                           for n in range(first, last)]
                 done = None
                 if side is not None:

@@ -1,0 +1,79 @@
+"""One RK3 step whose substeps the right-hand-side kernels apply themselves, in
+every kernel organisation that does so and in those that do not, against the
+oracle's right-hand sides and substeps: the same additions and products in the
+same order, so every value is equal."""
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as ol
+from spectre_amd import _Pybindings as pyb, dg, workloads as wl
+from spectre_amd._lib import SYSTEMS
+
+pytestmark = pytest.mark.gpu
+
+DT = 0.004
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float64)).cuda()
+
+
+def host(t):
+    return t.cpu().numpy()
+
+
+def check(domain, system, rhs, u, params, inv):
+    l0 = rhs(u)
+    u1 = ol.rk3_substep(0, DT, u, u, l0)
+    u2 = ol.rk3_substep(1, DT, u, u1, rhs(u1))
+    end = ol.rk3_substep(2, DT, u, u2, rhs(u2))
+    d_p, d_i = dev(params), dev(inv)
+    args = domain.handle, SYSTEMS[system], DT
+    for complete in (True, False):  # with the stage inputs kept
+        d_u = dev(u)
+        s1, s2, work, out = (torch.empty_like(d_u) for _ in range(4))
+        pyb.rk3_step(*args, d_u, d_p, d_i, s1, s2, work, out if complete else None)
+        assert np.array_equal(host(s1), u1) and np.array_equal(host(s2), u2)
+        assert np.array_equal(host(d_u), u)
+        if complete:
+            assert np.array_equal(host(out), end)
+    d_u = dev(u)  # in place, with one stage array and the work array
+    pyb.rk3_step(*args, d_u, d_p, d_i, s1, work, work, d_u)
+    assert np.array_equal(host(d_u), end)
+
+
+@pytest.mark.parametrize("n", [2, 6, 10])
+@pytest.mark.parametrize("kernel", ["fused", "composite"])
+def test_scalar_wave_step(n, kernel):
+    print(f"rk3 step scalar wave {n} {kernel}", flush=True)
+    brick, u, g2, inv = wl.scalar_wave_plane_wave_3d(seed=2, elements=(2, 1, 3), extents=(n, n, n))
+    domain = dg.Domain.from_brick(brick)
+    domain.set_kernel("scalar_wave", kernel)
+    check(domain, "scalar_wave", lambda v: ol.sw_rhs(brick.extents, brick.neighbors, v, g2, inv),
+          u, g2, inv)
+
+
+@pytest.mark.parametrize("n", [2, 6])
+@pytest.mark.parametrize("kernel", ["fused", "composite", "auto"])
+def test_gh_step(n, kernel):
+    print(f"rk3 step gh {n} {kernel}", flush=True)
+    brick, u, ga, inv = wl.gh_kerr_schild_brick(seed=5, elements=(2, 1, 2), extents=(n, n, n))
+    domain = dg.Domain.from_brick(brick)
+    domain.set_kernel("gh", kernel)
+    check(domain, "gh", lambda v: ol.gh_rhs(brick.extents, brick.neighbors, v, ga, inv), u, ga, inv)
+
+
+@pytest.mark.parametrize("kernel", ["auto", "mixed_batched"])
+def test_mixed_steps(kernel):
+    print(f"rk3 step mixed {kernel}", flush=True)
+    brick, u, g2, inv = wl.scalar_wave_plane_wave_mixed(seed=3, elements=(2, 1, 2))
+    domain = dg.MixedDomain.from_brick(brick)
+    domain.set_kernel("scalar_wave", kernel)
+    check(domain, "scalar_wave",
+          lambda v: ol.sw_rhs_mixed(brick.extents, brick.neighbors, v, g2, inv), u, g2, inv)
+    brick, u, ga, inv = wl.gh_kerr_schild_mixed(seed=4, elements=(1, 2, 1), lowest=3, highest=10)
+    domain = dg.MixedDomain.from_brick(brick)
+    domain.set_kernel("gh", kernel)
+    check(domain, "gh", lambda v: ol.gh_rhs_mixed(brick.extents, brick.neighbors, v, ga, inv),
+          u, ga, inv)
