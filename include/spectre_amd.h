@@ -612,9 +612,10 @@ int sxd_scalar_wave_rhs_adjoint(const sxd_domain* domain, const double* gbar,
  * 20480, e.g. 18^3): u, gbar,
  * ubar [E][50][Np]; mixed-p domains (sxd_domain_create_mixed): the ragged
  * layout.  ubar must not alias u or gbar.  Uses the domain's work arrays,
- * allocated on first use: 150 doubles per grid point, and on uniform domains
- * 300 doubles per element and point of its largest face.  No counterpart in
- * the reference (which has no adjoints). */
+ * allocated on first use: 30 doubles per grid point, and on uniform domains
+ * 300 doubles per element and point of its largest face, on mixed-p ones 172
+ * per face point and 4 per mortar point.  No counterpart in the reference
+ * (which has no adjoints). */
 int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u,
                        const double* gammas, const double* inv_jac,
                        const double* gbar, double* ubar, void* stream);
@@ -628,6 +629,17 @@ int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u,
 int sxd_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,
                             const double* a, double* mu, double* lam_out,
                             void* stream);
+/* The transpose of one RK3 step (sxd_rk3_step): three adjoint right-hand sides
+ * with their transposed substeps.  lam3 is the adjoint of the step's result;
+ * mu receives that of its input.  GH: u, u1, u2 are the step's stage inputs, at
+ * which the RHS is linearised; ScalarWave (linear): they are not read and may
+ * be NULL.  a and lam are work arrays of a field each; lam3, a, lam and mu are
+ * distinct.  Domains as sxd_scalar_wave_rhs_adjoint and sxd_gh_rhs_adjoint. */
+int sxd_rk3_step_adjoint(const sxd_domain* domain, int system, double dt,
+                         const double* u, const double* u1, const double* u2,
+                         const double* params, const double* inv_jac,
+                         const double* lam3, double* a, double* lam, double* mu,
+                         void* stream);
 
 /* A full Rk3HesthavenSsp step (three right-hand sides and three update_u
  * substeps, Time/TimeSteppers/Rk3HesthavenSsp.cpp:55-81) of `system` on

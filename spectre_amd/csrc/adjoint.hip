@@ -27,16 +27,18 @@
 #include "device_common.hpp"
 #include "gh_adjoint.hpp"
 #include "kernels.hpp"
+#include "rk3.hpp"
 #include "sw_point.hpp"
 
 namespace sxd {
 namespace {
 
-template <int N>
+template <int N, bool UPDATE>
 __global__ void __launch_bounds__((N * N * N + 63) / 64 * 64)
 sw_rhs_adjoint_kernel(const int32_t* __restrict__ nbr, const double* __restrict__ gbar,
                       const double* __restrict__ gamma2, const double* __restrict__ inv_jac,
-                      double* __restrict__ ubar, const double* __restrict__ dtab) {
+                      double* __restrict__ ubar, const double* __restrict__ dtab,
+                      Rk3AdjointUpdate update) {
   constexpr int NP = N * N * N;
   __shared__ double s_x[15 * NP];  // logical-derivative adjoints [c][j][p]
   const int64_t e = xcd_local_element(blockIdx.x, gridDim.x);
@@ -178,6 +180,13 @@ sw_rhs_adjoint_kernel(const int32_t* __restrict__ nbr, const double* __restrict_
       for (int i = 0; i < 3; ++i) ub[2 + i] = ub[2 + i] + ne[i] * s_ex;
     }
   }
+  if constexpr (UPDATE) {
+#pragma unroll
+    for (int c = 0; c < 5; ++c)
+      ub[c] = rk3_adjoint_value(update.substep, update.dt, gp[c], ub[c],
+                                update.mu + (e * 5 + c) * NP + t);
+    if (update.substep == 0) return;
+  }
 #pragma unroll
   for (int c = 0; c < 5; ++c) ubar[(e * 5 + c) * NP + t] = ub[c];
 }
@@ -185,10 +194,12 @@ sw_rhs_adjoint_kernel(const int32_t* __restrict__ nbr, const double* __restrict_
 template <int N>
 int launch_sw_adjoint_n(int num_elements, const int32_t* nbr, const double* gbar,
                         const double* gamma2, const double* inv_jac, double* ubar,
-                        const double* dtab, hipStream_t stream) {
+                        const double* dtab, hipStream_t stream, const Rk3AdjointUpdate& up) {
   constexpr int threads = (N * N * N + 63) / 64 * 64;
-  hipLaunchKernelGGL(sw_rhs_adjoint_kernel<N>, dim3(num_elements), dim3(threads), 0, stream,
-                     nbr, gbar, gamma2, inv_jac, ubar, dtab);
+  hipLaunchKernelGGL((up.substep < 0 ? &sw_rhs_adjoint_kernel<N, false>
+                                     : &sw_rhs_adjoint_kernel<N, true>),
+                     dim3(num_elements), dim3(threads), 0, stream, nbr, gbar, gamma2, inv_jac,
+                     ubar, dtab, up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 
@@ -204,16 +215,8 @@ rk3_adjoint_substep_kernel(int substep, int64_t n, double dt, const double* lam,
                            double* lam_out) {  // lam_out may be lam (element-wise in place)
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const double l = lam[i];
-  if (substep == 2) {
-    lam_out[i] = (2.0 / 3.0) * (l + dt * a[i]);
-    mu[i] = (1.0 / 3.0) * l;
-  } else if (substep == 1) {
-    lam_out[i] = 0.25 * (l + dt * a[i]);
-    mu[i] = mu[i] + 0.75 * l;
-  } else {
-    mu[i] = mu[i] + (l + dt * a[i]);
-  }
+  const double out = rk3_adjoint_value(substep, dt, lam[i], a[i], mu + i);
+  if (substep > 0) lam_out[i] = out;
 }
 
 // ---------------------------------------------------------------------------
@@ -277,14 +280,15 @@ bool sw_adjoint_supported(const int32_t ext[3]) {
 
 int launch_sw_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t* nbr,
                           const double* gbar, const double* gamma2, const double* inv_jac,
-                          double* ubar, hipStream_t stream) {
+                          double* ubar, hipStream_t stream, const Rk3AdjointUpdate& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   if (!sw_adjoint_supported(ext)) return SXD_ERR_UNSUPPORTED;
   switch (ext[0]) {
 #define SXD_ADJ_CASE(n) \
   case n:               \
-    return launch_sw_adjoint_n<n>(num_elements, nbr, gbar, gamma2, inv_jac, ubar, dtab, stream);
+    return launch_sw_adjoint_n<n>(num_elements, nbr, gbar, gamma2, inv_jac, ubar, dtab, stream, \
+                                  up);
     SXD_ADJ_CASE(2)
     SXD_ADJ_CASE(3)
     SXD_ADJ_CASE(4)
@@ -306,7 +310,8 @@ int gh_adjoint_face_slots(const int32_t ext[3]) {
 int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t* nbr,
                           const double* u, const double* gammas, const double* inv_jac,
                           const double* gbar, double* ubar, double* work,
-                          double* scratch_faces, hipStream_t stream) {
+                          double* scratch_faces, hipStream_t stream,
+                          const Rk3AdjointUpdate& up) {
   if (!gh_adjoint_supported(ext)) return SXD_ERR_UNSUPPORTED;
   const int rc = launch_gh_adjoint_points(num_elements, ext, u, gammas, inv_jac, gbar, ubar,
                                           work, stream);
@@ -318,7 +323,7 @@ int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t*
                      inv_jac, gbar, scratch_faces);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
   return launch_gh_adjoint_sweeps(num_elements, ext, gammas, inv_jac, gbar, work, ubar,
-                                  scratch_faces, F, stream);
+                                  scratch_faces, F, stream, up);
 }
 
 int launch_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,

@@ -1665,6 +1665,11 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
 
 // ---- adjoints ------------------------------------------------------------------
 
+namespace {
+constexpr char kSwAdjointDomains[] =
+    "the ScalarWave adjoint needs a uniform domain with isotropic extents 2..10";
+}  // namespace
+
 int sxd_scalar_wave_rhs_adjoint(const sxd_domain* domain, const double* gbar, const double* gamma2,
                                 const double* inv_jac, double* ubar, void* stream) {
   if (int rc = check_periodic(domain); rc != SXD_OK) return rc;
@@ -1673,8 +1678,7 @@ int sxd_scalar_wave_rhs_adjoint(const sxd_domain* domain, const double* gbar, co
   SXD_REQUIRE_DEVICE(inv_jac);
   SXD_REQUIRE_DEVICE(ubar);
   if (domain->mixed || !sw_adjoint_supported(domain->ext))
-    return fail(SXD_ERR_UNSUPPORTED, "the ScalarWave adjoint needs a uniform domain with "
-                                     "isotropic extents 2..10");
+    return fail(SXD_ERR_UNSUPPORTED, "%s", kSwAdjointDomains);
   if (gbar == ubar) return fail(SXD_ERR_INVALID_ARGUMENT, "gbar and ubar must not alias");
   return finish(launch_sw_rhs_adjoint(domain->num_elements, domain->ext, domain->d_nbr, gbar,
                                       gamma2, inv_jac, ubar, static_cast<hipStream_t>(stream)),
@@ -1720,7 +1724,7 @@ namespace {
 // add the contributions.
 int run_gh_adjoint_mixed(sxd_domain* d, Scratch& sc, const double* u, const double* gammas,
                          const double* inv_jac, const double* gbar, double* ubar,
-                         hipStream_t stream) {
+                         hipStream_t stream, const Rk3AdjointUpdate& up) {
   if (!d->conforming_plan || mixed_face_adjoint_lds_bytes(d->kf, d->km) > 160 * 1024 ||
       (kStagedDiffDoubles + 3 * d->np_max) * 8 > 160 * 1024)
     return SXD_ERR_UNSUPPORTED;
@@ -1736,8 +1740,21 @@ int run_gh_adjoint_mixed(sxd_domain* d, Scratch& sc, const double* u, const doub
                                          stream);
   if (rc == SXD_OK)
     rc = launch_ragged_gh_adjoint_sweeps(d->classes, d->d_list, d->d_el, gammas, inv_jac, gbar,
-                                         work, ubar, d->plan.d_corrections, w.contrib, stream);
+                                         work, ubar, d->plan.d_corrections, w.contrib, stream,
+                                         up);
   return rc;
+}
+int run_gh_adjoint(sxd_domain* d, Scratch& sc, const double* u, const double* gammas,
+                   const double* inv_jac, const double* gbar, double* ubar, hipStream_t stream,
+                   const Rk3AdjointUpdate& up = {}) {
+  if (d->mixed) return run_gh_adjoint_mixed(d, sc, u, gammas, inv_jac, gbar, ubar, stream, up);
+  const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];
+  const size_t volume = kGhAdjointDoubles * np * d->num_elements;
+  const size_t faces = 300 * static_cast<size_t>(gh_adjoint_face_slots(d->ext)) * d->num_elements;
+  if (int rc = sc.reserve_block(kAdjointBlock, volume + faces); rc != SXD_OK) return rc;
+  double* work = sc.block[kAdjointBlock];
+  return launch_gh_rhs_adjoint(d->num_elements, d->ext, d->d_nbr, u, gammas, inv_jac, gbar, ubar,
+                               work, work + volume, stream, up);
 }
 }  // namespace
 
@@ -1755,20 +1772,57 @@ int sxd_gh_rhs_adjoint(const sxd_domain* domain, const double* u, const double* 
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
   std::lock_guard<std::mutex> enqueue(sc.enqueue);
-  if (d->mixed)
-    return finish(run_gh_adjoint_mixed(d, sc, u, gammas, inv_jac, gbar, ubar,
-                                       static_cast<hipStream_t>(stream)),
-                  __func__);
-  const size_t np = static_cast<size_t>(d->ext[0]) * d->ext[1] * d->ext[2];
-  const size_t volume = kGhAdjointDoubles * np * d->num_elements;
-  const size_t faces = 300 * static_cast<size_t>(gh_adjoint_face_slots(d->ext)) * d->num_elements;
-  if (int rc = sc.reserve_block(kAdjointBlock, volume + faces); rc != SXD_OK)
-    return finish(rc, __func__);
-  double* work = sc.block[kAdjointBlock];
-  return finish(launch_gh_rhs_adjoint(d->num_elements, d->ext, d->d_nbr, u, gammas, inv_jac, gbar,
-                                      ubar, work, work + volume,
-                                      static_cast<hipStream_t>(stream)),
+  return finish(run_gh_adjoint(d, sc, u, gammas, inv_jac, gbar, ubar,
+                               static_cast<hipStream_t>(stream)),
                 __func__);
+}
+
+int sxd_rk3_step_adjoint(const sxd_domain* domain, int system, double dt, const double* u,
+                         const double* u1, const double* u2, const double* params,
+                         const double* inv_jac, const double* lam3, double* a, double* lam,
+                         double* mu, void* stream) {
+  if (int rc = check_periodic(domain); rc != SXD_OK) return rc;
+  if (system != SXD_SYSTEM_SCALAR_WAVE && system != SXD_SYSTEM_GH)
+    return fail(SXD_ERR_INVALID_ARGUMENT, "unknown system %d", system);
+  const bool gh = system == SXD_SYSTEM_GH;
+  if (gh) {
+    SXD_REQUIRE_DEVICE(u);
+    SXD_REQUIRE_DEVICE(u1);
+    SXD_REQUIRE_DEVICE(u2);
+  }
+  SXD_REQUIRE_DEVICE(params);
+  SXD_REQUIRE_DEVICE(inv_jac);
+  SXD_REQUIRE_DEVICE(lam3);
+  SXD_REQUIRE_DEVICE(a);
+  SXD_REQUIRE_DEVICE(lam);
+  SXD_REQUIRE_DEVICE(mu);
+  if (gh && domain->mortars)
+    return fail(SXD_ERR_UNSUPPORTED, "%s: not built for mortar domains", __func__);
+  if (!gh && (domain->mixed || !sw_adjoint_supported(domain->ext)))
+    return fail(SXD_ERR_UNSUPPORTED, "%s", kSwAdjointDomains);
+  sxd_domain* d = const_cast<sxd_domain*>(domain);
+  const double* field[7] = {lam3, a, lam, mu, u, u1, u2};
+  for (int i = 0; i < 4; ++i)
+    for (int j = i + 1; j < (gh ? 7 : 4); ++j)
+      if (int rc = check_no_overlap(d, gh ? 50 : 5, field[i], field[j], __func__); rc != SXD_OK)
+        return rc;
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  Scratch& sc = stream_scratch(d, s);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
+  const double* states[3] = {u, u1, u2};
+  const double* from[3] = {a, lam, lam3};
+  double* to[3] = {lam, a, lam};  // after substep 0: the GH kernels' intermediate
+  Rk3AdjointUpdate up;
+  up.dt = dt;
+  up.mu = mu;
+  for (up.substep = 2; up.substep >= 0; --up.substep) {
+    const int k = up.substep;
+    const int rc = gh ? run_gh_adjoint(d, sc, states[k], params, inv_jac, from[k], to[k], s, up)
+                      : launch_sw_rhs_adjoint(d->num_elements, d->ext, d->d_nbr, from[k], params,
+                                              inv_jac, to[k], s, up);
+    if (rc != SXD_OK) return finish(rc, __func__);
+  }
+  return ok();
 }
 
 int sxd_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,

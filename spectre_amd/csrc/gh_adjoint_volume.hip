@@ -23,6 +23,7 @@
 #include "device_common.hpp"
 #include "gh_adjoint.hpp"
 #include "kernels.hpp"
+#include "rk3.hpp"
 
 namespace sxd {
 namespace {
@@ -222,14 +223,15 @@ gh_adjoint_point_kernel(int64_t total, int np_uniform, const MixedElement* __res
 // leave fewer than two workgroups per CU).  Dynamic LDS: 3 S Np doubles, then
 // the D matrices.  contrib: face terms, [E][6][50][F] (uniform domains) or per
 // record as `table` places them.
-template <bool RAGGED, int S>
+template <bool RAGGED, int S, bool UPDATE>
 __global__ void __launch_bounds__(512)
 gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* __restrict__ el,
                          const int32_t* __restrict__ list, const double* __restrict__ gammas,
                          const double* __restrict__ inv_jac, const double* __restrict__ gbar,
                          const double* __restrict__ work, double* __restrict__ ubar,
                          const double* __restrict__ dtab, const double* __restrict__ contrib,
-                         int F, const MortarCorrection* __restrict__ table) {
+                         int F, const MortarCorrection* __restrict__ table,
+                         Rk3AdjointUpdate update) {
   extern __shared__ double s_lds[];
   int64_t at;
   int pr;
@@ -326,6 +328,14 @@ gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* 
             for (int c = 0; c < S; ++c) acc[c] += from[comp[c0 + c] * nf];
         }
       }
+      if constexpr (UPDATE) {
+        double* mu = update.mu + 50 * m.off;
+#pragma unroll
+        for (int c = 0; c < S; ++c)
+          acc[c] = rk3_adjoint_value(update.substep, update.dt, (ge + comp[c0 + c] * np)[p],
+                                     acc[c], mu + comp[c0 + c] * np + p);
+        if (update.substep == 0) continue;
+      }
 #pragma unroll
       for (int c = 0; c < S; ++c) (ube + comp[c0 + c] * np)[p] = acc[c];
     }
@@ -374,23 +384,20 @@ int launch_sweeps(int count, int np, int d_doubles, const int32_t ext[3], const 
                   const int32_t* list, const double* gammas, const double* inv_jac,
                   const double* gbar, const double* work, double* ubar, const double* dtab,
                   const double* contrib, int F, const MortarCorrection* table,
-                  hipStream_t stream) {
+                  hipStream_t stream, const Rk3AdjointUpdate& up) {
   const bool five = 2 * (15 * np + d_doubles) <= kLdsDoubles;
   const int lds = ((five ? 15 : 3) * np + d_doubles) * 8;
-  const void* kernel = five
-                           ? reinterpret_cast<const void*>(&gh_adjoint_sweeps_kernel<RAGGED, 5>)
-                           : reinterpret_cast<const void*>(&gh_adjoint_sweeps_kernel<RAGGED, 1>);
-  if (!allow_lds(kernel, lds)) return SXD_ERR_UNSUPPORTED;
+  const bool update = up.substep >= 0;
+  const auto kernel = five ? (update ? &gh_adjoint_sweeps_kernel<RAGGED, 5, true>
+                                     : &gh_adjoint_sweeps_kernel<RAGGED, 5, false>)
+                           : (update ? &gh_adjoint_sweeps_kernel<RAGGED, 1, true>
+                                     : &gh_adjoint_sweeps_kernel<RAGGED, 1, false>);
+  if (!allow_lds(reinterpret_cast<const void*>(kernel), lds)) return SXD_ERR_UNSUPPORTED;
   const int blocks = RAGGED ? (count + kNumXcds - 1) / kNumXcds * kNumXcds * 10 : 10 * count;
   const int threads = np > 512 ? 512 : np > 128 ? 256 : 128;
-  if (five)
-    hipLaunchKernelGGL((gh_adjoint_sweeps_kernel<RAGGED, 5>), dim3(blocks), dim3(threads), lds,
-                       stream, count, ext[0], ext[1], ext[2], el, list, gammas, inv_jac, gbar,
-                       work, ubar, dtab, contrib, F, table);
-  else
-    hipLaunchKernelGGL((gh_adjoint_sweeps_kernel<RAGGED, 1>), dim3(blocks), dim3(threads), lds,
-                       stream, count, ext[0], ext[1], ext[2], el, list, gammas, inv_jac, gbar,
-                       work, ubar, dtab, contrib, F, table);
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), lds, stream, count, ext[0], ext[1],
+                     ext[2], el, list, gammas, inv_jac, gbar, work, ubar, dtab, contrib, F, table,
+                     up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 }  // namespace
@@ -415,13 +422,14 @@ int launch_gh_adjoint_points(int num_elements, const int32_t ext[3], const doubl
 
 int launch_gh_adjoint_sweeps(int num_elements, const int32_t ext[3], const double* gammas,
                              const double* inv_jac, const double* gbar, const double* work,
-                             double* ubar, const double* contrib, int F, hipStream_t stream) {
+                             double* ubar, const double* contrib, int F, hipStream_t stream,
+                             const Rk3AdjointUpdate& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   const int np = ext[0] * ext[1] * ext[2];
   const int d_doubles = ext[0] * ext[0] + ext[1] * ext[1] + ext[2] * ext[2];
   return launch_sweeps<false>(num_elements, np, d_doubles, ext, nullptr, nullptr, gammas, inv_jac,
-                              gbar, work, ubar, dtab, contrib, F, nullptr, stream);
+                              gbar, work, ubar, dtab, contrib, F, nullptr, stream, up);
 }
 
 int launch_ragged_gh_adjoint_points(const std::vector<RaggedClass>& classes, const int32_t* list,
@@ -448,14 +456,14 @@ int launch_ragged_gh_adjoint_sweeps(const std::vector<RaggedClass>& classes, con
                                     const double* inv_jac, const double* gbar,
                                     const double* work, double* ubar,
                                     const MortarCorrection* table, const double* contrib,
-                                    hipStream_t stream) {
+                                    hipStream_t stream, const Rk3AdjointUpdate& up) {
   const double* dtab = device_diff_matrices();
   if (dtab == nullptr) return SXD_ERR_DEVICE;
   const int32_t none[3] = {0, 0, 0};
   for (const RaggedClass& c : classes) {
     const int rc = launch_sweeps<true>(c.count, c.np_max, c.d_doubles, none, el, list + c.begin,
                                        gammas, inv_jac, gbar, work, ubar, dtab, contrib, 0, table,
-                                       stream);
+                                       stream, up);
     if (rc != SXD_OK) return rc;
   }
   return SXD_OK;

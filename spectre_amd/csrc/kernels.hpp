@@ -79,6 +79,15 @@ struct Rk3Update {
   double dt = 0.0;
   const double* dt_ptr = nullptr;
 };
+// The transposed substep (sxd_rk3_adjoint_substep) applied where an adjoint
+// kernel would store ubar = A^T lam for gbar = lam: `ubar` then receives
+// lam_out (not lam; after substep 0 its contents are unspecified), and mu is
+// updated.  substep < 0: none.
+struct Rk3AdjointUpdate {
+  int substep = -1;
+  double dt = 0.0;
+  double* mu = nullptr;
+};
 // fused: one launch per RHS (requires sw_fused_supported); otherwise the
 // composite path, which needs scratch_du [E][15][Np].  Faces whose neighbour
 // index is negative take their exterior state by bc_kind: kSwBcGhostArray
@@ -367,7 +376,8 @@ int launch_gh_adjoint_points(int num_elements, const int32_t ext[3], const doubl
                              double* ubar, double* work, hipStream_t stream);
 int launch_gh_adjoint_sweeps(int num_elements, const int32_t ext[3], const double* gammas,
                              const double* inv_jac, const double* gbar, const double* work,
-                             double* ubar, const double* contrib, int F, hipStream_t stream);
+                             double* ubar, const double* contrib, int F, hipStream_t stream,
+                             const Rk3AdjointUpdate& up = {});
 // The same on a ragged domain, in two steps (point_el: the element of each of the
 // total_points grid points); table, contrib: launch_gh_adjoint_faces' work.
 int launch_ragged_gh_adjoint_points(const std::vector<RaggedClass>& classes, const int32_t* list,
@@ -380,7 +390,7 @@ int launch_ragged_gh_adjoint_sweeps(const std::vector<RaggedClass>& classes, con
                                     const double* inv_jac, const double* gbar,
                                     const double* work, double* ubar,
                                     const MortarCorrection* table, const double* contrib,
-                                    hipStream_t stream);
+                                    hipStream_t stream, const Rk3AdjointUpdate& up = {});
 // Largest LDS of the face kernel the mixed-p adjoint's size limit stems from.
 int mixed_face_adjoint_lds_bytes(int kf, int km);
 // Adjoint (transpose) of the ScalarWave RHS on a uniform domain (isotropic
@@ -388,7 +398,7 @@ int mixed_face_adjoint_lds_bytes(int kf, int km);
 bool sw_adjoint_supported(const int32_t ext[3]);
 int launch_sw_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t* nbr,
                           const double* gbar, const double* gamma2, const double* inv_jac,
-                          double* ubar, hipStream_t stream);
+                          double* ubar, hipStream_t stream, const Rk3AdjointUpdate& up = {});
 // Adjoint of the GH RHS linearised at u (uniform extents with
 // 3 Np + N0^2 + N1^2 + N2^2 <= 20480):
 // ubar = (d dt / d u)^T gbar; work: kGhAdjointDoubles x E x Np doubles;
@@ -397,7 +407,8 @@ int gh_adjoint_face_slots(const int32_t ext[3]);
 int launch_gh_rhs_adjoint(int num_elements, const int32_t ext[3], const int32_t* nbr,
                           const double* u, const double* gammas, const double* inv_jac,
                           const double* gbar, double* ubar, double* work,
-                          double* scratch_faces, hipStream_t stream);
+                          double* scratch_faces, hipStream_t stream,
+                          const Rk3AdjointUpdate& up = {});
 int launch_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam,
                                const double* a, double* mu, double* lam_out, hipStream_t stream);
 int launch_rk3_substep(int64_t n, const Rk3Update& up, const double* uk, const double* lk,

@@ -308,6 +308,16 @@ PYBIND11_MODULE(_Pybindings, m) {
     check(sxd_rk3_substep(substep, n, dt, a, b, c, o, current_stream(out)));
     return out;
   });
+  m.def("rk3_step_adjoint", [](uintptr_t h, int system, double dt, py::object u, py::object u1,
+                               py::object u2, py::object params, py::object inv_jac,
+                               py::object lam3, py::object a, py::object lam, py::object mu) {
+    auto state = [](py::object t) { return t.is_none() ? nullptr : SXD_CPTR(t); };
+    const double *s0 = state(u), *s1 = state(u1), *s2 = state(u2);
+    const double *b = SXD_CPTR(params), *c = SXD_CPTR(inv_jac), *l3 = SXD_CPTR(lam3);
+    double *w = SXD_PTR(a), *l = SXD_PTR(lam), *o = SXD_PTR(mu);
+    check(sxd_rk3_step_adjoint(handle(h), system, dt, s0, s1, s2, b, c, l3, w, l, o,
+                               current_stream(lam3)));
+  });
   m.def("rk3_adjoint_substep", [](int substep, double dt, py::object lam, py::object a,
                                   py::object mu, py::object lam_out) {
     const int64_t n = lam.attr("numel")().cast<int64_t>();

@@ -15,8 +15,8 @@ Reference: Time/TimeSteppers/Rk3HesthavenSsp.cpp:55-81 (the forward step);
 the reference has no adjoint.
 
 Every device call of these Functions goes through the pybind11 module
-spectre_amd._Pybindings (the right-hand sides, their adjoints and the RK3
-substeps on the domain's handle), which calls the C ABI.
+spectre_amd._Pybindings (RK3 steps and their adjoints on the domain's handle),
+which calls the C ABI.
 """
 import numpy as np
 import torch
@@ -27,11 +27,6 @@ from ._lib import SYSTEMS as _SYSTEMS
 
 
 _SCALAR_WAVE, _GH = _SYSTEMS["scalar_wave"], _SYSTEMS["gh"]
-
-
-def _sw_rhs_adjoint(domain):
-    return lambda gbar, gamma2, inv_jac, out: _pyb.scalar_wave_rhs_adjoint(
-        domain.handle, gbar, gamma2, inv_jac, out)
 
 
 def rk3_adjoint_substep(substep, dt, lam, a, mu, lam_out=None):
@@ -100,7 +95,8 @@ class ScalarWaveEvolution(torch.autograd.Function):
                     _pyb.rk3_step(domain.handle, _SCALAR_WAVE, dt, u, gamma2, inv_jac, stage, l,
                                   l, u)
             for _ in range(last - first):
-                rk3_step_adjoint(_sw_rhs_adjoint(domain), lam3, gamma2, inv_jac, dt, a, lam, mu)
+                _pyb.rk3_step_adjoint(domain.handle, _SCALAR_WAVE, dt, None, None, None, gamma2,
+                                      inv_jac, lam3, a, lam, mu)
                 lam3, mu = mu, lam3
         ctx.checkpoints = None
         return lam3, None, None, None, None, None, None, None
@@ -214,14 +210,9 @@ class GhEvolution(torch.autograd.Function):
                         for t in st:
                             t.record_stream(main)
                 pending = recompute(seg - 1) if seg > 0 and side is not None else None
-            h = domain.handle
             for s0, s1, s2 in reversed(stages):
-                _pyb.gh_rhs_adjoint(h, s2, gammas, inv_jac, lam3, a)
-                rk3_adjoint_substep(2, dt, lam3, a, mu, lam)
-                _pyb.gh_rhs_adjoint(h, s1, gammas, inv_jac, lam, a)
-                rk3_adjoint_substep(1, dt, lam, a, mu, lam)
-                _pyb.gh_rhs_adjoint(h, s0, gammas, inv_jac, lam, a)
-                rk3_adjoint_substep(0, dt, lam, a, mu, None)
+                _pyb.rk3_step_adjoint(domain.handle, _GH, dt, s0, s1, s2, gammas, inv_jac, lam3, a,
+                                      lam, mu)
                 lam3, mu = mu, lam3
         ctx.checkpoints = ctx.last_stages = None
         return lam3, None, None, None, None, None, None, None

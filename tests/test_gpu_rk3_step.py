@@ -77,3 +77,65 @@ def test_mixed_steps(kernel):
     domain.set_kernel("gh", kernel)
     check(domain, "gh", lambda v: ol.gh_rhs_mixed(brick.extents, brick.neighbors, v, ga, inv),
           u, ga, inv)
+
+
+def step_adjoint(adjoint, lam3):
+    """mu of one transposed step; adjoint(k, lam) = A^T lam at stage input k."""
+    lam = (2.0 / 3.0) * (lam3 + DT * adjoint(2, lam3))
+    mu = (1.0 / 3.0) * lam3 + 0.75 * lam
+    lam = 0.25 * (lam + DT * adjoint(1, lam))
+    return mu + (lam + DT * adjoint(0, lam))
+
+
+def run_adjoint(domain, system, states, params, inv, lam3):
+    d_lam3 = dev(lam3)
+    a, lam, mu = (torch.full_like(d_lam3, float("nan")) for _ in range(3))
+    s = [None if t is None else dev(t) for t in states]
+    pyb.rk3_step_adjoint(domain.handle, SYSTEMS[system], DT, *s, dev(params), dev(inv), d_lam3, a,
+                         lam, mu)
+    assert np.array_equal(host(d_lam3), lam3)
+    return host(mu)
+
+
+@pytest.mark.parametrize("n", [2, 6, 10])
+def test_scalar_wave_step_adjoint(n):
+    print(f"rk3 step adjoint scalar wave {n}", flush=True)
+    brick, u, g2, inv = wl.scalar_wave_plane_wave_3d(seed=2, elements=(2, 1, 3), extents=(n, n, n))
+    lam3 = np.random.default_rng(3).standard_normal(u.shape)
+    ref = step_adjoint(lambda k, lam: ol.sw_rhs_adjoint(brick.extents, brick.neighbors, lam, g2,
+                                                        inv), lam3)
+    got = run_adjoint(dg.Domain.from_brick(brick), "scalar_wave", [None] * 3, g2, inv, lam3)
+    assert np.array_equal(got, ref)
+
+
+# the GH kernels add the adjoint's terms in another order than the tape, to
+# 1e-12 of the largest value per right-hand side; the three of a step add up,
+# each with a factor dt times an adjoint of norm ~ 1 / dt
+GH_TOL = 3e-12
+
+
+@pytest.mark.parametrize("extents", [(2, 2, 2), (8, 9, 9), (10, 9, 9)])
+def test_gh_step_adjoint(extents):
+    print(f"rk3 step adjoint gh {extents}", flush=True)
+    brick, u, ga, inv, _ = wl.gh_adjoint_workload(seed=1, elements=(1, 1, 2), extents=extents,
+                                                  noise=1e-3)
+    rng = np.random.default_rng(4)
+    states = [u * (1.0 + 1e-3 * rng.standard_normal(u.shape)) for _ in range(3)]
+    lam3 = rng.standard_normal(u.shape)
+    ref = step_adjoint(lambda k, lam: ol.gh_rhs_vjp(brick.extents, brick.neighbors, states[k], ga,
+                                                    inv, lam), lam3)
+    got = run_adjoint(dg.Domain.from_brick(brick), "gh", states, ga, inv, lam3)
+    assert np.max(np.abs(got - ref)) <= GH_TOL * np.max(np.abs(ref))
+
+
+def test_gh_step_adjoint_mixed():
+    print("rk3 step adjoint gh mixed", flush=True)
+    brick, u, ga, inv, _ = wl.gh_adjoint_workload_mixed(seed=5, elements=(1, 2, 1), lowest=3,
+                                                        highest=10, noise=1e-3)
+    rng = np.random.default_rng(4)
+    states = [u * (1.0 + 1e-3 * rng.standard_normal(u.shape)) for _ in range(3)]
+    lam3 = rng.standard_normal(u.shape)
+    ref = step_adjoint(lambda k, lam: ol.gh_rhs_mixed_vjp(brick.extents, brick.neighbors,
+                                                          states[k], ga, inv, lam), lam3)
+    got = run_adjoint(dg.MixedDomain.from_brick(brick), "gh", states, ga, inv, lam3)
+    assert np.max(np.abs(got - ref)) <= GH_TOL * np.max(np.abs(ref))
