@@ -17,7 +17,12 @@
 // Each point gathers the face contributions that land on it (its own faces'
 // interior terms and the neighbours' exterior terms) and adds them in the
 // order (contributing element, direction), the order in which the oracle
-// scatters them, so results equal the oracle bit for bit.
+// scatters them, so results equal the oracle bit for bit.  Bound by the latency
+// of its phases (512 x 6^3: 13.4 us, 5 us of traffic).  Face terms that were
+// sorted first and evaluated in turn, each with loads, square roots and a
+// division of its own, were a serial chain of six, and LDS reads of all
+// components in flight spilled up to 1 KB per thread: 512 elements of 6^3 14.5,
+// of 7^3 29.5 -> 16.3, of 8^3 45.5 -> 23.2, of 10^3 278 -> 58 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -40,13 +45,31 @@ sw_rhs_adjoint_kernel(const int32_t* __restrict__ nbr, const double* __restrict_
                       double* __restrict__ ubar, const double* __restrict__ dtab,
                       Rk3AdjointUpdate update) {
   constexpr int NP = N * N * N;
-  __shared__ double s_x[15 * NP];  // logical-derivative adjoints [c][j][p]
+  // logical-derivative adjoints [c][j][p]; then, a column per point, the face
+  // terms' factors [slot] and normals [d][i]
+  __shared__ double s_x[15 * NP];
   const int64_t e = xcd_local_element(blockIdx.x, gridDim.x);
   const int t = threadIdx.x;
   const double* g = gbar + e * 5 * NP;
   const double* ij = inv_jac + e * 9 * NP;
   double gp[5], g2 = 0.0;
+  const int idx[3] = {t % N, (t / N) % N, t / (N * N)};
+  // the neighbours' values of all faces of the point, in flight during the sums
+  int64_t nbr_of[3] = {0, 0, 0};
+  double ijn[3][3], gn[3][4];
   if (t < NP) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      if (idx[d] != 0 && idx[d] != N - 1) continue;
+      const int64_t en = nbr[6 * e + 2 * d + (idx[d] == 0 ? 0 : 1)];
+      const int stride = d == 0 ? 1 : d == 1 ? N : N * N;
+      const int q = t + (idx[d] == 0 ? 1 : -1) * (N - 1) * stride;
+      nbr_of[d] = en;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) ijn[d][i] = inv_jac[(en * 9 + ij3(d, i)) * NP + q];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) gn[d][c] = gbar[(en * 5 + 1 + c) * NP + q];
+    }
 #pragma unroll
     for (int c = 0; c < 5; ++c) gp[c] = g[c * NP + t];
     g2 = gamma2[e * NP + t];
@@ -72,16 +95,17 @@ sw_rhs_adjoint_kernel(const int32_t* __restrict__ nbr, const double* __restrict_
       }
   }
   __syncthreads();
-  if (t >= NP) return;
-  const int idx[3] = {t % N, (t / N) % N, t / (N * N)};
   const double* D = diff_matrix(dtab, N);
   double ub[5];
-  ub[0] = 0.0;
-  ub[1] = 0.0 - gp[0];
+  if (t < NP) {
+    ub[0] = 0.0;
+    ub[1] = 0.0 - gp[0];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) ub[2 + i] = 0.0 - g2 * gp[2 + i];
+    for (int i = 0; i < 3; ++i) ub[2 + i] = 0.0 - g2 * gp[2 + i];
+  }
 #pragma unroll
   for (int c = 0; c < 5; ++c) {
+    if (t >= NP) break;
     double acc = ub[c];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -92,93 +116,73 @@ sw_rhs_adjoint_kernel(const int32_t* __restrict__ nbr, const double* __restrict_
         acc = fma(D[m * N + idx[j]], s_x[(3 * c + j) * NP + base + m * stride], acc);
     }
     ub[c] = acc;
+    // a component's LDS reads stay behind the sums before: all in flight at
+    // once they need more registers than there are
+    __builtin_amdgcn_sched_barrier(0);
   }
-  // face contributions: (element, direction, exterior?) sorted by element
-  // then direction.  Six fixed slots (slots of faces the point is not on are
-  // keyed last) and a fully unrolled exchange sort keep the lists in
-  // registers; a runtime index into them would place them in scratch memory.
+  // Face terms, added in ascending (element, direction) order of the face they
+  // stem from: slot 2 d the interior term of the own face, slot 2 d + 1 the
+  // exterior term of the neighbour's.  Their factors are formed together, and
+  // the order is a packed list of slots by rank.
   constexpr int64_t kNoFace = INT64_MAX;
   int64_t key[6];
-  int dim_of[6];
-  bool ext_of[6];
+  int terms = 0;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     const bool on = idx[d] == 0 || idx[d] == N - 1;
     const int s = idx[d] == 0 ? 0 : 1;
-    key[2 * d] = on ? static_cast<int64_t>(e) * 8 + 2 * d + s : kNoFace;
-    dim_of[2 * d] = d;
-    ext_of[2 * d] = false;
-    key[2 * d + 1] =
-        on ? static_cast<int64_t>(nbr[6 * e + 2 * d + s]) * 8 + 2 * d + (1 - s) : kNoFace;
-    dim_of[2 * d + 1] = d;
-    ext_of[2 * d + 1] = true;
+    key[2 * d] = on ? e * 8 + 2 * d + s : kNoFace;
+    key[2 * d + 1] = on ? nbr_of[d] * 8 + 2 * d + (1 - s) : kNoFace;
+    terms += on ? 2 : 0;
   }
+  __syncthreads();  // the sweeps have read the LDS
+  if (t >= NP) return;
+  double* mine = s_x + t;
+  unsigned order = 0;
 #pragma unroll
-  for (int a = 0; a < 5; ++a)
+  for (int d = 0; d < 3; ++d) {
+    if (idx[d] != 0 && idx[d] != N - 1) continue;
+    const int s = idx[d] == 0 ? 0 : 1;
+    int rank_in = 0, rank_ex = 0;
 #pragma unroll
-    for (int b = 0; b < 5 - a; ++b) {
-      const bool swap = key[b + 1] < key[b];
-      const int64_t k0 = key[b], k1 = key[b + 1];
-      key[b] = swap ? k1 : k0;
-      key[b + 1] = swap ? k0 : k1;
-      const int d0 = dim_of[b], d1 = dim_of[b + 1];
-      dim_of[b] = swap ? d1 : d0;
-      dim_of[b + 1] = swap ? d0 : d1;
-      const bool x0 = ext_of[b], x1 = ext_of[b + 1];
-      ext_of[b] = swap ? x1 : x0;
-      ext_of[b + 1] = swap ? x0 : x1;
+    for (int x = 0; x < 6; ++x) {
+      rank_in += key[x] < key[2 * d];
+      rank_ex += key[x] < key[2 * d + 1];
     }
+    order |= static_cast<unsigned>(2 * d) << (3 * rank_in) |
+             static_cast<unsigned>(2 * d + 1) << (3 * rank_ex);
+    // own normal (as interior and as the neighbour's exterior normal), and the
+    // neighbour's own
+    double n[3], nq[3], mag, magq;
 #pragma unroll
-  for (int x = 0; x < 6; ++x) {
-    if (key[x] == kNoFace) continue;
-    const int d = dim_of[x];
-    const int id = d == 0 ? idx[0] : (d == 1 ? idx[1] : idx[2]);
-    const int s = id == 0 ? 0 : 1;
-    if (!ext_of[x]) {
-      // interior term of this element's face (d, s)
-      double n[3], mag;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) n[i] = s == 0 ? ij[ij3(d, i) * NP + t] * -1.0 : ij[ij3(d, i) * NP + t];
-      flat_normalize(n, &mag);
-      const double fac = lift_factor(N, mag);
-      const double a = fac * gp[1];
-      double bn = (fac * gp[2]) * n[0];
-      bn = fma(fac * gp[3], n[1], bn);
-      bn = fma(fac * gp[4], n[2], bn);
-      const double s_in = 0.5 * (bn - a);
-      ub[0] = ub[0] + g2 * s_in;
-      ub[1] = ub[1] - s_in;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) ub[2 + i] = ub[2 + i] + n[i] * s_in;
-    } else {
-      // exterior term of the neighbour's face (d, 1 - s): its interior point
-      // is the matching point q of the neighbour
-      const int64_t en = nbr[6 * e + 2 * d + s];
-      const int qd = s == 0 ? N - 1 : 0;
-      const int q = (d == 0 ? qd : idx[0]) + N * ((d == 1 ? qd : idx[1]) +
-                                                  N * (d == 2 ? qd : idx[2]));
-      double nq[3], magq, ne[3], mage;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const double vq = inv_jac[(en * 9 + ij3(d, i)) * NP + q];
-        nq[i] = (1 - s) == 0 ? vq * -1.0 : vq;      // neighbour's own normal
-        const double vp = ij[ij3(d, i) * NP + t];
-        ne[i] = (1 - s) == 1 ? vp * -1.0 : vp;      // its exterior normal
-      }
-      flat_normalize(nq, &magq);
-      flat_normalize(ne, &mage);
-      const double fac = lift_factor(N, magq);
-      const double* gq = gbar + en * 5 * NP + q;
-      const double a = fac * gq[NP];
-      double bn = (fac * gq[2 * NP]) * ne[0];
-      bn = fma(fac * gq[3 * NP], ne[1], bn);
-      bn = fma(fac * gq[4 * NP], ne[2], bn);
-      const double s_ex = -0.5 * (a + bn);
-      ub[0] = ub[0] - g2 * s_ex;
-      ub[1] = ub[1] + s_ex;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) ub[2 + i] = ub[2 + i] + ne[i] * s_ex;
+    for (int i = 0; i < 3; ++i) {
+      const double v = ij[ij3(d, i) * NP + t];
+      n[i] = s == 0 ? v * -1.0 : v;
+      nq[i] = s == 1 ? ijn[d][i] * -1.0 : ijn[d][i];
     }
+    flat_normalize(n, &mag);
+    flat_normalize(nq, &magq);
+    // s_in = 0.5 (fac b.n - fac a), s_ex = -0.5 (fac a + fac b.n)
+    auto half_sum = [&](double fac, const double* b, double sign) {
+      const double a = fac * b[0];
+      double bn = (fac * b[1]) * n[0];
+      bn = fma(fac * b[2], n[1], bn);
+      bn = fma(fac * b[3], n[2], bn);
+      return sign > 0.0 ? 0.5 * (bn - a) : -0.5 * (a + bn);
+    };
+    mine[2 * d * NP] = half_sum(lift_factor(N, mag), gp + 1, 1.0);
+    mine[(2 * d + 1) * NP] = half_sum(lift_factor(N, magq), gn[d], -1.0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) mine[(6 + 3 * d + i) * NP] = n[i];
+  }
+  for (int x = 0; x < terms; ++x, order >>= 3) {
+    const int slot = order & 7, exterior = slot & 1;
+    const double f = mine[slot * NP];
+    const double* n = mine + (6 + 3 * (slot >> 1)) * NP;
+    ub[0] = exterior ? ub[0] - g2 * f : ub[0] + g2 * f;
+    ub[1] = exterior ? ub[1] + f : ub[1] - f;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) ub[2 + i] = ub[2 + i] + n[i * NP] * f;
   }
   if constexpr (UPDATE) {
 #pragma unroll
