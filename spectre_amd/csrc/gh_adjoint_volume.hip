@@ -220,7 +220,7 @@ gh_adjoint_point_kernel(int64_t total, int np_uniform, const MixedElement* __res
 }
 
 // S fields of the pair at a time (5, or 1 where their 15 Np derivative adjoints
-// leave fewer than two workgroups per CU).  Dynamic LDS: 3 S Np doubles, then
+// exceed the LDS).  Dynamic LDS: 3 S Np doubles, then
 // the D matrices.  contrib: face terms, [E][6][50][F] (uniform domains) or per
 // record as `table` places them.
 template <bool RAGGED, int S, bool UPDATE>
@@ -385,7 +385,10 @@ int launch_sweeps(int count, int np, int d_doubles, const int32_t ext[3], const 
                   const double* gbar, const double* work, double* ubar, const double* dtab,
                   const double* contrib, int F, const MortarCorrection* table,
                   hipStream_t stream, const Rk3AdjointUpdate& up) {
-  const bool five = 2 * (15 * np + d_doubles) <= kLdsDoubles;
+  // All five fields also where they leave one workgroup per CU: a field at a time
+  // each point's scalars are read and its adjoints formed five times (300 elements
+  // of 6^3 .. 10^3 223 -> 149 us, whole adjoint of 256 elements of 10^3 671 -> 618).
+  const bool five = 15 * np + d_doubles <= kLdsDoubles;
   const int lds = ((five ? 15 : 3) * np + d_doubles) * 8;
   const bool update = up.substep >= 0;
   const auto kernel = five ? (update ? &gh_adjoint_sweeps_kernel<RAGGED, 5, true>

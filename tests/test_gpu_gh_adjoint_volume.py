@@ -1,7 +1,8 @@
 """The kernels of the GH adjoint at the edges of their routes, against
 the oracle's reverse-mode tape: elements whose 15 derivative adjoints per point
-still leave two workgroups per CU and ones where they do not (8 x 9 x 9, 10 x 9 x
-9), elements whose five fields exceed the LDS (16^3), the smallest and flat
+leave two workgroups per CU or one (8 x 9 x 9, 10 x 9 x 9), the largest whose fit
+the LDS and ones beyond (11 x 12 x 10, 12 x 11 x 11), elements whose five fields
+exceed it (16^3), the smallest and flat
 ones, several point rounds per thread, and ragged elements of both size
 classes, whose mortars reach the largest LDS (extents 12 and 13)."""
 import numpy as np
@@ -32,7 +33,8 @@ def check(domain, u, gammas, inv, gbar, ref):
 
 @pytest.mark.parametrize("elements,extents", [((2, 1, 2), (2, 2, 2)), ((1, 2, 1), (20, 2, 3)),
                                               ((1, 2, 1), (8, 9, 9)), ((1, 1, 2), (10, 9, 9)),
-                                              ((1, 1, 1), (11, 12, 10)), ((1, 1, 1), (16, 16, 16))])
+                                              ((1, 1, 1), (11, 12, 10)), ((1, 1, 1), (16, 16, 16)),
+                                              ((1, 1, 1), (12, 11, 11))])
 def test_gh_adjoint_volume_edges(elements, extents):
     print(f"gh adjoint {elements} x {extents}", flush=True)
     brick, u, gammas, inv, _ = wl.gh_adjoint_workload(seed=1, elements=elements, extents=extents,
