@@ -59,9 +59,6 @@ __device__ __forceinline__ ElementShape element_shape(int64_t at, int n0, int n1
   return s;
 }
 
-// Points per thread whose sums are held in registers over the pairs of a half.
-constexpr int kSumRounds = 2;
-
 // S fields of a pair are staged together (5, or 1 for elements whose five fields
 // exceed the LDS), next to each other per point.  Dynamic LDS: S Np doubles,
 // then the D matrices.
@@ -84,90 +81,84 @@ gh_adjoint_sums_kernel(int n0, int n1, int n2, const MixedElement* __restrict__ 
   const double* ije = inv_jac + 9 * m.off;
   const double* ga = gammas + 3 * m.off;
   const int T = blockDim.x;
-  for (int base = 0; base < np; base += kSumRounds * T) {
-    double acc[kSumRounds][10];
+  for (int base = 0; base < np; base += T) {
+    const unsigned p = base + threadIdx.x;
+    const bool active = p < static_cast<unsigned>(np);
+    const int row = p / m.n0, k = row / m.n1;
+    const int i = p - row * m.n0, j = row - k * m.n1;
+    double a[10], ij[9], gamma1 = 0.0, gamma2 = 0.0;
 #pragma unroll
-    for (int r = 0; r < kSumRounds; ++r)
+    for (int x = 0; x < 10; ++x) a[x] = 0.0;
+    if (active) {
 #pragma unroll
-      for (int x = 0; x < 10; ++x) acc[r][x] = 0.0;
+      for (int c = 0; c < 9; ++c) ij[c] = (ije + c * np)[p];
+      gamma1 = (ga + np)[p];
+      gamma2 = (ga + 2 * np)[p];
+    }
 #pragma unroll 1
     for (int pr = 5 * half; pr < 5 * half + 5; ++pr) {
       const int comp[5] = {pr, 10 + pr, 20 + 3 * pr, 21 + 3 * pr, 22 + 3 * pr};
 #pragma unroll
       for (int c0 = 0; c0 < 5; c0 += S) {
         __syncthreads();
-        for (unsigned p = threadIdx.x; p < static_cast<unsigned>(np); p += T)
+        for (unsigned x = threadIdx.x; x < static_cast<unsigned>(np); x += T)
 #pragma unroll
-          for (int c = 0; c < S; ++c) s_lds[S * p + c] = (ue + comp[c0 + c] * np)[p];
+          for (int c = 0; c < S; ++c) s_lds[S * x + c] = (ue + comp[c0 + c] * np)[x];
         __syncthreads();
+        if (!active) continue;
+        double der[S][3];
+        auto sums = [&](int d, int nd, const double* w, const double* x, int step) {
 #pragma unroll
-        for (int r = 0; r < kSumRounds; ++r) {
-          const unsigned p = base + r * T + threadIdx.x;
-          if (p >= static_cast<unsigned>(np)) continue;
-          const int row = p / m.n0, k = row / m.n1;
-          const int i = p - row * m.n0, j = row - k * m.n1;
-          double der[S][3];
-          auto sums = [&](int d, int nd, const double* w, const double* x, int step) {
-#pragma unroll
-            for (int c = 0; c < S; ++c) der[c][d] = w[0] * x[c];
+          for (int c = 0; c < S; ++c) der[c][d] = w[0] * x[c];
 #pragma unroll 2
-            for (int l = 1; l < nd; ++l) {
-              x += step;
-              const double a = w[l];
+          for (int l = 1; l < nd; ++l) {
+            x += step;
+            const double a = w[l];
 #pragma unroll
-              for (int c = 0; c < S; ++c) der[c][d] = fma(a, x[c], der[c][d]);
+            for (int c = 0; c < S; ++c) der[c][d] = fma(a, x[c], der[c][d]);
+          }
+        };
+        sums(0, m.n0, D[0] + i * m.n0, s_lds + S * row * m.n0, S);
+        sums(1, m.n1, D[1] + j * m.n1, s_lds + S * (i + m.n0 * m.n1 * k), S * m.n0);
+        sums(2, m.n2, D[2] + k * m.n2, s_lds + S * (i + m.n0 * j), S * m.n0 * m.n1);
+        double w[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) w[c] = (ge + comp[c] * np)[p];
+#pragma unroll
+        for (int c = 0; c < S; ++c) {
+          const int f = c0 + c;  // field of the pair: g, Pi, Phi_0..2
+          double d[3];
+#pragma unroll
+          for (int x = 0; x < 3; ++x)
+            d[x] = fma(ij[ij3(2, x)], der[c][2],
+                       fma(ij[ij3(1, x)], der[c][1], ij[ij3(0, x)] * der[c][0]));
+          if (f == 0) {
+            const double s = gamma1 * gamma2 * w[1] + (1.0 + gamma1) * w[0];
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+              a[0] = fma(gamma2 * w[2 + x], d[x], a[0]);
+              a[1 + x] = fma(s, d[x], a[1 + x]);
             }
-          };
-          sums(0, m.n0, D[0] + i * m.n0, s_lds + S * row * m.n0, S);
-          sums(1, m.n1, D[1] + j * m.n1, s_lds + S * (i + m.n0 * m.n1 * k), S * m.n0);
-          sums(2, m.n2, D[2] + k * m.n2, s_lds + S * (i + m.n0 * j), S * m.n0 * m.n1);
-          double w[5], ij[9];
+          } else if (f == 1) {
 #pragma unroll
-          for (int c = 0; c < 5; ++c) w[c] = (ge + comp[c] * np)[p];
+            for (int x = 0; x < 3; ++x) {
+              a[0] = fma(-w[2 + x], d[x], a[0]);
+              a[1 + x] = fma(w[1], d[x], a[1 + x]);
+            }
+          } else {
 #pragma unroll
-          for (int c = 0; c < 9; ++c) ij[c] = (ije + c * np)[p];
-          const double gamma1 = (ga + np)[p], gamma2 = (ga + 2 * np)[p];
-          double* a = acc[r];
-#pragma unroll
-          for (int c = 0; c < S; ++c) {
-            const int f = c0 + c;  // field of the pair: g, Pi, Phi_0..2
-            double d[3];
-#pragma unroll
-            for (int x = 0; x < 3; ++x)
-              d[x] = fma(ij[ij3(2, x)], der[c][2],
-                         fma(ij[ij3(1, x)], der[c][1], ij[ij3(0, x)] * der[c][0]));
-            if (f == 0) {
-              const double s = gamma1 * gamma2 * w[1] + (1.0 + gamma1) * w[0];
-#pragma unroll
-              for (int x = 0; x < 3; ++x) {
-                a[0] = fma(gamma2 * w[2 + x], d[x], a[0]);
-                a[1 + x] = fma(s, d[x], a[1 + x]);
-              }
-            } else if (f == 1) {
-#pragma unroll
-              for (int x = 0; x < 3; ++x) {
-                a[0] = fma(-w[2 + x], d[x], a[0]);
-                a[1 + x] = fma(w[1], d[x], a[1 + x]);
-              }
-            } else {
-#pragma unroll
-              for (int x = 0; x < 3; ++x) {
-                a[1 + x] = fma(w[f], d[x], a[1 + x]);
-                a[4 + sym3(x, f - 2)] = fma(w[1], d[x], a[4 + sym3(x, f - 2)]);
-              }
+            for (int x = 0; x < 3; ++x) {
+              a[1 + x] = fma(w[f], d[x], a[1 + x]);
+              a[4 + sym3(x, f - 2)] = fma(w[1], d[x], a[4 + sym3(x, f - 2)]);
             }
           }
         }
       }
     }
+    if (!active) continue;
     double* out = work + kGhAdjointDoubles * m.off + kSums * half * np;
 #pragma unroll
-    for (int r = 0; r < kSumRounds; ++r) {
-      const unsigned p = base + r * T + threadIdx.x;
-      if (p >= static_cast<unsigned>(np)) continue;
-#pragma unroll
-      for (int x = 0; x < 10; ++x) (out + x * np)[p] = acc[r][x];
-    }
+    for (int x = 0; x < 10; ++x) (out + x * np)[p] = a[x];
   }
 }
 
@@ -342,10 +333,10 @@ gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* 
   }
 }
 
-// Threads for np points in at most kSumRounds rounds where 512 allow it.
-int sums_threads(int np) {
-  return std::min(512, std::max(64, (np + 64 * kSumRounds - 1) / (64 * kSumRounds) * 64));
-}
+// A thread per point up to 512: two workgroups per element are few, so that more
+// waves count for more than fewer stagings (300 x 6^3: 33.8 us with two points
+// per thread, 24.9 with one).
+int sums_threads(int np) { return std::min(512, (np + 63) / 64 * 64); }
 
 constexpr int kLdsDoubles = 160 * 1024 / 8;
 
