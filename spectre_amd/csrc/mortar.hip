@@ -17,9 +17,10 @@
 //
 // Two organisations.  Where every mortar is local, mortar_faces.hip takes each
 // mortar from the fields to both sides' lifted corrections in one workgroup.
-// Here, around an exchange of boundary messages, the packages stay in HBM between the steps and the
-// receiver gathers the partner's package through a per-record index table (the
-// partner's oriented offsets, inverted on the host), so no data is reordered:
+// Here, around an exchange of boundary messages, the packages stay in HBM
+// between the steps and the receiver gathers the partner's package through a
+// per-record index table (the partner's oriented offsets, inverted on the
+// host), so no data is reordered:
 //   1. mortar_package_kernel: one workgroup per face, the package of every
 //      face point and |n| (SW 13 values, GH 10 pairs x 13 + 4 speeds);
 //      mortar_direct_kernel instead for a face whose single mortar differs
