@@ -1725,9 +1725,7 @@ namespace {
 int run_gh_adjoint_mixed(sxd_domain* d, Scratch& sc, const double* u, const double* gammas,
                          const double* inv_jac, const double* gbar, double* ubar,
                          hipStream_t stream, const Rk3AdjointUpdate& up) {
-  if (!d->conforming_plan || mixed_face_adjoint_lds_bytes(d->kf, d->km) > 160 * 1024 ||
-      (kStagedDiffDoubles + 3 * d->np_max) * 8 > 160 * 1024)
-    return SXD_ERR_UNSUPPORTED;
+  if (!d->conforming_plan) return SXD_ERR_UNSUPPORTED;
   const size_t volume = kGhAdjointDoubles * static_cast<size_t>(d->total_points);
   const GhAdjointFacesWork size(d->plan, nullptr);
   if (int rc = sc.reserve_block(kAdjointBlock, size.doubles + volume); rc != SXD_OK) return rc;

@@ -391,8 +391,6 @@ int launch_ragged_gh_adjoint_sweeps(const std::vector<RaggedClass>& classes, con
                                     const double* work, double* ubar,
                                     const MortarCorrection* table, const double* contrib,
                                     hipStream_t stream, const Rk3AdjointUpdate& up = {});
-// Largest LDS of the face kernel the mixed-p adjoint's size limit stems from.
-int mixed_face_adjoint_lds_bytes(int kf, int km);
 // Adjoint (transpose) of the ScalarWave RHS on a uniform domain (isotropic
 // extents 2..10) and of one RK3 substep.
 bool sw_adjoint_supported(const int32_t ext[3]);

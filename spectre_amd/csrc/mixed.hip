@@ -1003,6 +1003,4 @@ int launch_mixed_gh_face_passes(int count, const int32_t* list, const MixedEleme
   return SXD_OK;
 }
 
-int mixed_face_adjoint_lds_bytes(int kf, int km) { return (30 * kf + 51 * km) * 8; }
-
 }  // namespace sxd
