@@ -1070,8 +1070,9 @@ int run_mixed(sxd_domain* d, Scratch& sc, bool gh, int kernel, const double* u,
                             inv_jac, dt, scratch, threads, stream, ghost, bc_kind);
   for (const auto& b : d->buckets) {
     const int rc = launch_mixed_rhs(gh, {{0, b.second, d->np_max, kStagedDiffDoubles}},
-                                    d->d_buckets + b.first, d->d_el, d->d_nbr, d->kf, d->km, u, params, inv_jac, dt,
-                                    scratch, threads, stream, ghost, bc_kind);
+                                    d->d_buckets + b.first, d->d_el, d->d_nbr, d->kf, d->km, u,
+                                    params, inv_jac, dt, scratch, threads, stream, ghost,
+                                    bc_kind);
     if (rc != SXD_OK) return rc;
   }
   return SXD_OK;

@@ -484,9 +484,9 @@ int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* n
                      dim3(128), 0, stream, total, ext[0], ext[1], ext[2], nullptr, nullptr, u,
                      gammas, inv_jac, work, sides);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(pair_kernel, dim3(10 * num_elements), dim3(pair_threads(np)), lds, stream, num_elements, ext[0], ext[1], ext[2],
-                     nullptr, nullptr, nbr, u, gammas, inv_jac, work, sides, ghost, dt, dtab, nullptr,
-                     nullptr, up);
+  hipLaunchKernelGGL(pair_kernel, dim3(10 * num_elements), dim3(pair_threads(np)), lds, stream,
+                     num_elements, ext[0], ext[1], ext[2], nullptr, nullptr, nbr, u, gammas,
+                     inv_jac, work, sides, ghost, dt, dtab, nullptr, nullptr, up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 
