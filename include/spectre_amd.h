@@ -555,7 +555,11 @@ int sxd_gh_rhs_bjorhus(const sxd_domain* domain, int bjorhus_type, const double*
  * SXD_ERR_UNSUPPORTED if the kernel cannot run these extents.  Not
  * thread-safe against concurrent RHS calls on the same domain. */
 int sxd_domain_set_kernel(sxd_domain* domain, int system, int kernel);
-/* The kernel the next RHS call on this domain will use. */
+/* The kernel the next RHS call on this domain will use.  Where the library
+ * chose SXD_KERNEL_COMPOSITE for GH extents that the fused kernel also takes
+ * (AUTO or autotuned, not set), a call under stream capture, one whose work
+ * array cannot be allocated and sxd_gh_rhs_noalloc run the fused kernel, which
+ * needs no work array and gives the same result. */
 int sxd_domain_get_kernel(const sxd_domain* domain, int system, int* kernel);
 /* Threads per workgroup (tile shape): mixed-p kernels 64, 128 or 256
  * (default 128); the fused GH kernel at 7^3 and 8^3 points 256 (one wave per

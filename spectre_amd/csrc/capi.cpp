@@ -145,9 +145,11 @@ struct sxd_domain {
   // streams never share one.
   std::mutex scratch_mutex;
   std::vector<std::pair<void*, std::unique_ptr<sxd::Scratch>>> scratch;
-  // Kernel choice per system (SXD_SYSTEM_*), SXD_KERNEL_AUTO until set, and
-  // threads per workgroup of the mixed-p kernels.
+  // Kernel choice per system (SXD_SYSTEM_*), SXD_KERNEL_AUTO until set or
+  // timed, whether the caller set it, and threads per workgroup of the mixed-p
+  // kernels.
   int kernel[2] = {SXD_KERNEL_AUTO, SXD_KERNEL_AUTO};
+  bool pinned[2] = {false, false};
   int threads[2] = {128, 128};
   // Mixed p: per-element extents and offsets (ragged layout).
   bool mixed = false;
@@ -956,16 +958,22 @@ int resolve_kernel(const sxd_domain* d, int system) {
   return k[0];
 }
 
+// Whether a GH call may run the fused kernel in place of `kernel`: the pair
+// kernels, chosen by the library (gh_pairs_faster or the autotuner) and not by
+// the caller.
+bool fused_stands_in(const sxd_domain* d, int kernel) {
+  return kernel == SXD_KERNEL_COMPOSITE && !d->pinned[SXD_SYSTEM_GH] && !d->mixed &&
+         gh_fused_supported(d->ext);
+}
+
 // The GH kernel of one call on `stream`.  Where the pair kernels stand in for
-// the fused one (gh_pairs_faster) they need a work array that the fused kernel
-// does not: a call recorded into the caller's graph, whose replays may run
-// beside later calls or outlive the array, and a call whose array cannot be
-// allocated, keep the fused kernel.
+// the fused one they need a work array that the fused kernel does not: a call
+// recorded into the caller's graph, whose replays may run beside later calls or
+// outlive the array, and a call whose array cannot be allocated, keep the fused
+// kernel.
 int gh_call_kernel(const sxd_domain* d, Scratch& sc, hipStream_t stream) {
   const int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
-  if (kernel != SXD_KERNEL_COMPOSITE || d->kernel[SXD_SYSTEM_GH] != SXD_KERNEL_AUTO ||
-      d->mixed || !gh_fused_supported(d->ext))
-    return kernel;
+  if (!fused_stands_in(d, kernel)) return kernel;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
       capture != hipStreamCaptureStatusNone)
@@ -1299,8 +1307,7 @@ int sxd_gh_rhs_noalloc(const sxd_domain* domain, const double* u, const double* 
   sxd_domain* d = const_cast<sxd_domain*>(domain);
   int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
   // no work arrays where the caller has not asked for a kernel that needs them
-  if (d->kernel[SXD_SYSTEM_GH] == SXD_KERNEL_AUTO && !d->mixed && gh_fused_supported(d->ext))
-    kernel = SXD_KERNEL_FUSED;
+  if (fused_stands_in(d, kernel)) kernel = SXD_KERNEL_FUSED;
   // the mortar organisation's package buffers do not fit the fixed array at
   // useful sizes: mixed-p domains run the batched mixed-p kernels here
   if (kernel == SXD_KERNEL_MORTAR) kernel = SXD_KERNEL_MIXED_BATCHED;
@@ -1583,6 +1590,7 @@ int sxd_domain_set_kernel(sxd_domain* domain, int system, int kernel) {
       return fail(SXD_ERR_UNSUPPORTED, "kernel %d is not available for these extents", kernel);
   }
   domain->kernel[system] = kernel;
+  domain->pinned[system] = kernel != SXD_KERNEL_AUTO;
   return ok();
 }
 
@@ -1659,6 +1667,7 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
   (void)hipEventDestroy(ev[1]);
   if (rc != SXD_OK) return finish(rc, __func__);
   domain->kernel[system] = best;
+  domain->pinned[system] = false;
   if (chosen != nullptr) *chosen = best;
   if (milliseconds != nullptr) *milliseconds = best_ms;
   return ok();
