@@ -567,6 +567,9 @@ int sxd_domain_get_kernel(const sxd_domain* domain, int system, int* kernel);
  * thread).  Results do not depend on it. */
 int sxd_domain_set_threads(sxd_domain* domain, int system, int threads);
 int sxd_domain_get_threads(const sxd_domain* domain, int system, int* threads);
+/* Give `domain` the kernel and thread choices of `from`, a domain over elements
+ * of the same extents: set by the caller, timed by the autotuner, or AUTO. */
+int sxd_domain_copy_choices(sxd_domain* domain, const sxd_domain* from);
 /* Autotuner: time every kernel available for (domain, system) on the given
  * inputs (one warm-up, then `repetitions` timed calls each, HIP events on
  * `stream`), keep the fastest for later calls and return it in *chosen and

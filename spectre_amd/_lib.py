@@ -94,6 +94,7 @@ _SIGNATURES = {
                                               _vp]),
     "sxd_rk3_stepper_step": (ctypes.c_int, [_vp, ctypes.c_double, ctypes.c_int, _vp]),
     "sxd_rk3_stepper_destroy": (ctypes.c_int, [_vp]),
+    "sxd_domain_copy_choices": (ctypes.c_int, [_vp, _vp]),
     "sxd_domain_get_kernel": (ctypes.c_int, [_vp, ctypes.c_int, _ip]),
     "sxd_domain_autotune": (ctypes.c_int, [_vp, ctypes.c_int, _vp, _vp, _vp, _vp, ctypes.c_int, _vp,
                                            _ip, ctypes.POINTER(ctypes.c_float)]),

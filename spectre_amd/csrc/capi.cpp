@@ -1594,6 +1594,20 @@ int sxd_domain_set_kernel(sxd_domain* domain, int system, int kernel) {
   return ok();
 }
 
+int sxd_domain_copy_choices(sxd_domain* domain, const sxd_domain* from) {
+  if (domain == nullptr || from == nullptr) return fail(SXD_ERR_INVALID_ARGUMENT, "null domain");
+  if (domain->mixed != from->mixed || domain->mortars != from->mortars ||
+      domain->conforming_plan != from->conforming_plan ||
+      (!domain->mixed && std::memcmp(domain->ext, from->ext, sizeof(domain->ext)) != 0))
+    return fail(SXD_ERR_INVALID_ARGUMENT, "%s: domains of different kinds or extents", __func__);
+  for (int system = 0; system < 2; ++system) {
+    domain->kernel[system] = from->kernel[system];
+    domain->pinned[system] = from->pinned[system];
+    domain->threads[system] = from->threads[system];
+  }
+  return ok();
+}
+
 int sxd_domain_get_kernel(const sxd_domain* domain, int system, int* kernel) {
   if (int rc = check_domain(domain); rc != SXD_OK) return rc;
   if (system != SXD_SYSTEM_SCALAR_WAVE && system != SXD_SYSTEM_GH)

@@ -539,9 +539,7 @@ class Domain:
         tile choices and work arrays of its own, for RHS calls on another
         stream at the same time as this domain's."""
         t = type(self)(*self._args)
-        for system in SYSTEMS:
-            t.set_kernel(system, self.kernel(system))
-            t.set_threads(system, self.threads(system))
+        check(lib().sxd_domain_copy_choices(t.handle, self._handle))
         return t
 
     def set_threads(self, system, threads):

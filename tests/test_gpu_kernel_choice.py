@@ -59,3 +59,23 @@ def test_autotuned_choice_without_work_arrays():
     assert domain.kernel("gh") == "composite"
     got = domain.gh_rhs_noalloc(u, gammas, inv, torch.empty_like(u))
     assert np.array_equal(host(got), host(domain.gh_rhs(u, gammas, inv)))
+
+
+@pytest.mark.parametrize("choice", ["auto", "autotuned", "fused", "composite"])
+def test_twin_has_the_same_choice(choice):
+    """A twin is chosen for like its domain: pinned only where that is."""
+    print(f"twin of {choice}", flush=True)
+    brick, u, gammas, inv = gh_case((2, 2, 2), 6)
+    domain = dg.Domain.from_brick(brick)
+    if choice == "autotuned":
+        domain.autotune("gh", u, gammas, inv, torch.empty_like(u))
+    else:
+        domain.set_kernel("gh", choice)
+    domain.set_threads("gh", 512)
+    twin = domain.twin()
+    assert twin.kernel("gh") == domain.kernel("gh") and twin.threads("gh") == 512
+    if choice != "composite":  # pinned, it needs its work array before a capture
+        replay_against_eager(twin, u, gammas, inv)
+    other = dg.Domain((5, 5, 5), brick.neighbors)
+    with pytest.raises(dg.SpectreAmdError, match="different"):
+        dg.check(dg.lib().sxd_domain_copy_choices(other.handle, domain.handle))
