@@ -966,11 +966,22 @@ bool fused_stands_in(const sxd_domain* d, int kernel) {
          gh_fused_supported(d->ext);
 }
 
-// The GH kernel of one call on `stream`.  Where the pair kernels stand in for
-// the fused one they need a work array that the fused kernel does not: a call
-// recorded into the caller's graph, whose replays may run beside later calls or
-// outlive the array, and a call whose array cannot be allocated, keep the fused
-// kernel.
+// The GH kernel that runs with the work arrays sc.  Where the pair kernels stand
+// in for the fused one they need a work array that the fused kernel does not:
+// if it cannot be allocated the fused kernel runs.
+int gh_kernel_with_arrays(const sxd_domain* d, Scratch& sc) {
+  const int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
+  if (fused_stands_in(d, kernel) &&
+      sc.reserve_block(SXD_SYSTEM_GH, gh_pairs_work_doubles(d->num_elements, d->ext)) != SXD_OK) {
+    (void)hipGetLastError();
+    return SXD_KERNEL_FUSED;
+  }
+  return kernel;
+}
+
+// The GH kernel of one call on `stream`: a call recorded into the caller's graph,
+// whose replays may run beside later calls or outlive the work array, also
+// runs the fused kernel where the pair kernels stand in for it.
 int gh_call_kernel(const sxd_domain* d, Scratch& sc, hipStream_t stream) {
   const int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
   if (!fused_stands_in(d, kernel)) return kernel;
@@ -978,11 +989,7 @@ int gh_call_kernel(const sxd_domain* d, Scratch& sc, hipStream_t stream) {
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
       capture != hipStreamCaptureStatusNone)
     return SXD_KERNEL_FUSED;
-  if (sc.reserve_block(SXD_SYSTEM_GH, gh_pairs_work_doubles(d->num_elements, d->ext)) != SXD_OK) {
-    (void)hipGetLastError();
-    return SXD_KERNEL_FUSED;
-  }
-  return kernel;
+  return gh_kernel_with_arrays(d, sc);
 }
 
 // Reserve work arrays (status only; finish() words the message).
@@ -1865,6 +1872,7 @@ int sxd_rk3_adjoint_substep(int substep, int64_t n, double dt, const double* lam
 struct sxd_rk3_stepper {
   sxd_domain* domain = nullptr;
   int system = 0;
+  int kernel = SXD_KERNEL_AUTO;  // of its right-hand sides, resolved at creation
   int64_t n = 0;                 // doubles per field
   double* u = nullptr;           // caller's state, updated in place
   double* d_stage = nullptr;     // u1 (and u2, where the work array holds the RHS)
@@ -1894,9 +1902,8 @@ int enqueue_rk3_step(sxd_rk3_stepper* s, const double* params, const double* inv
                      hipStream_t stream) {
   Rk3Update up;
   up.dt_ptr = s->d_dt;
-  return run_rk3_step(s->domain, s->scratch, s->system, resolve_kernel(s->domain, s->system),
-                      params, inv_jac, up, s->u, s->d_stage, s->d_work, s->d_work, s->u, s->n,
-                      stream);
+  return run_rk3_step(s->domain, s->scratch, s->system, s->kernel, params, inv_jac, up, s->u,
+                      s->d_stage, s->d_work, s->d_work, s->u, s->n, stream);
 }
 }  // namespace
 
@@ -1933,8 +1940,10 @@ int sxd_rk3_stepper_create(sxd_rk3_stepper** stepper, sxd_domain* domain, int sy
   // sets kernel attributes, so the captured region only enqueues kernels.
   // The graph refers to those arrays only: calls on the domain afterwards
   // (which may grow the domain's own work arrays) cannot move them.
-  int rc = run_system(domain, s->scratch, system, resolve_kernel(domain, system), u, params,
-                      inv_jac, s->d_work, s->capture);
+  s->kernel = system == SXD_SYSTEM_GH ? gh_kernel_with_arrays(domain, s->scratch)
+                                      : resolve_kernel(domain, system);
+  int rc = run_system(domain, s->scratch, system, s->kernel, u, params, inv_jac, s->d_work,
+                      s->capture);
   if (rc == SXD_OK && hipStreamSynchronize(s->capture) != hipSuccess) rc = SXD_ERR_DEVICE;
   if (rc != SXD_OK) {
     destroy_stepper(s);

@@ -1,6 +1,8 @@
 """The kernel that a call runs where the library, not the caller, made the
 choice: the same results with and without room for work arrays, inside and
 outside of a captured graph."""
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -79,3 +81,50 @@ def test_twin_has_the_same_choice(choice):
     other = dg.Domain((5, 5, 5), brick.neighbors)
     with pytest.raises(dg.SpectreAmdError, match="different"):
         dg.check(dg.lib().sxd_domain_copy_choices(other.handle, domain.handle))
+
+
+@contextlib.contextmanager
+def only_free(free_bytes):
+    """Hold all but free_bytes of the device's memory."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    held = []
+    try:
+        while (spare := torch.cuda.mem_get_info()[0] - free_bytes) >= 64 << 20:
+            held.append(torch.empty(min(spare, 16 << 30), dtype=torch.uint8, device="cuda"))
+        yield
+    finally:
+        torch.cuda.synchronize()
+        held.clear()
+        torch.cuda.empty_cache()
+
+
+def test_no_room_for_work_arrays():
+    """8000 elements of 7^3: a field takes 1.1 GB, the pair kernels' work array
+    1.0 GB.  With room for the fields but not for it, a stepper, a step and an
+    RHS run the fused kernel; pinned pair kernels report the missing memory."""
+    print("no room for work arrays", flush=True)
+    _, u, gammas, inv = gh_case((1, 1, 1), 7)
+    elements = (20, 20, 20)
+    u, gammas, inv = (t.repeat(8000, 1, 1).contiguous() for t in (u, gammas, inv))
+    field = u.numel() * 8
+    create = lambda kernel: (d := dg.Domain((7, 7, 7), wl.periodic_neighbors(elements)),
+                             d.set_kernel("gh", kernel))[0]
+    start, out = u.clone(), torch.empty_like(u)
+    stepper = dg.Rk3Stepper(create("fused"), "gh", u, gammas, inv)
+    stepper.step(1e-4)
+    stepper.close()
+    after, rhs = u.clone(), create("fused").gh_rhs(u, gammas, inv)
+    u.copy_(start)
+    assert create("auto").kernel("gh") == "composite"
+    with only_free(2 * field + (550 << 20)):
+        with pytest.raises(dg.SpectreAmdError, match="work arrays"):
+            dg.Rk3Stepper(create("composite"), "gh", u, gammas, inv)
+        stepper = dg.Rk3Stepper(create("auto"), "gh", u, gammas, inv)
+        stepper.step(1e-4)
+        with pytest.raises(dg.SpectreAmdError, match="work arrays"):
+            create("composite").gh_rhs(u, gammas, inv, out)
+        create("auto").gh_rhs(u, gammas, inv, out)
+        torch.cuda.synchronize()
+        stepper.close()
+    assert torch.equal(u, after) and torch.equal(out, rhs)
