@@ -104,11 +104,17 @@ struct Scratch {
       if (n > fixed_doubles) return SXD_ERR_UNSUPPORTED;
       block[system] = du;
     }
-    if (block[system] == nullptr && hipMalloc(&block[system], n * sizeof(double)) != hipSuccess) {
-      block[system] = nullptr;
-      return SXD_ERR_OUT_OF_MEMORY;
-    }
-    return SXD_OK;
+    if (block[system] != nullptr) return SXD_OK;
+    // The array keeps its place while the domain lives, so that it may also be
+    // allocated while a stream is captured, by this thread or another: an
+    // allocation in the default mode would end that capture.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return SXD_ERR_OUT_OF_MEMORY;
+    const hipError_t err = hipMalloc(&block[system], n * sizeof(double));
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (err == hipSuccess) return SXD_OK;
+    block[system] = nullptr;
+    return SXD_ERR_OUT_OF_MEMORY;
   }
   void release() {
     if (!fixed) {

@@ -2,6 +2,8 @@
 choice: the same results with and without room for work arrays, inside and
 outside of a captured graph."""
 import contextlib
+import gc
+import threading
 
 import numpy as np
 import pytest
@@ -83,15 +85,75 @@ def test_twin_has_the_same_choice(choice):
         dg.check(dg.lib().sxd_domain_copy_choices(other.handle, domain.handle))
 
 
+def test_first_rhs_in_a_graph_after_other_calls():
+    """A stream that has run the adjoint or a condition that needs work arrays
+    may record its first RHS."""
+    print("first rhs in a graph", flush=True)
+    brick, u, gammas, inv = gh_case((1, 2, 1), 12)
+    stream = torch.cuda.Stream()
+    for other in ("adjoint", "bjorhus"):
+        domain = dg.Domain.from_brick(brick)
+        out = torch.empty_like(u)
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            if other == "adjoint":
+                domain.gh_rhs_adjoint(u, gammas, inv, u, out)
+            else:
+                domain.gh_rhs_bjorhus(u, gammas, inv, dev(brick.coordinates()), out)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            domain.gh_rhs(u, gammas, inv, out)
+        ref = host(dg.Domain.from_brick(brick).gh_rhs(u, gammas, inv))
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            assert np.array_equal(host(out), ref)
+
+
+def test_first_rhs_beside_a_capture():
+    """A thread's first RHS leaves another thread's capture valid."""
+    print("first rhs beside a capture", flush=True)
+    brick, u, gammas, inv = gh_case((2, 2, 2), 6)
+    ref = host(dg.Domain.from_brick(brick).gh_rhs(u, gammas, inv))
+    domain, got = dg.Domain.from_brick(brick), torch.empty_like(u)
+    x = torch.ones(8, device="cuda")
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    done = []
+
+    def call():
+        with torch.cuda.stream(stream):
+            domain.gh_rhs(u, gammas, inv, got)
+        done.append(True)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1.0)
+        thread = threading.Thread(target=call)
+        thread.start()
+        thread.join(60)
+    assert done == [True]
+    graph.replay()
+    assert np.array_equal(host(got), ref) and host(x)[0] == 2.0
+
+
 @contextlib.contextmanager
 def only_free(free_bytes):
-    """Hold all but free_bytes of the device's memory."""
+    """Hold all but free_bytes (and at most 64 MiB more) of the device's memory."""
+    gc.collect()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    room = torch.empty(free_bytes, dtype=torch.uint8, device="cuda")
     held = []
     try:
-        while (spare := torch.cuda.mem_get_info()[0] - free_bytes) >= 64 << 20:
-            held.append(torch.empty(min(spare, 16 << 30), dtype=torch.uint8, device="cuda"))
+        for size in (16 << 30, 1 << 30, 64 << 20):
+            with contextlib.suppress(torch.OutOfMemoryError):
+                while True:
+                    held.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+        del room
+        torch.cuda.empty_cache()
         yield
     finally:
         torch.cuda.synchronize()
