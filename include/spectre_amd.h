@@ -447,9 +447,10 @@ int sxd_gh_rhs(const sxd_domain* domain, const double* u, const double* gammas,
  * is for callers that cannot allocate (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  The domain (and so its
  * device tables) must already exist.  SXD_ERR_UNSUPPORTED if the domain's
- * work arrays exceed the fixed array: 150 doubles per grid point on mixed-p
- * domains (about 111,000 points), 162 per point with the composite kernel,
- * none with the fused kernels (mixed-p domains run their batched mixed-p
+ * work arrays exceed the fixed array: 35 doubles per grid point on mixed-p
+ * domains (about 479,000 points); with the composite kernel 35 per point and 12
+ * per face point for elements of up to about 14^3 (45 per point at 7^3), 162
+ * per point beyond; none with the fused kernels (mixed-p domains run their batched mixed-p
  * kernels here, also where SXD_KERNEL_MORTAR is selected; mortar domains
  * return SXD_ERR_UNSUPPORTED).  Every call on one device shares that device's
  * array, which keeps the last call's contents: calls that overlap on one GPU

@@ -1081,8 +1081,8 @@ int run_mixed(sxd_domain* d, Scratch& sc, bool gh, int kernel, const double* u,
   }
   double* scratch = nullptr;
   if (gh) {
-    if (int rc = reserve_scratch(sc, 150 * static_cast<size_t>(d->total_points), 0); rc != SXD_OK)
-      return rc;
+    const size_t states = kGhStateDoubles * static_cast<size_t>(d->total_points);
+    if (int rc = reserve_scratch(sc, states, 0); rc != SXD_OK) return rc;
     scratch = sc.du;
   }
   const int threads = d->threads[gh ? SXD_SYSTEM_GH : SXD_SYSTEM_SCALAR_WAVE];
@@ -1324,14 +1324,16 @@ int sxd_gh_rhs_noalloc(const sxd_domain* domain, const double* u, const double* 
   // the mortar organisation's package buffers do not fit the fixed array at
   // useful sizes: mixed-p domains run the batched mixed-p kernels here
   if (kernel == SXD_KERNEL_MORTAR) kernel = SXD_KERNEL_MIXED_BATCHED;
-  // work arrays the kernel organisation needs: 150 doubles per point (mixed
-  // p), 162 (composite), none (fused)
+  // work arrays the kernel organisation needs: the point states (mixed p, and
+  // with 12 doubles per face point the pair kernels), 162 doubles per point
+  // (composite kernels of larger elements), none (fused)
   const size_t points = static_cast<size_t>(domain_points(d));
   size_t need = 0;
   if (d->mixed)
-    need = 150 * points;
+    need = kGhStateDoubles * points;
   else if (kernel == SXD_KERNEL_COMPOSITE)
-    need = 162 * points;
+    need = gh_pairs_supported(d->ext) ? gh_pairs_work_doubles(d->num_elements, d->ext)
+                                      : 162 * points;
   if (need > noalloc_scratch_doubles())
     return fail(SXD_ERR_UNSUPPORTED,
                 "%s: the domain's work arrays need %zu doubles, above the fixed array's %zu "
@@ -1423,8 +1425,8 @@ int sxd_rhs_begin(const sxd_domain* domain, int system, const double* u, const d
   hipStream_t s = static_cast<hipStream_t>(stream);
   Scratch& sc = stream_scratch(d, s);
   std::lock_guard<std::mutex> enqueue(sc.enqueue);
-  const size_t du = gh ? 150 * static_cast<size_t>(d->total_points) : 0;
-  int rc = reserve_scratch(sc, du, mortar_work_doubles(gh, d->plan));
+  const size_t states = gh ? kGhStateDoubles * static_cast<size_t>(d->total_points) : 0;
+  int rc = reserve_scratch(sc, states, mortar_work_doubles(gh, d->plan));
   if (rc == SXD_OK)
     rc = run_ragged_volume(d, gh, u, params, inv_jac, dt, sc.du, s);
   if (rc == SXD_OK)

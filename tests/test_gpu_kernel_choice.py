@@ -65,6 +65,22 @@ def test_autotuned_choice_without_work_arrays():
     assert np.array_equal(host(got), host(domain.gh_rhs(u, gammas, inv)))
 
 
+@pytest.mark.parametrize("layout", ["composite", "mixed"])
+def test_noalloc_takes_what_fits_its_array(layout):
+    """343 elements of 7^3 (117,649 points): 45 (composite) and 35 (mixed)
+    doubles per point fit 16 Mi, 150 do not."""
+    print(f"noalloc {layout}", flush=True)
+    brick, u, gammas, inv = gh_case((7, 7, 7), 7)
+    if layout == "mixed":
+        domain = dg.MixedDomain(np.tile(brick.extents, (343, 1)), brick.neighbors)
+        u, gammas, inv = (t.reshape(-1) for t in (u, gammas, inv))
+    else:
+        domain = dg.Domain.from_brick(brick)
+        domain.set_kernel("gh", "composite")
+    got = domain.gh_rhs_noalloc(u, gammas, inv, torch.full_like(u, float("nan")))
+    assert np.array_equal(host(got), host(domain.gh_rhs(u, gammas, inv)))
+
+
 @pytest.mark.parametrize("choice", ["auto", "autotuned", "fused", "composite"])
 def test_twin_has_the_same_choice(choice):
     """A twin is chosen for like its domain: pinned only where that is."""
