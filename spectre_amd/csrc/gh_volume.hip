@@ -416,19 +416,19 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
   }
 }
 
-// Threads of a workgroup that takes np points in rounds: a multiple of 64, at
-// most 320, with the fewest idle lanes in the last round (the most threads
-// among equals).
-int pair_threads(int np) {
-  int best = 64, waste = 1 << 30;
-  for (int t = 64; t <= 320; t += 64) {
-    const int w = (np + t - 1) / t * t - np;
-    if (w <= waste && t < np + 64) {
-      best = t;
-      waste = w;
-    }
-  }
-  return best;
+// Threads of a workgroup that takes np points in rounds.  Up to 256 points, or
+// where the launch has no second workgroup for a CU: one round (2 elements of
+// 7x7x6 16.6 us, with 192 threads 19.3).  Up to 768, where several workgroups share a CU: 192 or 256, whichever
+// leaves fewer lanes idle in the last round (360 elements of 7x7x6 with 192 / 256 /
+// 320 / 512 threads 81 / 85 / 101 / 100 us, of 8x8x7 115 / 106 / 141 / 125, of 9^3
+// 202 / 191 / 224 / 197).  Beyond: 512, the more so where the LDS leaves one
+// workgroup per CU (360 of 10x9x9 283 / 259 / 251 / 228; 64 of 14^3 249 / 203 / 182 /
+// 154).  The fewest idle lanes alone can mean 64 threads: 526 us on 360 of
+// 10x9x9, 577 on 64 of 14^3.
+int pair_threads(int np, int workgroups) {
+  if (np > 768) return 512;
+  if (np <= 256 || workgroups <= 256) return std::min(512, (np + 63) / 64 * 64);
+  return (np + 191) / 192 * 192 < (np + 255) / 256 * 256 ? 192 : 256;
 }
 
 }  // namespace
@@ -484,7 +484,8 @@ int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* n
                      dim3(128), 0, stream, total, ext[0], ext[1], ext[2], nullptr, nullptr, u,
                      gammas, inv_jac, work, sides);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(pair_kernel, dim3(10 * num_elements), dim3(pair_threads(np)), lds, stream,
+  hipLaunchKernelGGL(pair_kernel, dim3(10 * num_elements),
+                     dim3(pair_threads(np, 10 * num_elements)), lds, stream,
                      num_elements, ext[0], ext[1], ext[2], nullptr, nullptr, nbr, u, gammas,
                      inv_jac, work, sides, ghost, dt, dtab, nullptr, nullptr, up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;

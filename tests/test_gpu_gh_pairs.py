@@ -37,6 +37,22 @@ def test_gh_rhs_pairs_edges(elements, extents):
     assert np.array_equal(host(domain.gh_rhs(dev(u), dev(gammas), dev(inv))), ref)
 
 
+# both sides of each line in the choice of threads: 256 and 768 points, 256
+# workgroups, and rounds that 192 or 256 threads fill better
+@pytest.mark.parametrize("elements,extents", [((1, 2, 1), (8, 8, 4)), ((1, 2, 1), (7, 7, 6)),
+                                              ((3, 3, 3), (7, 7, 6)), ((3, 3, 3), (7, 8, 7)),
+                                              ((1, 2, 1), (12, 8, 8)), ((3, 3, 3), (12, 8, 8)),
+                                              ((1, 1, 2), (11, 10, 7)), ((1, 1, 2), (10, 9, 9))])
+def test_gh_rhs_pairs_threads(elements, extents):
+    print(f"gh pairs threads {elements} x {extents}", flush=True)
+    brick, u, gammas, inv = wl.gh_kerr_schild_brick(seed=4, elements=elements, extents=extents,
+                                                    noise=1e-3)
+    ref = ol.gh_rhs(brick.extents, brick.neighbors, u, gammas, inv)
+    domain = dg.Domain.from_brick(brick)
+    domain.set_kernel("gh", "composite")
+    assert np.array_equal(host(domain.gh_rhs(dev(u), dev(gammas), dev(inv))), ref)
+
+
 @pytest.mark.parametrize("extents", [(2, 2, 2), (4, 6, 3), (7, 7, 7)])
 def test_gh_rhs_dirichlet_pairs(extents):
     print(f"gh pairs dirichlet {extents}", flush=True)
