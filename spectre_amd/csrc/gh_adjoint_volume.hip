@@ -1,7 +1,7 @@
 // Volume part of the GH adjoint (the RHS linearised at u) on uniform and ragged
 // domains, without a derivative array:
 //   gh_adjoint_sums_kernel: one workgroup per (element, half of the symmetric
-//     pairs): the partial derivatives of u from LDS, reduced on the spot to the
+//     pairs), of large elements per 512 points too: the partial derivatives of u from LDS, reduced on the spot to the
 //     ten weighted sums per point that the point-wise adjoint reads;
 //   gh_adjoint_point_kernel: one thread per point, the point-wise adjoint (50
 //     values into ubar) and the scalars that the adjoint of the derivatives needs;
@@ -61,7 +61,8 @@ __device__ __forceinline__ ElementShape element_shape(int64_t at, int n0, int n1
 
 // S fields of a pair are staged together (5, or 1 for elements whose five fields
 // exceed the LDS), next to each other per point.  Dynamic LDS: S Np doubles,
-// then the D matrices.
+// then the D matrices.  Grid: (elements and halves, chunks of the element's
+// points).
 template <bool RAGGED, int S>
 __global__ void __launch_bounds__(512)
 gh_adjoint_sums_kernel(int n0, int n1, int n2, const MixedElement* __restrict__ el,
@@ -81,7 +82,7 @@ gh_adjoint_sums_kernel(int n0, int n1, int n2, const MixedElement* __restrict__ 
   const double* ije = inv_jac + 9 * m.off;
   const double* ga = gammas + 3 * m.off;
   const int T = blockDim.x;
-  for (int base = 0; base < np; base += T) {
+  for (int base = blockIdx.y * T; base < np; base += gridDim.y * T) {
     const unsigned p = base + threadIdx.x;
     const bool active = p < static_cast<unsigned>(np);
     const int row = p / m.n0, k = row / m.n1;
@@ -162,8 +163,8 @@ gh_adjoint_sums_kernel(int n0, int n1, int n2, const MixedElement* __restrict__ 
   }
 }
 
-// One wave per workgroup; dynamic LDS: 50 fields of its 64 points (25.6 KB, so
-// that four waves, one per SIMD, share a CU).
+// One wave per workgroup; LDS: 50 fields of its 64 points (25.6 KB, so that four
+// waves, one per SIMD, share a CU).
 template <bool RAGGED>
 __global__ void __launch_bounds__(64)
 gh_adjoint_point_kernel(int64_t total, int np_uniform, const MixedElement* __restrict__ el,
@@ -360,7 +361,12 @@ int launch_sums(int count, int np, int d_doubles, const int32_t ext[3], const Mi
                            ? reinterpret_cast<const void*>(&gh_adjoint_sums_kernel<RAGGED, 5>)
                            : reinterpret_cast<const void*>(&gh_adjoint_sums_kernel<RAGGED, 1>);
   if (!allow_lds(kernel, lds)) return SXD_ERR_UNSUPPORTED;
-  const dim3 grid(2 * count), block(sums_threads(np));
+  // Field by field a chunk of the points stages the fields again in any case, so
+  // each chunk is a workgroup: with two per element for all of them whole
+  // adjoints of 8 x 16^3 took 1361 us, 64 x 16^3 2062, of 8 x 18^3 1438, with the
+  // chunks 347, 1200 and 366.
+  const int threads = sums_threads(np);
+  const dim3 grid(2 * count, five ? 1 : (np + threads - 1) / threads), block(threads);
   if (five)
     hipLaunchKernelGGL((gh_adjoint_sums_kernel<RAGGED, 5>), grid, block, lds, stream, ext[0],
                        ext[1], ext[2], el, list, u, gammas, inv_jac, gbar, work, dtab);

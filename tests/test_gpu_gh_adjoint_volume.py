@@ -47,6 +47,18 @@ def test_gh_adjoint_volume_edges(elements, extents):
     check(dg.Domain.from_brick(brick), u, gammas, inv, gbar, ref)
 
 
+# elements whose fields are staged one at a time, a workgroup per 512 points: the
+# smallest of them, with a last chunk that is nearly full, and one that is not
+@pytest.mark.parametrize("extents", [(17, 16, 15), (20, 18, 12)])
+def test_gh_adjoint_volume_chunks(extents):
+    print(f"gh adjoint chunks {extents}", flush=True)
+    brick, u, gammas, inv, _ = wl.gh_adjoint_workload(seed=3, elements=(1, 1, 1), extents=extents,
+                                                      noise=1e-3)
+    gbar = np.random.default_rng(5).standard_normal(u.shape)
+    ref = ol.gh_rhs_vjp(brick.extents, brick.neighbors, u, gammas, inv, gbar)
+    check(dg.Domain.from_brick(brick), u, gammas, inv, gbar, ref)
+
+
 @pytest.mark.parametrize("elements,lowest,highest", [((1, 1, 2), 2, 4), ((1, 2, 1), 8, 11),
                                                      ((1, 1, 2), 12, 13)])
 def test_gh_adjoint_volume_ragged_edges(elements, lowest, highest):
