@@ -1115,6 +1115,22 @@ int run_sw(sxd_domain* d, Scratch& sc, int kernel, const double* u, const double
                        kernel == SXD_KERNEL_FUSED, scratch, ghost, bc_kind, stream, up);
 }
 
+// One ScalarWave RHS call.  The fused kernel has no work arrays, so its calls do
+// not take turns on the stream's.
+int call_sw(const sxd_domain* domain, const double* u, const double* gamma2,
+            const double* inv_jac, double* dt, void* stream, const double* ghost = nullptr,
+            int bc_kind = kSwBcGhostArray) {
+  sxd_domain* d = const_cast<sxd_domain*>(domain);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const int kernel = resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE);
+  if (kernel == SXD_KERNEL_FUSED)
+    return launch_sw_rhs(d->num_elements, d->ext, d->d_nbr, u, gamma2, inv_jac, dt, true, nullptr,
+                         ghost, bc_kind, s);
+  Scratch& sc = stream_scratch(d, s);
+  std::lock_guard<std::mutex> enqueue(sc.enqueue);
+  return run_sw(d, sc, kernel, u, gamma2, inv_jac, dt, s, ghost, bc_kind);
+}
+
 int run_gh(sxd_domain* d, Scratch& sc, int kernel, const double* u, const double* gammas,
            const double* inv_jac, double* dt, hipStream_t stream,
            const double* ghost = nullptr, const Rk3Update& up = {}) {
@@ -1193,13 +1209,8 @@ int sxd_scalar_wave_rhs(const sxd_domain* domain, const double* u, const double*
   SXD_REQUIRE_DEVICE(gamma2);
   SXD_REQUIRE_DEVICE(inv_jac);
   SXD_REQUIRE_DEVICE(dt);
-  sxd_domain* d = const_cast<sxd_domain*>(domain);
-  if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
-  Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
-  std::lock_guard<std::mutex> enqueue(sc.enqueue);
-  return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
-                       static_cast<hipStream_t>(stream)),
-                __func__);
+  if (int rc = check_no_overlap(domain, 5, u, dt, __func__); rc != SXD_OK) return rc;
+  return finish(call_sw(domain, u, gamma2, inv_jac, dt, stream), __func__);
 }
 
 int sxd_scalar_wave_rhs_dirichlet(const sxd_domain* domain, const double* u,
@@ -1211,13 +1222,8 @@ int sxd_scalar_wave_rhs_dirichlet(const sxd_domain* domain, const double* u,
   SXD_REQUIRE_DEVICE(inv_jac);
   SXD_REQUIRE_DEVICE(ghost);
   SXD_REQUIRE_DEVICE(dt);
-  sxd_domain* d = const_cast<sxd_domain*>(domain);
-  if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
-  Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
-  std::lock_guard<std::mutex> enqueue(sc.enqueue);
-  return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
-                       static_cast<hipStream_t>(stream), ghost),
-                __func__);
+  if (int rc = check_no_overlap(domain, 5, u, dt, __func__); rc != SXD_OK) return rc;
+  return finish(call_sw(domain, u, gamma2, inv_jac, dt, stream, ghost), __func__);
 }
 
 int sxd_scalar_wave_rhs_spherical_radiation(const sxd_domain* domain, const double* u,
@@ -1233,15 +1239,11 @@ int sxd_scalar_wave_rhs_spherical_radiation(const sxd_domain* domain, const doub
       type != SXD_SPHERICAL_RADIATION_BAYLISS_TURKEL)
     return fail(SXD_ERR_INVALID_ARGUMENT, "unknown spherical radiation type %d", type);
   if (type == SXD_SPHERICAL_RADIATION_BAYLISS_TURKEL) SXD_REQUIRE_DEVICE(coords);
-  sxd_domain* d = const_cast<sxd_domain*>(domain);
-  if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
-  Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
-  std::lock_guard<std::mutex> enqueue(sc.enqueue);
+  if (int rc = check_no_overlap(domain, 5, u, dt, __func__); rc != SXD_OK) return rc;
   const int kind = type == SXD_SPHERICAL_RADIATION_SOMMERFELD ? kSwBcSommerfeld
                                                               : kSwBcBaylissTurkel;
-  return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
-                       static_cast<hipStream_t>(stream),
-                       kind == kSwBcBaylissTurkel ? coords : nullptr, kind),
+  return finish(call_sw(domain, u, gamma2, inv_jac, dt, stream,
+                        kind == kSwBcBaylissTurkel ? coords : nullptr, kind),
                 __func__);
 }
 
@@ -1258,14 +1260,10 @@ int sxd_scalar_wave_rhs_constraint_preserving_spherical_radiation(
     return fail(SXD_ERR_INVALID_ARGUMENT,
                 "unknown constraint-preserving spherical radiation type %d", type);
   if (type != SXD_CPSR_SOMMERFELD) SXD_REQUIRE_DEVICE(coords);
-  sxd_domain* d = const_cast<sxd_domain*>(domain);
-  if (int rc = check_no_overlap(d, 5, u, dt, __func__); rc != SXD_OK) return rc;
-  Scratch& sc = stream_scratch(d, static_cast<hipStream_t>(stream));
-  std::lock_guard<std::mutex> enqueue(sc.enqueue);
+  if (int rc = check_no_overlap(domain, 5, u, dt, __func__); rc != SXD_OK) return rc;
   const int kind = kSwBcCpsrSommerfeld + (type - SXD_CPSR_SOMMERFELD);
-  return finish(run_sw(d, sc, resolve_kernel(d, SXD_SYSTEM_SCALAR_WAVE), u, gamma2, inv_jac, dt,
-                       static_cast<hipStream_t>(stream),
-                       type == SXD_CPSR_SOMMERFELD ? nullptr : coords, kind),
+  return finish(call_sw(domain, u, gamma2, inv_jac, dt, stream,
+                        type == SXD_CPSR_SOMMERFELD ? nullptr : coords, kind),
                 __func__);
 }
 

@@ -10,6 +10,7 @@
 
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "device_common.hpp"
@@ -618,12 +619,14 @@ int launch_face_passes(bool gh, int num_elements, const int32_t ext[3], const in
 // its 15 derivatives from the LDS pencils, the volume terms, then the lifted
 // UpwindPenalty corrections of the faces it lies on (xi, eta, zeta order),
 // reading the neighbour's trace directly from HBM, and writes dt once.
-template <int N, bool GHOST, bool UPDATE>
+// Update: Rk3Update, or NoUpdate, whose launch does not carry the 32 bytes.
+struct NoUpdate {};
+template <int N, bool GHOST, typename Update>
 __global__ void __launch_bounds__((N * N * N + 63) / 64 * 64)
 sw_rhs_fused_kernel(const int32_t* __restrict__ nbr, const double* __restrict__ u,
                     const double* __restrict__ gamma2, const double* __restrict__ inv_jac,
                     double* __restrict__ dt, const double* __restrict__ dtab,
-                    const double* __restrict__ ghost, int bc_kind, Rk3Update update) {
+                    const double* __restrict__ ghost, int bc_kind, Update update) {
   constexpr int NP = N * N * N;
   __shared__ double s_u[5 * NP];
   const int64_t e = xcd_local_element(blockIdx.x, gridDim.x);
@@ -722,7 +725,8 @@ sw_rhs_fused_kernel(const int32_t* __restrict__ nbr, const double* __restrict__ 
 #pragma unroll
     for (int c = 0; c < 5; ++c) dtp[c] = dtp[c] + bc[c] * fac;
   }
-  if constexpr (UPDATE) rk3_apply<5>(dtp, update, up, (e * 5) * NP + t, NP);
+  if constexpr (std::is_same_v<Update, Rk3Update>)
+    rk3_apply<5>(dtp, update, up, (e * 5) * NP + t, NP);
 #pragma unroll
   for (int c = 0; c < 5; ++c) dt[(e * 5 + c) * NP + t] = dtp[c];
 }
@@ -752,14 +756,16 @@ static int launch_sw_fused_n(int num_elements, const int32_t* nbr, const double*
                              const double* dtab, const double* ghost, int bc_kind,
                              hipStream_t stream, const Rk3Update& up) {
   constexpr int threads = (N * N * N + 63) / 64 * 64;
-  if (ghost != nullptr || bc_kind != kSwBcGhostArray) {
-    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, true, false>), dim3(num_elements), dim3(threads), 0,
-                       stream, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, up);
-  } else {
-    hipLaunchKernelGGL((up.substep < 0 ? &sw_rhs_fused_kernel<N, false, false>
-                                       : &sw_rhs_fused_kernel<N, false, true>),
-                       dim3(num_elements), dim3(threads), 0, stream, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, up);
-  }
+  const dim3 grid(num_elements), block(threads);
+  if (ghost != nullptr || bc_kind != kSwBcGhostArray)
+    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, true, NoUpdate>), grid, block, 0, stream, nbr, u,
+                       gamma2, inv_jac, dt, dtab, ghost, bc_kind, NoUpdate{});
+  else if (up.substep < 0)
+    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, false, NoUpdate>), grid, block, 0, stream, nbr, u,
+                       gamma2, inv_jac, dt, dtab, ghost, bc_kind, NoUpdate{});
+  else
+    hipLaunchKernelGGL((sw_rhs_fused_kernel<N, false, Rk3Update>), grid, block, 0, stream, nbr,
+                       u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, up);
   return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
 }
 
@@ -906,7 +912,9 @@ rk3_substep_kernel(int64_t n, Rk3Update up, const double* __restrict__ uk,
                    const double* __restrict__ lk, double* __restrict__ out) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  out[i] = rk3_value(up.substep, rk3_step_size(up), up.u0[i], uk[i], lk[i]);
+  // the values before the step size, which may be a load of its own
+  const double u0 = up.u0[i], k = uk[i], l = lk[i];
+  out[i] = rk3_value(up.substep, rk3_step_size(up), u0, k, l);
 }
 
 int launch_rk3_substep(int64_t n, const Rk3Update& up, const double* uk, const double* lk,
