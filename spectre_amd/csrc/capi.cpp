@@ -1942,14 +1942,20 @@ int sxd_rk3_stepper_create(sxd_rk3_stepper** stepper, sxd_domain* domain, int sy
     destroy_stepper(s);
     return fail(SXD_ERR_DEVICE, "stream creation failed");
   }
-  // One RHS outside the capture allocates the stepper's own work arrays and
-  // sets kernel attributes, so the captured region only enqueues kernels.
+  // One RHS outside the capture, by the kernels that the captured step launches
+  // (its result is not used), allocates the stepper's own work arrays and sets
+  // kernel attributes, so the captured region only enqueues kernels.
   // The graph refers to those arrays only: calls on the domain afterwards
   // (which may grow the domain's own work arrays) cannot move them.
   s->kernel = system == SXD_SYSTEM_GH ? gh_kernel_with_arrays(domain, s->scratch)
                                       : resolve_kernel(domain, system);
+  Rk3Update up;
+  if (applies_update(domain, system, s->kernel)) {
+    up.substep = 0;
+    up.u0 = u;
+  }
   int rc = run_system(domain, s->scratch, system, s->kernel, u, params, inv_jac, s->d_work,
-                      s->capture);
+                      s->capture, up);
   if (rc == SXD_OK && hipStreamSynchronize(s->capture) != hipSuccess) rc = SXD_ERR_DEVICE;
   if (rc != SXD_OK) {
     destroy_stepper(s);

@@ -79,6 +79,25 @@ def test_mixed_steps(kernel):
           u, ga, inv)
 
 
+# steps of elements whose kernels need more than the default LDS, out of a graph
+@pytest.mark.parametrize("extents", [(13, 13, 13), (14, 14, 14)])
+def test_gh_stepper_large_elements(extents):
+    print(f"rk3 stepper gh {extents}", flush=True)
+    brick, u, ga, inv = wl.gh_kerr_schild_brick(seed=5, elements=(1, 1, 2), extents=extents)
+    rhs = lambda v: ol.gh_rhs(brick.extents, brick.neighbors, v, ga, inv)
+    u1 = ol.rk3_substep(0, DT, u, u, rhs(u))
+    u2 = ol.rk3_substep(1, DT, u, u1, rhs(u1))
+    end = ol.rk3_substep(2, DT, u, u2, rhs(u2))
+    d_u, d_ga, d_inv = dev(u), dev(ga), dev(inv)
+    stepper = dg.Rk3Stepper(dg.Domain.from_brick(brick), "gh", d_u, d_ga, d_inv)
+    for _ in range(3):
+        d_u.copy_(dev(u))
+        stepper.step(DT)
+        torch.cuda.synchronize()
+        assert np.array_equal(host(d_u), end)
+    stepper.close()
+
+
 def step_adjoint(adjoint, lam3):
     """mu of one transposed step; adjoint(k, lam) = A^T lam at stage input k."""
     lam = (2.0 / 3.0) * (lam3 + DT * adjoint(2, lam3))
