@@ -562,10 +562,15 @@ int sxd_domain_set_kernel(sxd_domain* domain, int system, int kernel);
  * array cannot be allocated and sxd_gh_rhs_noalloc run the fused kernel, which
  * needs no work array and gives the same result. */
 int sxd_domain_get_kernel(const sxd_domain* domain, int system, int* kernel);
-/* Threads per workgroup (tile shape): mixed-p kernels 64, 128 or 256
- * (default 128); the fused GH kernel at 7^3 and 8^3 points 256 (one wave per
- * SIMD, two points per thread) or 512 (two waves per SIMD, one point per
- * thread).  Results do not depend on it. */
+/* Threads per workgroup (tile shape) of the mixed-p kernels with face passes:
+ * 64, 128 or 256 (default 128), for SXD_KERNEL_MIXED_* and, whatever kernel is
+ * set, for domains with external faces (their face passes, and the volume
+ * kernels of the constraint-preserving conditions).  Of the fused GH kernel
+ * at 7^3 and 8^3 points: 256 (one wave per SIMD, two points per thread) or 512
+ * (two waves per SIMD, one point per thread).  The other kernels (MORTAR, the
+ * default of periodic mixed-p and of mortar domains; COMPOSITE; the volume
+ * terms of ragged domains) choose their own; the setting is accepted and kept.
+ * Results do not depend on it. */
 int sxd_domain_set_threads(sxd_domain* domain, int system, int threads);
 int sxd_domain_get_threads(const sxd_domain* domain, int system, int* threads);
 /* Give `domain` the kernel and thread choices of `from`, a domain over elements
@@ -574,7 +579,9 @@ int sxd_domain_copy_choices(sxd_domain* domain, const sxd_domain* from);
 /* Autotuner: time every kernel available for (domain, system) on the given
  * inputs (one warm-up, then `repetitions` timed calls each, HIP events on
  * `stream`), keep the fastest for later calls and return it in *chosen and
- * its mean time in *milliseconds (either may be NULL).  params is gamma2
+ * its mean time in *milliseconds (either may be NULL).  Kernels that take the
+ * domain's threads are timed with each of their tile shapes, and if one of them
+ * is the fastest its shape is kept as well.  params is gamma2
  * (ScalarWave) or gammas (GH); dt is overwritten.  Synchronises `stream`. */
 int sxd_domain_autotune(sxd_domain* domain, int system, const double* u,
                         const double* params, const double* inv_jac, double* dt,

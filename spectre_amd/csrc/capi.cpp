@@ -1660,7 +1660,9 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
   const int ncand = candidate_kernels(domain, system, cand);
   const int saved_threads = domain->threads[system];
   int best_threads = saved_threads;
-  // tile shapes: mixed p 64/128/256 threads; uniform GH fused 256/512
+  // tile shapes: mixed-p kernels 64/128/256 threads; uniform GH fused 256/512; the
+  // others choose their own, so that one pass times them, and if one of them
+  // is the fastest the domain's threads stay as they are
   const int mixed_tiles[3] = {64, 128, 256};
   const int fused_tiles[2] = {256, 512};
   const bool gh_fused_tiles = !domain->mixed && system == SXD_SYSTEM_GH && domain->ext[0] >= 7;
@@ -1668,6 +1670,8 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
   for (int cj = 0; cj < ncand * ntiles; ++cj) {
     const int ci = cj / ntiles;
     const int k = cand[ci];
+    const bool own_threads = k == SXD_KERNEL_MORTAR || k == SXD_KERNEL_COMPOSITE;
+    if (own_threads && cj % ntiles > 0) continue;
     if (domain->mixed) domain->threads[system] = mixed_tiles[cj % ntiles];
     if (gh_fused_tiles) domain->threads[system] = fused_tiles[cj % ntiles];
     rc = run_system(domain, sc, system, k, u, params, inv_jac, dt, s);  // warm-up
@@ -1686,7 +1690,7 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
     if (best < 0 || ms < best_ms) {
       best = k;
       best_ms = ms;
-      best_threads = domain->threads[system];
+      best_threads = own_threads ? saved_threads : domain->threads[system];
     }
   }
   domain->threads[system] = rc == SXD_OK ? best_threads : saved_threads;

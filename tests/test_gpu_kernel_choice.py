@@ -81,6 +81,20 @@ def test_noalloc_takes_what_fits_its_array(layout):
     assert np.array_equal(host(got), host(domain.gh_rhs(u, gammas, inv)))
 
 
+@pytest.mark.parametrize("system", ["scalar_wave", "gh"])
+def test_autotuner_leaves_threads_that_its_kernel_does_not_take(system):
+    print(f"autotuned threads {system}", flush=True)
+    make = (wl.scalar_wave_plane_wave_mixed if system == "scalar_wave" else
+            wl.gh_kerr_schild_mixed)
+    brick, u, params, inv = make(seed=1, elements=(3, 3, 3), lowest=4, highest=8)
+    u, params, inv = dev(u), dev(params), dev(inv)
+    domain = dg.MixedDomain.from_brick(brick)
+    for threads in (64, 256):
+        domain.set_threads(system, threads)
+        kernel, _ = domain.autotune(system, u, params, inv, torch.empty_like(u))
+        assert kernel == "mortar" and domain.threads(system) == threads
+
+
 @pytest.mark.parametrize("choice", ["auto", "autotuned", "fused", "composite"])
 def test_twin_has_the_same_choice(choice):
     """A twin is chosen for like its domain: pinned only where that is."""
