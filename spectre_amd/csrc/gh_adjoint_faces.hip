@@ -324,12 +324,16 @@ int launch_gh_adjoint_faces(const MortarPlan& plan, const MixedElement* el, cons
   for (const MortarClass& c : plan.classes[1]) {
     if (!allow_lds(reinterpret_cast<const void*>(&gh_adjoint_mortar_kernel), c.adjoint_lds_bytes))
       return SXD_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(gh_adjoint_mortar_kernel,
-                       dim3((c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10), dim3(192),
-                       c.adjoint_lds_bytes, stream, c.count, plan.d_jobs + c.begin, plan.d_gather,
-                       u, gammas, inv_jac, gbar, w.sides, w.speeds, w.contrib, w.side_adj, full,
-                       half);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    const int limit = launch_limit(10, 192);
+    for (int first = 0; first < c.count; first += limit) {
+      const int count = std::min(limit, c.count - first);
+      hipLaunchKernelGGL(gh_adjoint_mortar_kernel,
+                         dim3((count + kNumXcds - 1) / kNumXcds * kNumXcds * 10), dim3(192),
+                         c.adjoint_lds_bytes, stream, count, plan.d_jobs + c.begin + first,
+                         plan.d_gather, u, gammas, inv_jac, gbar, w.sides, w.speeds, w.contrib,
+                         w.side_adj, full, half);
+      if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    }
   }
   hipLaunchKernelGGL(gh_adjoint_sides_kernel, dim3(plan.num_faces), dim3(128), 0, stream, el,
                      plan.d_faces, plan.d_records, u, gammas, inv_jac, w.side_adj, w.contrib);

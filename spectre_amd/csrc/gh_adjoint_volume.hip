@@ -214,10 +214,11 @@ gh_adjoint_point_kernel(int64_t total, int np_uniform, const MixedElement* __res
 // S fields of the pair at a time (5, or 1 where their 15 Np derivative adjoints
 // exceed the LDS).  Dynamic LDS: 3 S Np doubles, then
 // the D matrices.  contrib: face terms, [E][6][50][F] (uniform domains) or per
-// record as `table` places them.
+// record as `table` places them.  list_or_first: RAGGED: length of `list`,
+// otherwise the launch's first element.
 template <bool RAGGED, int S, bool UPDATE>
 __global__ void __launch_bounds__(512)
-gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* __restrict__ el,
+gh_adjoint_sweeps_kernel(int list_or_first, int n0, int n1, int n2, const MixedElement* __restrict__ el,
                          const int32_t* __restrict__ list, const double* __restrict__ gammas,
                          const double* __restrict__ inv_jac, const double* __restrict__ gbar,
                          const double* __restrict__ work, double* __restrict__ ubar,
@@ -231,11 +232,12 @@ gh_adjoint_sweeps_kernel(int count, int n0, int n1, int n2, const MixedElement* 
     const int x = blockIdx.x % kNumXcds, slot = blockIdx.x / kNumXcds;
     at = slot / 10 * kNumXcds + x;
     pr = slot % 10;
-    if (at >= count) return;
+    if (at >= list_or_first) return;
   } else {
     const int64_t item = xcd_local_element(blockIdx.x, gridDim.x);
     at = item / 10;
     pr = static_cast<int>(item - 10 * at);
+    at += list_or_first;
   }
   const ElementShape m = element_shape<RAGGED>(at, n0, n1, n2, el, list);
   const int np = m.np;
@@ -357,23 +359,25 @@ int launch_sums(int count, int np, int d_doubles, const int32_t ext[3], const Mi
                 const double* gbar, double* work, const double* dtab, hipStream_t stream) {
   const bool five = 5 * np + d_doubles <= kLdsDoubles;
   const int lds = ((five ? 5 : 1) * np + d_doubles) * 8;
-  const void* kernel = five
-                           ? reinterpret_cast<const void*>(&gh_adjoint_sums_kernel<RAGGED, 5>)
-                           : reinterpret_cast<const void*>(&gh_adjoint_sums_kernel<RAGGED, 1>);
-  if (!allow_lds(kernel, lds)) return SXD_ERR_UNSUPPORTED;
+  const auto kernel = five ? &gh_adjoint_sums_kernel<RAGGED, 5>
+                           : &gh_adjoint_sums_kernel<RAGGED, 1>;
+  if (!allow_lds(reinterpret_cast<const void*>(kernel), lds)) return SXD_ERR_UNSUPPORTED;
   // Field by field a chunk of the points stages the fields again in any case, so
   // each chunk is a workgroup: with two per element for all of them whole
   // adjoints of 8 x 16^3 took 1361 us, 64 x 16^3 2062, of 8 x 18^3 1438, with the
   // chunks 347, 1200 and 366.
   const int threads = sums_threads(np);
-  const dim3 grid(2 * count, five ? 1 : (np + threads - 1) / threads), block(threads);
-  if (five)
-    hipLaunchKernelGGL((gh_adjoint_sums_kernel<RAGGED, 5>), grid, block, lds, stream, ext[0],
-                       ext[1], ext[2], el, list, u, gammas, inv_jac, gbar, work, dtab);
-  else
-    hipLaunchKernelGGL((gh_adjoint_sums_kernel<RAGGED, 1>), grid, block, lds, stream, ext[0],
-                       ext[1], ext[2], el, list, u, gammas, inv_jac, gbar, work, dtab);
-  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+  const int chunks = five ? 1 : (np + threads - 1) / threads;
+  // a uniform domain has too few elements for the limit: each has at least an eighth
+  // of the threads in points, at 150 doubles a point
+  const int limit = RAGGED ? launch_limit(2, threads) : count;
+  for (int first = 0; first < count; first += limit) {
+    hipLaunchKernelGGL(kernel, dim3(2 * std::min(limit, count - first), chunks), dim3(threads),
+                       lds, stream, ext[0], ext[1], ext[2], el, RAGGED ? list + first : nullptr, u,
+                       gammas, inv_jac, gbar, work, dtab);
+    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  }
+  return SXD_OK;
 }
 
 template <bool RAGGED>
@@ -393,12 +397,17 @@ int launch_sweeps(int count, int np, int d_doubles, const int32_t ext[3], const 
                            : (update ? &gh_adjoint_sweeps_kernel<RAGGED, 1, true>
                                      : &gh_adjoint_sweeps_kernel<RAGGED, 1, false>);
   if (!allow_lds(reinterpret_cast<const void*>(kernel), lds)) return SXD_ERR_UNSUPPORTED;
-  const int blocks = RAGGED ? (count + kNumXcds - 1) / kNumXcds * kNumXcds * 10 : 10 * count;
   const int threads = np > 512 ? 512 : np > 128 ? 256 : 128;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), lds, stream, count, ext[0], ext[1],
-                     ext[2], el, list, gammas, inv_jac, gbar, work, ubar, dtab, contrib, F, table,
-                     up);
-  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+  const int limit = launch_limit(10, threads);
+  for (int first = 0; first < count; first += limit) {
+    const int n = std::min(limit, count - first);
+    const int blocks = RAGGED ? (n + kNumXcds - 1) / kNumXcds * kNumXcds * 10 : 10 * n;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), lds, stream, RAGGED ? n : first,
+                       ext[0], ext[1], ext[2], el, RAGGED ? list + first : nullptr, gammas,
+                       inv_jac, gbar, work, ubar, dtab, contrib, F, table, up);
+    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  }
+  return SXD_OK;
 }
 }  // namespace
 

@@ -178,11 +178,12 @@ __host__ __device__ inline int pair_lds_doubles(int n0, int n1, int n2, bool fac
 // FACES (uniform domains): faces whose neighbour is -1 take the ghost state
 // [E][50][Np] as exterior state, as gh_face_pass_kernel does; their
 // corrections are added before those of the internal faces.
+// list_or_first: RAGGED: length of `list`, otherwise the launch's first element.
 // RAGGED: with a table of lifted corrections (launch_ragged_gh_volume) those of
 // the faces a point lies on are added, each face's mortars in order.
 template <bool RAGGED, bool FACES, bool UPDATE>
 __global__ void __launch_bounds__(512)
-gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __restrict__ el,
+gh_pair_kernel(int list_or_first, int n0, int n1, int n2, const MixedElement* __restrict__ el,
                const int32_t* __restrict__ list, const int32_t* __restrict__ nbr,
                const double* __restrict__ u, const double* __restrict__ gammas,
                const double* __restrict__ inv_jac, const double* __restrict__ state,
@@ -198,7 +199,7 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
     // next to each other on its XCD
     const int x = blockIdx.x % kNumXcds, slot = blockIdx.x / kNumXcds;
     const int at = slot / 10 * kNumXcds + x;
-    if (at >= num_elements) return;
+    if (at >= list_or_first) return;
     pr = slot % 10;
     e = list[at];
     const MixedElement m = el[e];
@@ -208,6 +209,7 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
     const int64_t item = xcd_local_element(blockIdx.x, gridDim.x);
     e = item / 10;
     pr = static_cast<int>(item - 10 * e);
+    e += list_or_first;
     off = e * n0 * n1 * n2;
   }
   const int np = n0 * n1 * n2;
@@ -425,9 +427,9 @@ gh_pair_kernel(int num_elements, int n0, int n1, int n2, const MixedElement* __r
 // workgroup per CU (360 of 10x9x9 283 / 259 / 251 / 228; 64 of 14^3 249 / 203 / 182 /
 // 154).  The fewest idle lanes alone can mean 64 threads: 526 us on 360 of
 // 10x9x9, 577 on 64 of 14^3.
-int pair_threads(int np, int workgroups) {
+int pair_threads(int np, int num_elements) {
   if (np > 768) return 512;
-  if (np <= 256 || workgroups <= 256) return std::min(512, (np + 63) / 64 * 64);
+  if (np <= 256 || num_elements <= 25) return std::min(512, (np + 63) / 64 * 64);
   return (np + 191) / 192 * 192 < (np + 255) / 256 * 256 ? 192 : 256;
 }
 
@@ -484,11 +486,16 @@ int launch_gh_rhs_pairs(int num_elements, const int32_t ext[3], const int32_t* n
                      dim3(128), 0, stream, total, ext[0], ext[1], ext[2], nullptr, nullptr, u,
                      gammas, inv_jac, work, sides);
   if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
-  hipLaunchKernelGGL(pair_kernel, dim3(10 * num_elements),
-                     dim3(pair_threads(np, 10 * num_elements)), lds, stream,
-                     num_elements, ext[0], ext[1], ext[2], nullptr, nullptr, nbr, u, gammas,
-                     inv_jac, work, sides, ghost, dt, dtab, nullptr, nullptr, up);
-  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+  const int threads = pair_threads(np, num_elements);
+  const int limit = launch_limit(10, threads);
+  for (int first = 0; first < num_elements; first += limit) {
+    hipLaunchKernelGGL(pair_kernel, dim3(10 * std::min(limit, num_elements - first)),
+                       dim3(threads), lds, stream, first, ext[0], ext[1], ext[2], nullptr, nullptr,
+                       nbr, u, gammas, inv_jac, work, sides, ghost, dt, dtab, nullptr, nullptr,
+                       up);
+    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  }
+  return SXD_OK;
 }
 
 int launch_ragged_gh_state(int count, const int32_t* list, const MixedElement* el, int np_max,
@@ -514,12 +521,16 @@ int launch_ragged_gh_volume(const std::vector<RaggedClass>& classes, const int32
   for (const RaggedClass& c : classes) {
     const int lds = (kPairStride * c.np_max + c.d_doubles) * 8;
     if (!allow_lds(reinterpret_cast<const void*>(pair_kernel), lds)) return SXD_ERR_UNSUPPORTED;
-    const int blocks = (c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10;
-    hipLaunchKernelGGL(pair_kernel, dim3(blocks),
-                       dim3(c.np_max > 910 ? 512 : c.np_max > 128 ? 256 : 128), lds, stream,
-                       c.count, 0, 0, 0, el, list + c.begin, nullptr, u, gammas, inv_jac, state,
-                       nullptr, nullptr, dt, dtab, table, corr, up);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    const int threads = c.np_max > 910 ? 512 : c.np_max > 128 ? 256 : 128;
+    const int limit = launch_limit(10, threads);
+    for (int first = 0; first < c.count; first += limit) {
+      const int count = std::min(limit, c.count - first);
+      hipLaunchKernelGGL(pair_kernel, dim3((count + kNumXcds - 1) / kNumXcds * kNumXcds * 10),
+                         dim3(threads), lds, stream, count, 0, 0, 0, el, list + c.begin + first,
+                         nullptr, u, gammas, inv_jac, state, nullptr, nullptr, dt, dtab, table,
+                         corr, up);
+      if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    }
   }
   return SXD_OK;
 }

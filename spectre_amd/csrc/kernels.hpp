@@ -126,6 +126,12 @@ int launch_gh_rhs_fused(int num_elements, const int32_t ext[3], const int32_t* n
                         const double* u, const double* gammas, const double* inv_jac,
                         double* dt, int variant, int threads, const double* ghost,
                         hipStream_t stream);
+// Elements (or mortars) that one launch takes with `workgroups` of `threads`
+// threads for each of them: a grid has fewer than 2^32 threads.  A multiple of
+// the XCDs, over which ragged lists are dealt out.
+inline int launch_limit(int workgroups, int threads) {
+  return static_cast<int>(UINT32_MAX / (static_cast<unsigned>(workgroups) * threads) / 8 * 8);
+}
 // Mixed p.  Per-element record of the ragged layout.
 struct MortarCorrection;
 struct MixedElement {

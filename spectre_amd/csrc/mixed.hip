@@ -896,10 +896,15 @@ int launch_ragged_sw_volume(const std::vector<RaggedClass>& classes, const int32
   const int lds = (5 * all.np_max + all.d_doubles) * 8;
   if (!allow_lds(reinterpret_cast<const void*>(&sw_ragged_volume_kernel), lds))
     return SXD_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(sw_ragged_volume_kernel, dim3(all.count),
-                     dim3(all.np_max > 256 ? 512 : all.np_max > 128 ? 256 : 128), lds, stream, el,
-                     list + all.begin, u, gamma2, inv_jac, dt, dtab, table, corr, up);
-  return hipGetLastError() == hipSuccess ? SXD_OK : SXD_ERR_DEVICE;
+  const int threads = all.np_max > 256 ? 512 : all.np_max > 128 ? 256 : 128;
+  const int limit = launch_limit(1, threads);
+  for (int first = 0; first < all.count; first += limit) {
+    hipLaunchKernelGGL(sw_ragged_volume_kernel, dim3(std::min(limit, all.count - first)),
+                       dim3(threads), lds, stream, el, list + all.begin + first, u, gamma2,
+                       inv_jac, dt, dtab, table, corr, up);
+    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+  }
+  return SXD_OK;
 }
 
 int launch_mixed_gh_volume_du(int count, const int32_t* list, const MixedElement* el, int np_max,

@@ -232,20 +232,24 @@ int launch_mortar_lifted_corrections(bool gh, const MortarPlan& plan, const Mixe
                             : reinterpret_cast<const void*>(&mortar_corrections_kernel<false>);
     const int lds = c.lds_bytes;
     if (!allow_lds(kernel, lds)) return SXD_ERR_DEVICE;
-    const MortarJob* jobs = plan.d_jobs + c.begin;
     // threads, measured on 1000 elements of extents 4 .. 12 with 64 / 128 / 192 /
     // 256: whole GH RHS 1055 / 912 / 864 / 864 us (768 refined and rotated elements
     // 448 / 403 / 401 / 412), 12 ScalarWave RHS 2155 / 1837 / 1728 / 1673 us
-    if (gh)
-      hipLaunchKernelGGL(mortar_corrections_kernel<true>,
-                         dim3((c.count + kNumXcds - 1) / kNumXcds * kNumXcds * 10),
-                         dim3(192), lds, stream, c.count, jobs, plan.d_gather, u, params, inv_jac,
-                         w.sides, w.speeds, w.corr, full, half);
-    else
-      hipLaunchKernelGGL(mortar_corrections_kernel<false>, dim3(c.count), dim3(256), lds,
-                         stream, c.count, jobs, plan.d_gather, u, params, inv_jac, nullptr,
-                         nullptr, w.corr, full, half);
-    if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    const int limit = gh ? launch_limit(10, 192) : launch_limit(1, 256);
+    for (int first = 0; first < c.count; first += limit) {
+      const int count = std::min(limit, c.count - first);
+      const MortarJob* jobs = plan.d_jobs + c.begin + first;
+      if (gh)
+        hipLaunchKernelGGL(mortar_corrections_kernel<true>,
+                           dim3((count + kNumXcds - 1) / kNumXcds * kNumXcds * 10), dim3(192),
+                           lds, stream, count, jobs, plan.d_gather, u, params, inv_jac, w.sides,
+                           w.speeds, w.corr, full, half);
+      else
+        hipLaunchKernelGGL(mortar_corrections_kernel<false>, dim3(count), dim3(256), lds, stream,
+                           count, jobs, plan.d_gather, u, params, inv_jac, nullptr, nullptr,
+                           w.corr, full, half);
+      if (hipGetLastError() != hipSuccess) return SXD_ERR_DEVICE;
+    }
   }
   return SXD_OK;
 }
