@@ -252,6 +252,10 @@ typedef struct sxd_domain sxd_domain;
 int sxd_domain_create(sxd_domain** domain, int num_elements,
                       const int32_t extents[3], const int32_t* neighbors);
 int sxd_domain_destroy(sxd_domain* domain);
+/* Free the device memory that destroyed domains and steppers have left for the
+ * next ones (work arrays, at most 256 MiB in all; also freed when an allocation
+ * of the library fails). */
+int sxd_release_cached_memory(void);
 
 /* A mixed-p set of conforming, aligned hexahedral elements: element e has its
  * own LGL extents extents[3 e .. 3 e + 2] (2..20 each; p-refinement).  Faces

@@ -49,6 +49,7 @@ _SIGNATURES = {
     "sxd_gh_upwind_penalty": (ctypes.c_int, [_i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "sxd_lift_flux": (ctypes.c_int, [_i64, ctypes.c_int, _vp, ctypes.c_int, _vp, _vp]),
     "sxd_domain_create": (ctypes.c_int, [ctypes.POINTER(_vp), ctypes.c_int, _ip, _ip]),
+    "sxd_release_cached_memory": (ctypes.c_int, []),
     "sxd_domain_destroy": (ctypes.c_int, [_vp]),
     "sxd_scalar_wave_rhs": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "sxd_scalar_wave_rhs_dirichlet": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp]),

@@ -86,7 +86,7 @@ def test_autotuner_leaves_threads_that_its_kernel_does_not_take(system):
     print(f"autotuned threads {system}", flush=True)
     make = (wl.scalar_wave_plane_wave_mixed if system == "scalar_wave" else
             wl.gh_kerr_schild_mixed)
-    brick, u, params, inv = make(seed=1, elements=(3, 3, 3), lowest=4, highest=8)
+    brick, u, params, inv = make(seed=1, elements=(4, 4, 4), lowest=4, highest=12)
     u, params, inv = dev(u), dev(params), dev(inv)
     domain = dg.MixedDomain.from_brick(brick)
     for threads in (64, 256):
@@ -175,6 +175,7 @@ def only_free(free_bytes):
     gc.collect()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    dg.lib().sxd_release_cached_memory()
     room = torch.empty(free_bytes, dtype=torch.uint8, device="cuda")
     held = []
     try:
