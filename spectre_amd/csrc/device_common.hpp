@@ -67,6 +67,24 @@ __host__ __device__ constexpr int pair_b(int p) {
 // InverseJacobian(logical j, inertial i) block.
 __host__ __device__ constexpr int ij3(int j, int i) { return j + 3 * i; }
 
+// Points of an element's faces before direction `dir`, both sides of each
+// dimension.
+__device__ __forceinline__ int face_begin(int n0, int n1, int n2, int dir) {
+  const int nf0 = n1 * n2, nf1 = n0 * n2, nf2 = n0 * n1;
+  const int d = dir >> 1, side = dir & 1;
+  return d == 0 ? side * nf0 : d == 1 ? 2 * nf0 + side * nf1 : 2 * (nf0 + nf1) + side * nf2;
+}
+
+// x / n for 0 <= x <= 8000 and 2 <= n <= 20, and for n = 1 and x < 4096 (a volume or
+// face index by an extent, or by half of one), with one multiplication by
+// m = divisor(n) = ceil(2^20 / n): x m stays below 2^32 and m n - 2^20 below n.
+__device__ __forceinline__ unsigned divisor(int n) {
+  return ((1u << 20) + static_cast<unsigned>(n) - 1) / static_cast<unsigned>(n);
+}
+__device__ __forceinline__ int divide(int x, unsigned m) {
+  return static_cast<int>((static_cast<unsigned>(x) * m) >> 20);
+}
+
 // Workgroup barrier that orders LDS accesses only.  __syncthreads() also
 // releases global memory, which makes every wave wait for its outstanding
 // global loads (s_waitcnt vmcnt(0)) at the barrier; with a local-address-space

@@ -131,13 +131,6 @@ sw_gauss_face_kernel(int d, int num_elements, int n0, int n1, int n2,
   }
 }
 
-// Points of the faces before direction `dir`, both sides of each dimension.
-__device__ __forceinline__ int faces_before(int n0, int n1, int n2, int dir) {
-  const int nf0 = n1 * n2, nf1 = n0 * n2, nf2 = n0 * n1;
-  const int d = dir >> 1, side = dir & 1;
-  return d == 0 ? side * nf0 : d == 1 ? 2 * nf0 + side * nf1 : 2 * (nf0 + nf1) + side * nf2;
-}
-
 // Own face values of every element: u (5), gamma2 and the face det J
 // interpolated along the normal pencils, face_values [E][7][face points in
 // direction order].  Grid (E, 7): a workgroup per field, a thread per pencil
@@ -176,8 +169,8 @@ sw_gauss_face_values_kernel(int n0, int n1, int n2, const double* __restrict__ u
       lower = fma(row[l], v, lower);
       upper = fma(row[nd + l], v, upper);
     }
-    out[faces_before(n0, n1, n2, 2 * d) + f] = lower;
-    out[faces_before(n0, n1, n2, 2 * d + 1) + f] = upper;
+    out[face_begin(n0, n1, n2, 2 * d) + f] = lower;
+    out[face_begin(n0, n1, n2, 2 * d + 1) + f] = upper;
   }
 }
 
@@ -213,7 +206,7 @@ sw_gauss_rhs_kernel(int n0, int n1, int n2, const int32_t* __restrict__ nbr,
   for (int x = threadIdx.x; x < points; x += blockDim.x) {
     const int d = x < 2 * nf0 ? 0 : x < 2 * (nf0 + nf1) ? 1 : 2;
     const int nf = d == 0 ? nf0 : d == 1 ? nf1 : nf2;
-    const int first = faces_before(n0, n1, n2, 2 * d);
+    const int first = face_begin(n0, n1, n2, 2 * d);
     const int side = x - first >= nf ? 1 : 0;
     const int f = x - first - side * nf;
     const int64_t en = nbr[6 * e + 2 * d + side];
@@ -280,7 +273,7 @@ sw_gauss_rhs_kernel(int n0, int n1, int n2, const int32_t* __restrict__ nbr,
       const int nd = d == 0 ? n0 : d == 1 ? n1 : n2;
       const int f = d == 0 ? j + n1 * k : d == 1 ? i + n0 * k : i + n0 * j;
       const int l = d == 0 ? i : d == 1 ? j : k;
-      const int x = faces_before(n0, n1, n2, dir) + f;
+      const int x = face_begin(n0, n1, n2, dir) + f;
       const double lift =
           gtab[kPackedDSize + packed_gauss_boundary_offset(nd) + (2 + side) * nd + l];
       const double scale = ((dij * lift) * s_bc[5 * points + x]) * s_bc[6 * points + x];

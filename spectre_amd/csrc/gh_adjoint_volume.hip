@@ -1,8 +1,9 @@
 // Volume part of the GH adjoint (the RHS linearised at u) on uniform and ragged
 // domains, without a derivative array:
 //   gh_adjoint_sums_kernel: one workgroup per (element, half of the symmetric
-//     pairs), of large elements per 512 points too: the partial derivatives of u from LDS, reduced on the spot to the
-//     ten weighted sums per point that the point-wise adjoint reads;
+//     pairs), of large elements per 512 points too: the partial derivatives of u
+//     from LDS, reduced on the spot to the ten weighted sums per point that the
+//     point-wise adjoint reads;
 //   gh_adjoint_point_kernel: one thread per point, the point-wise adjoint (50
 //     values into ubar) and the scalars that the adjoint of the derivatives needs;
 //   gh_adjoint_sweeps_kernel: one workgroup per (element, pair): the adjoint of
@@ -218,8 +219,8 @@ gh_adjoint_point_kernel(int64_t total, int np_uniform, const MixedElement* __res
 // otherwise the launch's first element.
 template <bool RAGGED, int S, bool UPDATE>
 __global__ void __launch_bounds__(512)
-gh_adjoint_sweeps_kernel(int list_or_first, int n0, int n1, int n2, const MixedElement* __restrict__ el,
-                         const int32_t* __restrict__ list, const double* __restrict__ gammas,
+gh_adjoint_sweeps_kernel(int list_or_first, int n0, int n1, int n2,
+                         const MixedElement* __restrict__ el, const int32_t* __restrict__ list, const double* __restrict__ gammas,
                          const double* __restrict__ inv_jac, const double* __restrict__ gbar,
                          const double* __restrict__ work, double* __restrict__ ubar,
                          const double* __restrict__ dtab, const double* __restrict__ contrib,
@@ -357,10 +358,12 @@ template <bool RAGGED>
 int launch_sums(int count, int np, int d_doubles, const int32_t ext[3], const MixedElement* el,
                 const int32_t* list, const double* u, const double* gammas, const double* inv_jac,
                 const double* gbar, double* work, const double* dtab, hipStream_t stream) {
-  const bool five = 5 * np + d_doubles <= kLdsDoubles;
+  // ragged elements have at most 193 points on a face, so that five fields fit
+  const bool five = RAGGED || 5 * np + d_doubles <= kLdsDoubles;
   const int lds = ((five ? 5 : 1) * np + d_doubles) * 8;
-  const auto kernel = five ? &gh_adjoint_sums_kernel<RAGGED, 5>
-                           : &gh_adjoint_sums_kernel<RAGGED, 1>;
+  auto kernel = &gh_adjoint_sums_kernel<RAGGED, 5>;
+  if constexpr (!RAGGED)
+    if (!five) kernel = &gh_adjoint_sums_kernel<RAGGED, 1>;
   if (!allow_lds(reinterpret_cast<const void*>(kernel), lds)) return SXD_ERR_UNSUPPORTED;
   // Field by field a chunk of the points stages the fields again in any case, so
   // each chunk is a workgroup: with two per element for all of them whole

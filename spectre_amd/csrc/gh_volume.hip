@@ -40,23 +40,8 @@ static_assert(kPartial + 10 == kGhStateDoubles, "state layout");
 // face points, the six faces in direction order.
 constexpr int kGhSideDoubles = 12;
 
-__device__ __forceinline__ int face_begin(int n0, int n1, int n2, int dir) {
-  const int nf0 = n1 * n2, nf1 = n0 * n2, nf2 = n0 * n1;
-  const int d = dir >> 1, side = dir & 1;
-  return d == 0 ? side * nf0 : d == 1 ? 2 * nf0 + side * nf1 : 2 * (nf0 + nf1) + side * nf2;
-}
-
 __device__ __forceinline__ int face_index(int n0, int n1, int d, int i, int j, int k) {
   return d == 0 ? j + n1 * k : d == 1 ? i + n0 * k : i + n0 * j;
-}
-
-// x / n for x <= 8000, n = 2 .. 20 and x n <= 8000 * 20 (a volume index by an
-// extent) with one multiplication: m = ceil(2^20 / n).
-__device__ __forceinline__ int divide(int x, unsigned m) {
-  return static_cast<int>((static_cast<unsigned>(x) * m) >> 20);
-}
-__device__ __forceinline__ unsigned divisor(int n) {
-  return ((1u << 20) + static_cast<unsigned>(n) - 1) / static_cast<unsigned>(n);
 }
 
 // RAGGED: grid (list length, chunks of 128 points of the largest element).
@@ -420,13 +405,13 @@ gh_pair_kernel(int list_or_first, int n0, int n1, int n2, const MixedElement* __
 
 // Threads of a workgroup that takes np points in rounds.  Up to 256 points, or
 // where the launch has no second workgroup for a CU: one round (2 elements of
-// 7x7x6 16.6 us, with 192 threads 19.3).  Up to 768, where several workgroups share a CU: 192 or 256, whichever
-// leaves fewer lanes idle in the last round (360 elements of 7x7x6 with 192 / 256 /
-// 320 / 512 threads 81 / 85 / 101 / 100 us, of 8x8x7 115 / 106 / 141 / 125, of 9^3
-// 202 / 191 / 224 / 197).  Beyond: 512, the more so where the LDS leaves one
-// workgroup per CU (360 of 10x9x9 283 / 259 / 251 / 228; 64 of 14^3 249 / 203 / 182 /
-// 154).  The fewest idle lanes alone can mean 64 threads: 526 us on 360 of
-// 10x9x9, 577 on 64 of 14^3.
+// 7x7x6 16.6 us, with 192 threads 19.3).  Up to 768, where several workgroups
+// share a CU: 192 or 256, whichever leaves fewer lanes idle in the last round (360
+// elements of 7x7x6 with 192 / 256 / 320 / 512 threads 81 / 85 / 101 / 100 us, of
+// 8x8x7 115 / 106 / 141 / 125, of 9^3 202 / 191 / 224 / 197).  Beyond: 512, the more
+// so where the LDS leaves one workgroup per CU (360 of 10x9x9 283 / 259 / 251 / 228;
+// 64 of 14^3 249 / 203 / 182 / 154).  The fewest idle lanes alone can mean 64 threads:
+// 526 us on 360 of 10x9x9, 577 on 64 of 14^3.
 int pair_threads(int np, int num_elements) {
   if (np > 768) return 512;
   if (np <= 256 || num_elements <= 25) return std::min(512, (np + 63) / 64 * 64);

@@ -782,15 +782,20 @@ int launch_sw_rhs(int num_elements, const int32_t ext[3], const int32_t* nbr,
   if (fused) {
     if (!sw_fused_supported(ext)) return SXD_ERR_UNSUPPORTED;
     switch (ext[0]) {
-      case 2: return launch_sw_fused_n<2>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 3: return launch_sw_fused_n<3>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 4: return launch_sw_fused_n<4>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 5: return launch_sw_fused_n<5>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 6: return launch_sw_fused_n<6>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 7: return launch_sw_fused_n<7>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 8: return launch_sw_fused_n<8>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 9: return launch_sw_fused_n<9>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
-      case 10: return launch_sw_fused_n<10>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost, bc_kind, stream, up);
+#define SXD_SW_CASE(n)                                                                       \
+  case n:                                                                                    \
+    return launch_sw_fused_n<n>(num_elements, nbr, u, gamma2, inv_jac, dt, dtab, ghost,      \
+                                bc_kind, stream, up);
+      SXD_SW_CASE(2)
+      SXD_SW_CASE(3)
+      SXD_SW_CASE(4)
+      SXD_SW_CASE(5)
+      SXD_SW_CASE(6)
+      SXD_SW_CASE(7)
+      SXD_SW_CASE(8)
+      SXD_SW_CASE(9)
+      SXD_SW_CASE(10)
+#undef SXD_SW_CASE
       default: return SXD_ERR_UNSUPPORTED;
     }
   }

@@ -45,14 +45,6 @@ __host__ __device__ inline int corrections_doubles(int km, const SideLds& a, con
   return faces > bc ? faces : bc;
 }
 
-// x / n for x < 8000 and n <= 20 with one multiplication.
-__device__ __forceinline__ unsigned divisor(int n) {
-  return ((1u << 20) + static_cast<unsigned>(n) - 1) / static_cast<unsigned>(n);
-}
-__device__ __forceinline__ int divide(int x, unsigned m) {
-  return static_cast<int>((static_cast<unsigned>(x) * m) >> 20);
-}
-
 // v[j] of the packaged values OFF[j] at mortar point (ra, rb) of a side:
 // dimension b of the interpolation (row: the matrix row of rb, null for the
 // identity) from the staged values.
@@ -122,7 +114,7 @@ struct MortarLds {
   __device__ __forceinline__ double* mag(bool second) const { return pick(second, mag1, mag0); }
 };
 
-// Steps 0 to 4 of mortar_faces.hip for the fields comp[] of the two elements: on
+// Steps 1 to 4 of mortar_faces.hip for the fields comp[] of the two elements: on
 // return (after a barrier) a side's corrections with dimension a projected back
 // are [mortar b][face a][5], for mortar_face_value.
 template <bool GH>

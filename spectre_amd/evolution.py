@@ -35,27 +35,6 @@ def rk3_adjoint_substep(substep, dt, lam, a, mu, lam_out=None):
     return mu, lam_out
 
 
-def rk3_step(domain, rhs, u, params, inv_jac, dt, stage, l):
-    """One Rk3HesthavenSsp step of u in place (stage, l: work arrays)."""
-    rhs(u, params, inv_jac, out=l)
-    _pyb.rk3_substep(0, dt, u, u, l, stage)
-    rhs(stage, params, inv_jac, out=l)
-    _pyb.rk3_substep(1, dt, u, stage, l, stage)
-    rhs(stage, params, inv_jac, out=l)
-    _pyb.rk3_substep(2, dt, u, stage, l, u)
-
-
-def rk3_step_adjoint(adjoint_rhs, lam3, params, inv_jac, dt, a, lam, mu):
-    """Adjoint of one RK3 step of a linear RHS: mu = S^T lam3 (a, lam: work)."""
-    adjoint_rhs(lam3, params, inv_jac, out=a)
-    rk3_adjoint_substep(2, dt, lam3, a, mu, lam)        # lam = lam2, mu = lam3 / 3
-    adjoint_rhs(lam, params, inv_jac, out=a)
-    rk3_adjoint_substep(1, dt, lam, a, mu, lam)         # lam = lam1, mu += 3/4 lam2
-    adjoint_rhs(lam, params, inv_jac, out=a)
-    rk3_adjoint_substep(0, dt, lam, a, mu, None)        # mu += lam1 + dt A^T lam1
-    return mu
-
-
 class ScalarWaveEvolution(torch.autograd.Function):
     """u_final = S^steps u0 for the ScalarWave DG RHS on `domain`."""
 
@@ -102,24 +81,10 @@ class ScalarWaveEvolution(torch.autograd.Function):
         return lam3, None, None, None, None, None, None, None
 
 
-def rk3_step_states(rhs, u, params, inv_jac, dt, l, complete=True):
+def _gh_step_stages(domain, u, gammas, inv_jac, dt, l, complete=True):
     """One RK3 step of u (in place) returning its stage inputs (u, u1, u2).
     complete=False stops after the stage inputs (u is left unchanged): the
     step's result is not needed."""
-    u0 = u.clone() if complete else u
-    rhs(u, params, inv_jac, out=l)
-    u1 = _pyb.rk3_substep(0, dt, u, u, l, torch.empty_like(u))
-    rhs(u1, params, inv_jac, out=l)
-    u2 = _pyb.rk3_substep(1, dt, u, u1, l, torch.empty_like(u))
-    if complete:
-        rhs(u2, params, inv_jac, out=l)
-        _pyb.rk3_substep(2, dt, u, u2, l, u)
-    return u0, u1, u2
-
-
-def _gh_step_stages(domain, u, gammas, inv_jac, dt, l, complete=True):
-    """rk3_step_states of the GH RHS on `domain`, the substeps applied by its
-    kernels."""
     u0 = u.clone() if complete else u
     u1, u2 = torch.empty_like(u), torch.empty_like(u)
     _pyb.rk3_step(domain.handle, _GH, dt, u, gammas, inv_jac, u1, u2, l, u if complete else None)
@@ -155,8 +120,9 @@ class GhEvolution(torch.autograd.Function):
                               u)
         ctx.domain, ctx.dt, ctx.steps, ctx.k = domain, dt, steps, checkpoint_every
         # overlap the recompute with the adjoint (see backward): on by default
-        # for mixed-p domains; the uniform fused RHS kernel fills whole CUs
-        # and only competes with the adjoint kernels
+        # for mixed-p domains; uniform domains run one after the other (the fused
+        # RHS kernel, where it runs, fills whole CUs and only competes with the
+        # adjoint kernels)
         ctx.overlap = isinstance(domain, dg.MixedDomain) if overlap is None else bool(overlap)
         ctx.checkpoints, ctx.last_stages = checkpoints, last_stages
         ctx.save_for_backward(gammas, inv_jac)
