@@ -101,6 +101,7 @@ __device__ __forceinline__ void lds_barrier() {
 // contiguous run of about E / 8 elements, so that an element and the
 // neighbours whose face traces it reads (numbered next to it) share an L2.
 constexpr int kNumXcds = 8;
+constexpr int kNumCus = 256;  // compute units of the chip
 __device__ __forceinline__ int64_t xcd_local_element(int64_t b, int64_t num_elements) {
   const int64_t x = b % kNumXcds, slot = b / kNumXcds;
   const int64_t per = num_elements / kNumXcds, rem = num_elements % kNumXcds;

@@ -414,14 +414,14 @@ gh_pair_kernel(int list_or_first, int n0, int n1, int n2, const MixedElement* __
 // 526 us on 360 of 10x9x9, 577 on 64 of 14^3.
 int pair_threads(int np, int num_elements) {
   if (np > 768) return 512;
-  if (np <= 256 || num_elements <= 25) return std::min(512, (np + 63) / 64 * 64);
+  if (np <= 256 || 10 * num_elements <= kNumCus) return std::min(512, (np + 63) / 64 * 64);
   return (np + 191) / 192 * 192 < (np + 255) / 256 * 256 ? 192 : 256;
 }
 
 }  // namespace
 
 // Whether the two kernels take less time than the fused one (isotropic N = 3
-// .. 8).  The fused kernel fills whole CUs, so its time goes in rounds of 256 x
+// .. 8).  The fused kernel fills whole CUs, so its time goes in rounds of kNumCus x
 // (workgroups per CU) elements; the pair kernel's workgroups are a tenth of an
 // element and its time is a launch's worth plus a time per element.
 // Measured in microseconds (periodic; the Dirichlet closure has the same
@@ -439,7 +439,7 @@ bool gh_pairs_faster(int num_elements, const int32_t ext[3]) {
                                {0.155, 34.0, 1}, {0.25, 79.0, 1},  {0.366, 71.0, 1}};
   if (ext[0] < 3 || ext[0] > 8 || ext[1] != ext[0] || ext[2] != ext[0]) return false;
   const Cost& c = cost[ext[0] - 3];
-  const int per_round = 256 * c.per_cu;
+  const int per_round = kNumCus * c.per_cu;
   const int rounds = (num_elements + per_round - 1) / per_round;
   return 14.0 + c.element * num_elements < c.round * rounds;
 }

@@ -101,3 +101,28 @@ def test_gh_auto_choice_in_a_graph():
         graph.replay()
         eager = domain.gh_rhs(u, gammas, inv)
         assert np.array_equal(host(out), host(eager))
+
+
+# the choice at the element counts where it changes, by rounds of workgroups on
+# 256 compute units; 7^3 always takes the pair kernels
+@pytest.mark.parametrize("n,pairs,fused", [(3, (428, 1025), (429, 1024)),
+                                           (4, (488, 1025), (489, 1024)),
+                                           (5, (270, 513), (271, 512)),
+                                           (6, (129, 257, 348), (130, 256, 349)),
+                                           (7, (1, 255, 256, 257, 600), ()),
+                                           (8, (155, 257, 349), (156, 256, 350))])
+def test_gh_auto_choice_lines(n, pairs, fused):
+    brick, u, gammas, inv = wl.gh_kerr_schild_brick(seed=7, elements=(1, 1, 1),
+                                                    extents=(n, n, n), noise=1e-3)
+    arrays = [dev(a) for a in (u, gammas, inv)]
+    for counts, kernel in ((pairs, "composite"), (fused, "fused")):
+        for count in counts:
+            print(f"gh auto {count} x {n}^3", flush=True)
+            args = [a.repeat(count, 1, 1) for a in arrays]
+            args[0] = args[0] * (1.0 + 1e-3 * torch.sin(torch.arange(
+                count, dtype=torch.float64, device="cuda")))[:, None, None]
+            domain = dg.Domain((n, n, n), wl.periodic_neighbors((count, 1, 1)))
+            assert domain.kernel("gh") == kernel
+            got = domain.gh_rhs(*args)
+            domain.set_kernel("gh", "fused" if kernel == "composite" else "composite")
+            assert torch.equal(got, domain.gh_rhs(*args))
