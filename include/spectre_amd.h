@@ -584,8 +584,8 @@ int sxd_domain_copy_choices(sxd_domain* domain, const sxd_domain* from);
  * inputs (one warm-up, then `repetitions` timed calls each, HIP events on
  * `stream`), keep the fastest for later calls and return it in *chosen and
  * its mean time in *milliseconds (either may be NULL).  Kernels that take the
- * domain's threads are timed with each of their tile shapes, and if one of them
- * is the fastest its shape is kept as well.  params is gamma2
+ * domain's threads are timed with each of their tile shapes; the fastest of these
+ * is kept for the calls that take it, whichever kernel is chosen.  params is gamma2
  * (ScalarWave) or gammas (GH); dt is overwritten.  Synchronises `stream`. */
 int sxd_domain_autotune(sxd_domain* domain, int system, const double* u,
                         const double* params, const double* inv_jac, double* dt,

@@ -1743,15 +1743,15 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
     return fail(SXD_ERR_DEVICE, "hipEventCreate failed");
   }
   int best = -1;
-  float best_ms = 0.0f;
+  float best_ms = 0.0f, tile_ms = 0.0f;
   int rc = SXD_OK;
   int cand[3];
   const int ncand = candidate_kernels(domain, system, cand);
   const int saved_threads = domain->threads[system];
   int best_threads = saved_threads;
   // tile shapes: mixed-p kernels 64/128/256 threads; uniform GH fused 256/512; the
-  // others choose their own, so that one pass times them, and if one of them
-  // is the fastest the domain's threads stay as they are
+  // others choose their own, so that one pass times them.  The fastest shape is
+  // kept for the calls that take it, also where a kernel that does not is chosen.
   const int mixed_tiles[3] = {64, 128, 256};
   const int fused_tiles[2] = {256, 512};
   const bool gh_fused_tiles = !domain->mixed && system == SXD_SYSTEM_GH && domain->ext[0] >= 7;
@@ -1779,7 +1779,10 @@ int sxd_domain_autotune(sxd_domain* domain, int system, const double* u, const d
     if (best < 0 || ms < best_ms) {
       best = k;
       best_ms = ms;
-      best_threads = own_threads ? saved_threads : domain->threads[system];
+    }
+    if (!own_threads && (tile_ms == 0.0f || ms < tile_ms)) {
+      tile_ms = ms;
+      best_threads = domain->threads[system];
     }
   }
   domain->threads[system] = rc == SXD_OK ? best_threads : saved_threads;

@@ -81,18 +81,50 @@ def test_noalloc_takes_what_fits_its_array(layout):
     assert np.array_equal(host(got), host(domain.gh_rhs(u, gammas, inv)))
 
 
+def call_ms(call, calls=20):
+    call()
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    begin.record()
+    for _ in range(calls):
+        call()
+    end.record()
+    end.synchronize()
+    return begin.elapsed_time(end) / calls
+
+
 @pytest.mark.parametrize("system", ["scalar_wave", "gh"])
-def test_autotuner_leaves_threads_that_its_kernel_does_not_take(system):
+def test_autotuned_threads(system):
+    """The autotuner takes the mortar kernels, which choose their own threads; the
+    threads it keeps are the ones that suit the kernels with face passes."""
     print(f"autotuned threads {system}", flush=True)
     make = (wl.scalar_wave_plane_wave_mixed if system == "scalar_wave" else
             wl.gh_kerr_schild_mixed)
     brick, u, params, inv = make(seed=1, elements=(4, 4, 4), lowest=4, highest=12)
     u, params, inv = dev(u), dev(params), dev(inv)
+    out = torch.empty_like(u)
     domain = dg.MixedDomain.from_brick(brick)
-    for threads in (64, 256):
+    kernel, _ = domain.autotune(system, u, params, inv, out, repetitions=20)
+    assert kernel == "mortar"
+    kept = domain.threads(system)
+    domain.set_kernel(system, "mixed_batched")
+    rhs = domain.scalar_wave_rhs if system == "scalar_wave" else domain.gh_rhs
+    times = {}
+    for threads in (64, 128, 256):
         domain.set_threads(system, threads)
-        kernel, _ = domain.autotune(system, u, params, inv, torch.empty_like(u))
-        assert kernel == "mortar" and domain.threads(system) == threads
+        times[threads] = call_ms(lambda: rhs(u, params, inv, out))
+    print(f"kept {kept}: {times}", flush=True)
+    assert times[kept] <= 1.1 * min(times.values())
+
+
+def test_autotuner_leaves_threads_that_no_kernel_takes():
+    print("autotuned threads on a mortar domain", flush=True)
+    brick, u, params, inv = wl.gh_mortar_workload(seed=1, base=(2, 2, 2), refine={0: (0, 1)})
+    u, params, inv = dev(u), dev(params), dev(inv)
+    domain = dg.MortarDomain.from_brick(brick)
+    for threads in (64, 256):
+        domain.set_threads("gh", threads)
+        domain.autotune("gh", u, params, inv, torch.empty_like(u))
+        assert domain.threads("gh") == threads
 
 
 @pytest.mark.parametrize("choice", ["auto", "autotuned", "fused", "composite"])
