@@ -1081,10 +1081,11 @@ int gh_call_kernel(const sxd_domain* d, Scratch& sc, hipStream_t stream) {
   const int kernel = resolve_kernel(d, SXD_SYSTEM_GH);
   if (!fused_stands_in(d, kernel)) return kernel;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
-      capture != hipStreamCaptureStatusNone)
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+    (void)hipGetLastError();  // the null stream beside the capture of a blocking one
     return SXD_KERNEL_FUSED;
-  return gh_kernel_with_arrays(d, sc);
+  }
+  return capture != hipStreamCaptureStatusNone ? SXD_KERNEL_FUSED : gh_kernel_with_arrays(d, sc);
 }
 
 // Reserve work arrays (status only; finish() words the message).

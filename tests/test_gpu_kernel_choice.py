@@ -2,6 +2,7 @@
 choice: the same results with and without room for work arrays, inside and
 outside of a captured graph."""
 import contextlib
+import ctypes
 import gc
 import threading
 
@@ -199,6 +200,29 @@ def test_first_rhs_beside_a_capture():
     assert done == [True]
     graph.replay()
     assert np.array_equal(host(got), ref) and host(x)[0] == 2.0
+
+
+def test_rhs_on_the_null_stream_beside_a_capture():
+    """The capture of a stream that synchronises with the null stream does not
+    fail a call on the null stream."""
+    print("null stream beside a capture", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    brick, u, gammas, inv = gh_case((2, 2, 2), 6)
+    domain = dg.Domain.from_brick(brick)
+    ref = host(dg.Domain.from_brick(brick).gh_rhs(u, gammas, inv))
+    got = torch.empty_like(u)
+    assert torch.cuda.current_stream().cuda_stream == 0
+    torch.cuda.synchronize()
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, 2) == 0  # hipStreamCaptureModeRelaxed
+    try:
+        domain.gh_rhs(u, gammas, inv, got)
+    finally:
+        assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        hip.hipGraphDestroy(graph)
+        hip.hipStreamDestroy(stream)
+    assert np.array_equal(host(got), ref)
 
 
 @contextlib.contextmanager
