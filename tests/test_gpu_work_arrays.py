@@ -1,6 +1,7 @@
 """Work arrays that pass from one domain to the next, and calls of several host
 threads on one stream, which share them."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -66,12 +67,20 @@ def test_kept_memory_is_given_back():
         domain.gh_rhs(*args)
     torch.cuda.synchronize()
     before = torch.cuda.mem_get_info()[0]
+
+    def freed(bytes_):
+        """Whether so much more is free, the driver being given 10 seconds."""
+        for _ in range(100):
+            if torch.cuda.mem_get_info()[0] >= before + bytes_:
+                return True
+            time.sleep(0.1)
+        return False
+
     for domain in domains:
         domain.close()
-    kept = 14 * 27e6 - (torch.cuda.mem_get_info()[0] - before)
-    assert kept <= (256 << 20) + 14e6
+    assert freed(14 * 27e6 - (256 << 20) - 14e6)
     dg.lib().sxd_release_cached_memory()
-    assert torch.cuda.mem_get_info()[0] >= before + 14 * 26e6
+    assert freed(14 * 26e6)
 
 
 def test_two_threads_on_one_stream():
